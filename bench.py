@@ -36,6 +36,7 @@ from __future__ import annotations
 import argparse
 import json
 import os
+import re
 import sys
 import time
 
@@ -112,12 +113,19 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
         names = ["col_fwd", "row", "col_inv", "norm"]
     rns = 3 if "NTT3" in plan else 2
     N = 1 << n
+    # the double-precision limb transform (what an engine squares with unless a plan is fixed)
+    f64 = re.search(r"in doubles \(.* (\d) 49-bit primes, cols 2\^(\d+)", plan)
     # the transform: rns primes x N residues, or for the two-digit-limb transform 4 primes x N/2 limbs
     tn, tp = (n - 1, 4) if limb else (n, rns)
     words = tp << tn
     dom = max(range(4), key=lambda i: km[i])
     ng = t.get_plan()[2]
-    if limb and fused:  # digits (+ range carries) in, residues out | row | residues in, digits + carries out
+    if f64:  # as the fused limb plan, residues of 8 bytes, ranges of 16 limbs
+        names = ["col_fwd", "row", "col_inv_norm", "norm"]
+        tn, tp = n - 1, int(f64.group(1))
+        words, slots = tp << tn, N // 2
+        alg = {0: 4 * N + 8 * words + slots, 1: 16 * words, 2: 8 * words + 4 * N + slots, 3: 0}
+    elif limb and fused:  # digits (+ range carries) in, residues out | row | residues in, digits + carries out
         slots = 16 * (N // 2) // ng
         alg = {0: 4 * N + 4 * words + slots, 1: 8 * words, 2: 4 * words + 4 * N + slots, 3: 0}
     elif fused:  # digits in, residues out | row | residues in, digits out | segment carries
@@ -135,11 +143,12 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
                           "GBps": round(sq_bytes / (ms / steps * 1e-3) / 1e9, 1),
                           "frac": round(sq_bytes / (ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
     # butterflies of the dominant pass (row: (n - a) levels fwd + inv, N/2 per level per prime)
-    a = t.get_plan()[0]
-    levels = {0: a, 1: 2 * (tn - a), 2: a}.get(dom, 0)
+    a = int(f64.group(2)) if f64 else t.get_plan()[0]
+    row_levels = tn - a - (2 if f64 else 0)  # the double-precision rows stop two levels early
+    levels = {0: a, 1: 2 * row_levels, 2: a}.get(dom, 0)
     bfly = tp * levels * ((1 << tn) // 2)
     bfly_rate = bfly / (km[dom] * 1e-3) if levels else 0.0
-    meas = measured(names[dom], t.get_plan())
+    meas = MEASURED.get(("f64", names[dom], a), {}) if f64 else measured(names[dom], t.get_plan())
     ipb = meas.get("valu_instr_per_butterfly")
     res = {
         "b": b, "plan": plan, "plan_tuple": list(t.get_plan()), "limb": limb, "ms_per_step": ms / steps, "ns_per_squaring": ms / steps * 1e6,
@@ -152,7 +161,7 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
             "duration_source": f"HIP events around {kreps} back-to-back launches of the kernel alone on the engine's stream",
             "traffic_source": (f"profile constant: {meas['profile']} ({meas['kernel']}, FETCH_SIZE x 1.998 + WRITE_SIZE)"
                                if meas else None),
-            "note": "the kernel is bound by integer VALU issue (see valu), not by HBM",
+            "note": "see valu for the kernel's share of the VALU issue rate",
         },
         "valu": {
             "kernel": names[dom], "butterflies": bfly, "butterflies_per_s": round(bfly_rate),

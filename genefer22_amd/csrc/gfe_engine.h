@@ -14,6 +14,7 @@
 #include "gfe_spec.h"
 #include "gfe_fused.h"
 #include "gfe_limb.h"
+#include "gfe_f64_host.h"
 
 namespace gfe {
 
@@ -95,6 +96,18 @@ struct Engine {
     int tp() const { return plan.limb ? 4 : rns; }               // primes of the transform
     const uint32_t *cur_tw() const { return plan.limb ? tw_limb : tw; }
     const PrimeArgs &cur_pr() const { return plan.limb ? pr4 : pr; }
+    // Double-precision limb transform (gfe_f64.h).  An engine squares with it from its creation where
+    // it is exact (f64_k primes, 0: it is not); gfe_set_plan selects the integer passes instead.
+    // Products run in the transform that holds the multiplicand (zp_f64).
+    bool f64 = false, zp_f64 = false;
+    int f64_k = 0;
+    F64Shape shape;
+    double *tw64 = nullptr;
+    F64Crt *crt64 = nullptr;
+    int f64_select();
+    F64Args f64_args(int dup) const;
+    void f64_run(uint32_t src, uint32_t *out, int mode);
+    void f64_finish(int dup);  // the product in ws into register 0
     int rounds = 0;   // carry rounds of the fused inverse column pass
     int cus = 0;      // compute units of the device
     std::map<std::tuple<const void *, int, size_t>, unsigned> resident;  // per (kernel, threads, LDS)
@@ -106,7 +119,8 @@ struct Engine {
     // registers runs the carry kernel first (flush_carry).
     bool carry_pending = false;
     // what the pending carries are: 0 k_norm's workgroup carries, 1 k_norm_limb's boundary pairs,
-    // 2 the range slots of ks_col_inv_norm_limb (ranges of 2^pend_rlog limbs)
+    // 2 the range slots of ks_col_inv_norm_limb (ranges of 2^pend_rlog limbs), 3 those of the
+    // double-precision transform (16 limbs)
     int pend_kind = 0, pend_rlog = 0;
     bool defer_carry() const { return plan.spec && !plan.pipe && (!plan.fused || plan.limb) && !plan.fuse_sq; }
     void flush_carry();

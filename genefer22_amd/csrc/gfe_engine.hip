@@ -412,10 +412,16 @@ bool limb_fused_ok(uint32_t b, uint32_t n, int ng) {
     return 2 * ranges * per_range < P / 4;
 }
 
-// Device bytes of an engine: registers, work space, multiplicand and twiddles of rns primes, the
-// carry buffer (N bytes) and, with limb_tables, the limb transform's twiddles (4 x N/2 words).
+// Bytes of the work space and of the multiplicand: rns x N residues of 4 bytes, or the
+// double-precision limb transform's 3 x N/2 of 8.
+static size_t work_bytes(size_t N) { return 4 * (size_t)F64_PRIMES * N; }
+
+// Device bytes of an engine: registers, work space and multiplicand, the twiddles of rns primes, the
+// carry buffer (N bytes), with limb_tables the limb transform's twiddles (4 x N/2 words), and the
+// double-precision transform's (3 x N/8 doubles).
 size_t engine_bytes(int rns, size_t N, uint32_t num_regs, bool limb_tables) {
-    return (size_t)num_regs * N * 4 + 3 * (size_t)rns * N * 4 + N + (limb_tables ? 8 * N : 0);
+    return (size_t)num_regs * N * 4 + 2 * work_bytes(N) + (size_t)rns * N * 4 + N + (limb_tables ? 8 * N : 0) +
+           (size_t)F64_PRIMES * N;
 }
 
 // An engine's first plan: the limb transform where it is exact (with the inverse column pass and
@@ -702,6 +708,7 @@ void engine_set_lds_attributes() {
     set_lds_attributes();
     spec_set_lds_attributes();
     fused_set_lds_attributes();
+    f64_set_lds_attributes();
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -713,6 +720,8 @@ Engine::~Engine() {
         if (stream) (void)hipStreamSynchronize(stream);
         (void)hipFree(regs); (void)hipFree(ws); (void)hipFree(zp); (void)hipFree(carry);
         (void)hipFree(tw); (void)hipFree(crt);
+        if (tw64) (void)hipFree(tw64);
+        if (crt64) (void)hipFree(crt64);
         if (tw_limb) (void)hipFree(tw_limb);
         if (limb_crt) (void)hipFree(limb_crt);
         if (stream) (void)hipStreamDestroy(stream);
@@ -732,13 +741,14 @@ int Engine::init(uint32_t b_, uint32_t n_, uint32_t num_regs_, int device_) {
     set_lds_attributes();
     spec_set_lds_attributes();
     fused_set_lds_attributes();
+    f64_set_lds_attributes();
     if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return set_error(GFE_EHIP, "stream");
     plan = default_plan(n);
     rounds = carry_rounds(b, n);
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 256;
-    if (hipMalloc(&regs, (size_t)num_regs * N * 4) != hipSuccess || hipMalloc(&ws, (size_t)rns * N * 4) != hipSuccess ||
-        hipMalloc(&zp, (size_t)rns * N * 4) != hipSuccess || hipMalloc(&carry, (N / 8) * 8) != hipSuccess ||
-
+    const size_t wb = work_bytes(N);
+    if (hipMalloc(&regs, (size_t)num_regs * N * 4) != hipSuccess || hipMalloc(&ws, wb) != hipSuccess ||
+        hipMalloc(&zp, wb) != hipSuccess || hipMalloc(&carry, (N / 8) * 8) != hipSuccess ||
         hipMalloc(&tw, (size_t)rns * N * 4) != hipSuccess || hipMalloc(&crt, sizeof(CrtConst)) != hipSuccess) {
         dev_ok = true;
         return set_error(GFE_ENOMEM, "device allocation failed");
@@ -776,6 +786,12 @@ int Engine::init(uint32_t b_, uint32_t n_, uint32_t num_regs_, int device_) {
         }
         plan = engine_plan_for(b, n);
     }
+    // the double-precision transform's tables, of three primes whatever b needs: a rebase may need them
+    if (hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess || hipMalloc(&crt64, sizeof(F64Crt)) != hipSuccess)
+        return set_error(GFE_ENOMEM, "device allocation failed");
+    if (f64_build_twiddles(n, tw64, stream) != 0) return set_error(GFE_EHIP, "twiddles");
+    const int rc = f64_select();
+    if (rc != GFE_OK) return rc;
     if (hipMemsetAsync(regs, 0, (size_t)num_regs * N * 4, stream) != hipSuccess) return set_error(GFE_EHIP, "memset");
     for (int i = 0; i < 12; ++i) { hipEvent_t ev; if (hipEventCreate(&ev) != hipSuccess) return set_error(GFE_EHIP, "event"); events.push_back(ev); }
     if (hipStreamSynchronize(stream) != hipSuccess) return set_error(GFE_EHIP, "init sync");
@@ -821,6 +837,7 @@ unsigned Engine::resident_blocks(const void *fn, int threads, size_t lds) {
 
 // Forward column pass from register `src` into `dst` (ws or zp).
 void Engine::launch_col_fwd(uint32_t src, uint32_t *dst) {
+    if (carry_pending && pend_kind == 3) flush_carry();
     // the fused limb plans' forward pass stages the four primes' digits once (ks_col_fwd_limb_all)
     // and takes only the range carries
     const bool staged = plan.limb && plan.fused && plan.spec && spec_col_fwd_limb_all(plan.col_loge, plan.a) != nullptr;
@@ -1017,7 +1034,8 @@ void Engine::flush_carry() {
 }
 
 void Engine::launch_carry() {
-    if (pend_kind == 2) launch_carry_slots();
+    if (pend_kind == 3) f64_launch_flush(f64_args(0), stream);
+    else if (pend_kind == 2) launch_carry_slots();
     else if (pend_kind == 1) launch_carry_limbs();
     else launch_carry_digits();
 }
@@ -1049,7 +1067,49 @@ void Engine::launch_fused(int dup) {
     hipLaunchKernelGGL(fused_square_fn((int)n), dim3(1), dim3(fused_threads((int)n)), fused_lds_bytes((int)n), stream, A);
 }
 
+// The double-precision transform for the engine's (b, n), where it is exact.
+int Engine::f64_select() {
+    f64_k = f64_primes(b, n);
+    f64 = zp_f64 = f64_k != 0;
+    if (!f64) return GFE_OK;
+    const F64Crt c = make_f64_crt(n, b, f64_k);
+    shape = f64_shape(n, 1);
+    return hipMemcpy(crt64, &c, sizeof(c), hipMemcpyHostToDevice) == hipSuccess ? GFE_OK : set_error(GFE_EHIP, "crt upload");
+}
+
+F64Args Engine::f64_args(int dup) const {
+    F64Args A;
+    memset(&A, 0, sizeof(A));
+    A.regs = regs; A.ws = reinterpret_cast<double *>(ws); A.zp = reinterpret_cast<const double *>(zp);
+    A.tw = tw64; A.tws = (uint32_t)f64_tw_words(n); A.slots = reinterpret_cast<int4 *>(carry); A.crt = crt64;
+    A.nslots = 1; A.K = f64_k; A.tn = (int)n - 1; A.a = shape.a; A.ng = shape.row_ng; A.dup = dup;
+    return A;
+}
+
+// Register `src` through the passes up to the row pass of `mode`, into `out` (ws or zp); from register 0
+// its range carries are added on the way in, and the caller overwrites the register.
+void Engine::f64_run(uint32_t src, uint32_t *out, int mode) {
+    if (carry_pending && (src != 0 || pend_kind != 3)) flush_carry();
+    F64Args A = f64_args(0);
+    A.reg_off = src * (uint32_t)N;
+    A.ws = reinterpret_cast<double *>(out);
+    A.absorb = carry_pending;
+    if (!shape.whole) f64_launch_fwd(A, shape, stream);
+    f64_launch_mid(A, shape, mode, stream);
+}
+
+void Engine::f64_finish(int dup) {
+    f64_launch_inv(f64_args(dup), shape, stream);
+    pend_kind = 3;
+    carry_pending = true;
+}
+
 void Engine::square(int dup) {
+    if (f64) {
+        f64_run(0, ws, F64_SQUARE);
+        f64_finish(dup);
+        return;
+    }
     if (plan.fuse_sq) {
         flush_carry();
         launch_fused(dup);
@@ -1062,6 +1122,11 @@ void Engine::square(int dup) {
 }
 
 void Engine::mul() {
+    if (zp_f64) {
+        f64_run(0, ws, F64_MUL);
+        f64_finish(0);
+        return;
+    }
     launch_col_fwd(0, ws);
     launch_row(ROW_MUL, ws);
     launch_col_inv(0);
@@ -1070,6 +1135,11 @@ void Engine::mul() {
 
 void Engine::init_multiplicand(uint32_t src) {
     flush_carry();  // register 0 is read but not rewritten
+    zp_f64 = f64;
+    if (f64) {
+        f64_run(src, zp, F64_FWD);
+        return;
+    }
     launch_col_fwd(src, zp);
     launch_row(ROW_FWD, zp);
 }
@@ -1349,6 +1419,8 @@ int gfe_info(const gfe_engine *e, char *buf, size_t len) {
     ss << "NTT" << g.rns << (g.is32 ? "u" : "s");
     if (g.ref_is32 != g.is32) ss << " (reference set NTT" << g.rns << (g.ref_is32 ? "u" : "s") << ")";
     ss << " n=" << g.n << " b=" << g.b << "; " << gfe::plan_str(g.plan, g.n);
+    if (g.f64)
+        ss << "; " << gfe::f64_str(g.n, g.f64_k, g.shape);
     snprintf(buf, len, "%s", ss.str().c_str());
     return GFE_OK;
 }
@@ -1390,7 +1462,18 @@ int gfe_time_squarings(gfe_engine *e, uint32_t count, uint64_t dup_bits, double 
         };
         for (int k = 0; k < 5; ++k) kernel_ms[k] = 0.0;
         int rc = GFE_OK;
-        if (g.plan.fuse_sq) {
+        if (g.f64) {  // as the fused limb plan below
+            g.flush_carry();
+            g.f64_run(0, g.ws, gfe::F64_SQUARE);
+            gfe::F64Args A = g.f64_args(0);
+            rc = time_k([&]() { gfe::f64_launch_inv(A, g.shape, g.stream); }, &kernel_ms[2]);
+            g.pend_kind = 3;
+            g.carry_pending = true;
+            A.absorb = 1;  // as between squarings; ws alone is written
+            if (rc == GFE_OK && !g.shape.whole)
+                rc = time_k([&]() { gfe::f64_launch_fwd(A, g.shape, g.stream); }, &kernel_ms[0]);
+            if (rc == GFE_OK) rc = time_k([&]() { gfe::f64_launch_mid(A, g.shape, gfe::F64_SQUARE, g.stream); }, &kernel_ms[1]);
+        } else if (g.plan.fuse_sq) {
             rc = time_k([&]() { g.launch_fused(0); }, &kernel_ms[0]);
         } else if (g.plan.limb && g.plan.fused) {
             // the fused inverse column pass reads the row pass's output and writes register 0, so it is
@@ -1441,6 +1524,8 @@ int gfe_tune(gfe_engine *e, uint32_t reps) {
         for (const gfe::Plan &P : gfe::candidate_limb_plans(g.n))
             if (!P.fused || gfe::limb_fused_ok(g.b, g.n, P.col_ng)) plans.push_back(P);
     const gfe::Plan orig = g.plan;
+    const bool f64_was = g.f64;
+    g.f64 = false;
     // ms for `count` squarings under plan P (after one untimed), < 0 on a launch error
     auto time_plan = [&](const gfe::Plan &P, uint32_t count, double *ms) -> int {
         g.plan = P;
@@ -1462,7 +1547,7 @@ int gfe_tune(gfe_engine *e, uint32_t reps) {
     std::vector<std::pair<double, size_t>> screen;
     for (size_t k = 0; k < plans.size(); ++k) {
         double ms = 0;
-        if (time_plan(plans[k], reps, &ms) != GFE_OK) { g.plan = orig; return GFE_EHIP; }
+        if (time_plan(plans[k], reps, &ms) != GFE_OK) { g.plan = orig; g.f64 = f64_was; return GFE_EHIP; }
         if (ms >= 0) screen.emplace_back(ms, k);
     }
     std::sort(screen.begin(), screen.end());
@@ -1470,8 +1555,14 @@ int gfe_tune(gfe_engine *e, uint32_t reps) {
     double best_ms = 1e30;
     for (size_t j = 0; j < std::min<size_t>(8, screen.size()); ++j) {
         double ms = 0;
-        if (time_plan(plans[screen[j].second], 8 * reps, &ms) != GFE_OK) { g.plan = orig; return GFE_EHIP; }
+        if (time_plan(plans[screen[j].second], 8 * reps, &ms) != GFE_OK) { g.plan = orig; g.f64 = f64_was; return GFE_EHIP; }
         if (ms >= 0 && ms < best_ms) { best_ms = ms; best = plans[screen[j].second]; }
+    }
+    if (g.f64_k) {  // the double-precision transform against the fastest plan
+        g.f64 = true;
+        double ms = 0;
+        if (time_plan(best, 8 * reps, &ms) != GFE_OK) { g.plan = orig; g.f64 = f64_was; return GFE_EHIP; }
+        g.f64 = ms >= 0 && ms < best_ms;
     }
     g.plan = best;
     g.carry_pending = false;
@@ -1549,7 +1640,8 @@ int gfe_rebase(gfe_engine *e, uint32_t b) {
         for (int k = 0; k < 4; ++k) g.bm4[k] = gfe::mulw_const(b % g.pr4.p[k], g.pr4.p[k]);
     }
     g.plan = g.can_limb ? gfe::engine_plan_for(b, g.n) : gfe::default_plan(g.n);
-    return g.check("rebase");
+    const int rc = g.f64_select();
+    return rc != GFE_OK ? rc : g.check("rebase");
 }
 
 int gfe_set_plan(gfe_engine *e, const int32_t plan[6]) {
@@ -1563,6 +1655,7 @@ int gfe_set_plan(gfe_engine *e, const int32_t plan[6]) {
     e->eng.flush_carry();
     if (hipStreamSynchronize(e->eng.stream) != hipSuccess) return set_error(GFE_EHIP, "set_plan sync");
     e->eng.plan = P;
+    e->eng.f64 = false;
     return GFE_OK;
 }
 

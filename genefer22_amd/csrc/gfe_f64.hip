@@ -1,0 +1,443 @@
+// gfe_f64.hip -- kernels and host constants of the double-precision limb transform (gfe_f64.h).
+//
+// One squaring is three launches: forward column pass (digits -> residues of every prime), row pass
+// (forward, square, inverse), inverse column pass with the CRT and the carry; or, where a prime's
+// transform fits one workgroup's LDS (2^14 limbs), two: the whole transform of each prime, then the CRT
+// and the carry.
+#include "gfe_f64_host.h"
+
+#include <cstring>
+#include <mutex>
+
+namespace gfe {
+
+// Work of workgroup blockIdx.x of a launch of `per` workgroups a slot: slot and index within it.  Slots
+// follow each other, or with pin slot s takes workgroups of XCD s mod 8 only (workgroups go to the 8
+// XCDs in turn).
+struct F64Job {
+    uint32_t slot, w;
+    F64CrtP c;
+    int K;
+    bool run;
+};
+__device__ __forceinline__ F64Job f64_job(const F64Args &A, uint32_t per) {
+    F64Job J;
+    const uint32_t id = blockIdx.x;
+    if (A.K) {
+        J.slot = 0; J.w = id; J.c = (F64CrtP)A.crt; J.K = A.K; J.run = true;
+        return J;
+    }
+    if (A.pin) {
+        const uint32_t i = id >> 3, g = i / per;
+        J.slot = (g << 3) + (id & 7u);
+        J.w = i - g * per;
+    } else {
+        J.slot = id / per;
+        J.w = id - J.slot * per;
+    }
+    J.run = J.slot < A.nslots && !(A.active && !A.active[J.slot]);
+    J.c = (F64CrtP)(A.crt + (J.run ? J.slot : 0));
+    J.run = J.run && J.c->n == A.tn + 1;  // a mixed batch's slots of another n
+    J.K = J.c->K;
+    return J;
+}
+// Column block of index x of nb (XCD by XCD, unless the slot is on one).
+__device__ __forceinline__ unsigned f64_block(const F64Args &A, unsigned x, unsigned nb) { return A.pin ? x : xcd_block(x, nb); }
+
+// C / 16 workgroups a slot, or with `split` one per column block and prime: 16 columns for all primes
+// from one read of the digits, or for one.
+template <int LOGG>
+__global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_fwd(F64Args A, int split) {
+    extern __shared__ double lds64[];
+    constexpr int LOGE = F64_COL_E;
+    const uint32_t M = 1u << A.tn, C = M >> LOGG, nb = C / 16, t = threadIdx.x;
+    const F64Job J = f64_job(A, split ? 3 * nb : nb);
+    if (!J.run) return;
+    const F64CrtP c = J.c;
+    const int K = J.K, k0 = split ? (int)(J.w / nb) : 0, k1 = split ? k0 + 1 : K;
+    if (k0 >= K) return;
+    const unsigned blk = f64_block(A, split ? J.w - k0 * nb : J.w, nb);
+    int2 d[1 << LOGE];
+    f64_load_digits<LOGE, LOGG>(d, A.regs + J.slot * A.reg_stride + A.reg_off,
+                                A.absorb ? A.slots + J.slot * A.slot_stride : nullptr, C, blk, t);
+    const double bd = c->bd;
+    const bool reduce = c->big == 2;
+    double *ws = A.ws + J.slot * A.ws_stride;
+#pragma unroll 1
+    for (int k = k0; k < k1; ++k)
+        f64_col_fwd<LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, d, ws + (size_t)k * M, A.tw + (size_t)k * A.tws, C, blk, t,
+                                lds64, bd, reduce);
+}
+
+constexpr int f64_row_threads(int logg) { return logg > 12 ? 1 << (logg - 4) : 256; }
+
+// 3 2^a / ng workgroups a slot.
+template <int LOGG, int MODE>
+__global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
+    extern __shared__ double lds64[];
+    constexpr uint32_t SPR = 1u << (LOGG - 4);
+    const uint32_t nb = (1u << A.a) / (uint32_t)A.ng;
+    const F64Job J = f64_job(A, 3 * nb);
+    const int k = (int)(J.w / nb);
+    if (!J.run || k >= J.K) return;
+    const uint32_t t = threadIdx.x, q = t / SPR, s = t % SPR;
+    uint32_t row = (J.w - (uint32_t)k * nb) * (uint32_t)A.ng + q;
+    if constexpr (SPR >= 64) row = __builtin_amdgcn_readfirstlane(row);
+    const size_t at = J.slot * A.ws_stride + ((size_t)k << A.tn) + ((size_t)row << LOGG);
+    const F64Mod md{J.c->p[k], J.c->pinv[k]};
+    double *data = A.ws + at;
+    const auto load = [&](double (&x)[16], uint32_t base, auto yl) {
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) x[rr] = data[base + ((uint32_t)rr << decltype(yl)::value)];
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) x[rr] = md.red(x[rr]);
+    };
+    f64_row_pass<LOGG, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s, lds64 + q * f64_row_words(LOGG),
+                             MODE == F64_EITHER && A.mulf[J.slot]);
+}
+
+// 3 workgroups a slot, 2^LOGG / 16 threads: a prime's whole transform, from the digits.
+template <int LOGG, int MODE>
+__global__ void __launch_bounds__(1 << (LOGG - 4)) k64_whole(F64Args A) {
+    extern __shared__ double lds64[];
+    const F64Job J = f64_job(A, 3);
+    const int k = (int)J.w;
+    if (!J.run || k >= J.K) return;
+    const F64CrtP c = J.c;
+    const uint32_t s = threadIdx.x;
+    const F64Mod md{c->p[k], c->pinv[k]};
+    const double bd = c->bd;
+    const bool reduce = c->big != 0;
+    const int2 *src = reinterpret_cast<const int2 *>(A.regs + J.slot * A.reg_stride + A.reg_off);
+    const int4 *ls = A.absorb ? A.slots + J.slot * A.slot_stride : nullptr;
+    const size_t at = J.slot * A.ws_stride + ((size_t)k << LOGG);
+    const auto load = [&](double (&x)[16], uint32_t base, auto yl) {
+        constexpr int YL = decltype(yl)::value;
+        int2 d[16];
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) d[rr] = src[base + ((uint32_t)rr << YL)];
+        if (ls && (base & 15u) < 2) {  // as f64_load_digits
+            const uint32_t q = base & 1u;
+            int2 e[16];
+#pragma unroll
+            for (int rr = 0; rr < 16; ++rr) e[rr] = reinterpret_cast<const int2 *>(ls + ((base + ((uint32_t)rr << YL)) >> 4))[q];
+#pragma unroll
+            for (int rr = 0; rr < 16; ++rr) {
+                d[rr].x += e[rr].x;
+                d[rr].y += q == 0 ? e[rr].y : 0;
+            }
+        }
+#pragma unroll
+        for (int rr = 0; rr < 16; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
+    };
+    f64_row_pass<LOGG, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds64,
+                             MODE == F64_EITHER && A.mulf[J.slot]);
+}
+
+template <int K, int LOGG>
+__device__ __forceinline__ void f64_inv_body(const F64Args &A, const F64Job &J, int dup, double *lds) {
+    constexpr int LOGE = F64_COL_E;
+    const uint32_t M = 1u << A.tn, C = M >> LOGG, t = threadIdx.x;
+    const unsigned blk = f64_block(A, J.w, C / 16);
+    const double *ws = A.ws + J.slot * A.ws_stride;
+    double x[K][1 << LOGE];
+#pragma unroll
+    for (int k = 0; k < K; ++k) f64_col_load<LOGE, LOGG>(x[k], ws + (size_t)k * M, C, blk, t);
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+        f64_col_inv<LOGE, LOGG>(F64Mod{J.c->p[k], J.c->pinv[k]}, x[k], A.tw + (size_t)k * A.tws, t, lds);
+    f64_norm_store<K, LOGE, LOGG>(J.c, x, C, blk, t, dup, A.regs + J.slot * A.reg_stride + A.reg_off,
+                                  A.slots + J.slot * A.slot_stride);
+}
+
+// C / 16 workgroups a slot.
+template <int LOGG>
+__global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_inv(F64Args A) {
+    extern __shared__ double lds64[];
+    const F64Job J = f64_job(A, (1u << A.tn) >> (LOGG + 4));
+    if (!J.run) return;
+    const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
+    if (J.K == 2) f64_inv_body<2, LOGG>(A, J, dup, lds64);
+    else f64_inv_body<3, LOGG>(A, J, dup, lds64);
+}
+
+template <int K>
+__device__ __forceinline__ void f64_norm_body(const F64Args &A, const F64Job &J, int dup) {
+    const uint32_t M = 1u << A.tn, i0 = J.w * F64_NORM_RANGE + threadIdx.x;
+    const double *ws = A.ws + J.slot * A.ws_stride;
+    double r[F64_NORM_PER][K];
+#pragma unroll
+    for (int j = 0; j < F64_NORM_PER; ++j)
+#pragma unroll
+        for (int k = 0; k < K; ++k) r[j][k] = ws[(size_t)k * M + i0 + j * F64_NORM_T];
+#pragma unroll
+    for (int j = 0; j < F64_NORM_PER; ++j)
+        f64_norm_limb<K>(J.c, r[j], dup, i0 + j * F64_NORM_T, M, A.regs + J.slot * A.reg_stride + A.reg_off,
+                         A.slots + J.slot * A.slot_stride);
+}
+
+// The normalisation after k64_whole: M / F64_NORM_RANGE workgroups a slot.
+__global__ void __launch_bounds__(F64_NORM_T) k64_norm(F64Args A) {
+    const F64Job J = f64_job(A, (1u << A.tn) / F64_NORM_RANGE);
+    if (!J.run) return;
+    const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
+    if (J.K == 2) f64_norm_body<2>(A, J, dup);
+    else f64_norm_body<3>(A, J, dup);
+}
+
+// Register 0 of the slots in grid.y with its pending range carries, balanced (f64_flush_body).
+__global__ void __launch_bounds__(256) k64_flush(F64Args A) {
+    const uint32_t s = blockIdx.y, w = blockIdx.x * 256u + threadIdx.x;
+    if (A.active && !A.active[s]) return;
+    const F64CrtP c = (F64CrtP)(A.crt + s);
+    if (c->n == 0 || w >= (1u << c->n) / 32) return;
+    f64_flush_body(A.regs + s * A.reg_stride, A.slots + s * A.slot_stride, c->b, w);
+}
+
+__global__ void __launch_bounds__(256) k64_carry(F64Args A) {
+    const uint32_t s = blockIdx.y, w = blockIdx.x * 256u + threadIdx.x;
+    if (A.active && !A.active[s]) return;
+    const F64CrtP c = (F64CrtP)(A.crt + s);
+    if (c->n == 0 || w >= (1u << c->n) / 32) return;
+    f64_carry_body(A.regs + s * A.reg_stride, A.slots + s * A.slot_stride, (1u << c->n) / 32, c->b, w);
+}
+
+struct F64TwArgs {
+    double *tw;
+    uint32_t words;                       // per prime
+    int bits;                             // log2 M
+    double p[F64_PRIMES], pinv[F64_PRIMES];
+    double pw[F64_PRIMES][24];            // psi^(2^i)
+};
+
+// Psi[j] = psi^bitrev(j): bit i of j contributes psi^(2^(bits - 1 - i)).
+__global__ void __launch_bounds__(256) k64_twiddles(F64TwArgs A) {
+    const uint32_t j = blockIdx.x * 256u + threadIdx.x;
+    const int k = blockIdx.y;
+    if (j >= A.words) return;
+    const F64Mod md{A.p[k], A.pinv[k]};
+    double w = 1.0;
+    for (int i = 0; i < A.bits; ++i)
+        if ((j >> i) & 1u) w = md.mul(w, A.pw[k][A.bits - 1 - i]);
+    A.tw[(size_t)k * A.words + j] = w;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Host constants
+
+static uint64_t mul64(uint64_t a, uint64_t b, uint64_t p) { return (uint64_t)((unsigned __int128)a * b % p); }
+static uint64_t pow64(uint64_t a, uint64_t e, uint64_t p) {
+    uint64_t r = 1;
+    for (; e; e >>= 1, a = mul64(a, a, p))
+        if (e & 1) r = mul64(r, a, p);
+    return r;
+}
+static uint64_t inv64(uint64_t a, uint64_t p) { return pow64(a % p, p - 2, p); }
+static double bal64(uint64_t a, uint64_t p) { return a > p / 2 ? -(double)(p - a) : (double)a; }
+
+// Largest doubled coefficient against the primes' product.  Limbs are at most L = (b/2 + 4)(b + 1),
+// but for the first two of a range of 16, which enter with the range carry added: the first's
+// digits take |u0| <= b/2 and |u1| <= 0.55 b + G / b + 2, the second's low digit v <= G + 2, where
+// G >= |g4| is the largest coefficient over b^4.  By Cauchy-Schwarz a doubled coefficient is at most
+// X = 2 (M / 16)(L0^2 + L1^2 + 14 L^2), which gives G in turn: the pair is settled by iteration.
+// Three primes need X < 0.3 P (the mixed-radix digit v3 is then the centred one, whatever the
+// rounding of its quotient); with two the last digit's quotient has the larger rounding: 0.1 P.
+static bool f64_bound(uint32_t b, uint32_t n, int K) {
+    const long double bb = b, M = (long double)((uint64_t)1 << (n - 1));
+    long double P = 1;
+    for (int k = 0; k < K; ++k) P *= (long double)F64_P[k];
+    const long double L = (bb / 2 + 4) * (bb + 1);
+    long double G = M / 2 + 4, X = 0;
+    for (int it = 0; it < 64; ++it) {
+        const long double L0 = (bb + 5) + bb * (1.05L * bb + 6 + G / bb + 2), L1 = L + G + 2;
+        X = 2 * (M / 16) * (L0 * L0 + L1 * L1 + 14 * L * L);
+        const long double g = X / (bb * bb * bb * bb) + 4;
+        if (g <= G) break;
+        G = g * 1.001L;
+        if (G > bb * bb || G > 1.0e8L) return false;
+    }
+    return G <= bb * bb && G <= 1.0e8L && X < (K == 3 ? 0.3L : 0.1L) * P;
+}
+
+int f64_primes(uint32_t b, uint32_t n) {
+    if (n < 12 || n > 23 || b < 1024) return 0;
+    if (f64_bound(b, n, 2)) return 2;
+    // three primes: p1 in three base-b pieces
+    return (b >= (1u << 17) && f64_bound(b, n, 3)) ? 3 : 0;
+}
+
+F64Crt make_f64_crt(uint32_t n, uint32_t b, int K) {
+    F64Crt c;
+    memset(&c, 0, sizeof(c));
+    for (int k = 0; k < 3; ++k) {
+        const uint64_t p = F64_P[k];
+        c.p[k] = (double)p;
+        c.pinv[k] = 1.0 / (double)p;
+        // n - 3 of the transform's n - 1 levels are run and undone: 2^(n-3) comes out of the inverse
+        const uint64_t s = inv64((uint64_t)1 << (n - 3), p);
+        c.s[0][k] = bal64(s, p);
+        c.s[1][k] = bal64(mul64(s, 2, p), p);
+    }
+    c.i12 = bal64(inv64(F64_P[0], F64_P[1]), F64_P[1]);
+    c.i13 = bal64(inv64(F64_P[0], F64_P[2]), F64_P[2]);
+    c.i23 = bal64(inv64(F64_P[1], F64_P[2]), F64_P[2]);
+    auto split = [&](__int128 x, int pieces, double *w, uint32_t *wl) {
+        for (int i = 0; i < pieces; ++i) {
+            __int128 r = x;
+            if (i < pieces - 1) {
+                r = x % b;
+                if (r > b / 2) r -= b;
+                x = (x - r) / b;
+            }
+            w[i] = (double)(int64_t)r;
+            wl[i] = (uint32_t)(int64_t)r;
+        }
+    };
+    split((__int128)F64_P[0], K == 3 ? 3 : 5, c.w1, c.w1l);
+    if (K == 3) split((__int128)F64_P[0] * F64_P[1], 5, c.w2, c.w2l);
+    c.bd = (double)b;
+    c.binv = 1.0 / (double)b;
+    c.qb = 0.25 * c.binv;
+    c.b = b;
+    const double limb = 1.1 * (double)b * (double)b + (double)((uint64_t)1 << n);  // range carry included
+    c.big = limb > 0x1p50 ? 2 : limb > 0x1p48 ? 1 : 0;
+    c.n = (int32_t)n;
+    c.K = K;
+    return c;
+}
+
+int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
+    F64TwArgs A;
+    memset(&A, 0, sizeof(A));
+    A.tw = tw;
+    A.words = (uint32_t)f64_tw_words(n);
+    A.bits = (int)n - 1;
+    for (int k = 0; k < F64_PRIMES; ++k) {
+        const uint64_t p = F64_P[k];
+        A.p[k] = (double)p;
+        A.pinv[k] = 1.0 / (double)p;
+        uint64_t w = pow64(F64_G[k], (p - 1) >> n, p);  // a primitive 2M-th root, M = 2^(n-1)
+        for (int i = 0; i < A.bits; ++i, w = mul64(w, w, p)) A.pw[k][i] = bal64(w, p);
+    }
+    hipLaunchKernelGGL(k64_twiddles, dim3((A.words + 255) / 256, F64_PRIMES, 1), dim3(256), 0, stream, A);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// ------------------------------------------------------------------------------------------------
+// Dispatch
+
+
+// One candidate, timed on MI355X (us per squaring, three primes unless said).  Up to 2^12 limbs the
+// two launches with a prime's transform in one workgroup beat the three (2^11 limbs 9.3 against
+// 13.1, 2^12 11.0 against 13.4; at 2^13 one workgroup's arithmetic takes longer, 16.8 against 14.0).
+// With three passes, up to 2^19 limbs each is bound by latency, so the shapes that win are those with
+// the most workgroups: short columns, one wave per row workgroup, a workgroup per prime in the
+// forward column pass (2^15 limbs: 15.0 with 2^5-point columns, 15.5 with 2^6, 16.3 with all primes
+// in one workgroup; 2^18: 23.5 with 2^6, 25.3 with 2^7).  From 2^20 limbs the passes are bound by
+// memory and fp64 issue and longer columns pay, the digits then being read once for all primes
+// (2^21 limbs: 81.8 with 2^8-point columns, 89.6 with 2^7).  The integer passes at the same sizes:
+// 14.5, 15.6, 15.9, 16.5, 18.8, 20.0, 25.8, 36.9, 41.8, 57.8, 89.3 at n = 12, 13, .., 22 (the last
+// eight limbs of two digits where those are exact).
+F64Shape f64_shape(uint32_t n, uint32_t slots) {
+    F64Shape S;
+    const int tn = (int)n - 1;
+    S.whole = n <= 13;
+    S.a = tn <= 15 ? 5 : tn <= 18 ? 6 : tn == 19 ? 7 : 8;
+    S.split = tn <= 19;
+    const int spr = 1 << (tn - S.a - 4);
+    S.row_ng = spr >= 64 ? 1 : 64 / spr;
+    return S;
+}
+
+std::string f64_str(uint32_t n, int K, const F64Shape &S) {
+    std::string s = "squares in doubles (limbs of two digits, " + (K ? std::to_string(K) : std::string("2 or 3")) + " 49-bit primes, ";
+    if (S.whole) return s + "a prime's 2^" + std::to_string(n - 1) + " limbs in one workgroup)";
+    return s + "cols 2^" + std::to_string(S.a) + " x rows 2^" + std::to_string((int)n - 1 - S.a) + ")";
+}
+
+typedef void (*F64ColFn)(F64Args, int);
+typedef void (*F64Fn)(F64Args);
+
+template <int LOGG = F64_COL_MIN>
+static F64ColFn fwd_fn(int a) {
+    if constexpr (LOGG > F64_COL_MAX) return nullptr;
+    else return a == LOGG ? k64_col_fwd<LOGG> : fwd_fn<LOGG + 1>(a);
+}
+template <int LOGG = F64_COL_MIN>
+static F64Fn inv_fn(int a) {
+    if constexpr (LOGG > F64_COL_MAX) return nullptr;
+    else return a == LOGG ? k64_col_inv<LOGG> : inv_fn<LOGG + 1>(a);
+}
+template <int MODE, int LOGG = F64_ROW_MIN>
+static F64Fn row_fn(int logg) {
+    if constexpr (LOGG > F64_ROW_MAX) return nullptr;
+    else return logg == LOGG ? k64_row<LOGG, MODE> : row_fn<MODE, LOGG + 1>(logg);
+}
+template <int MODE, int LOGG = F64_WHOLE_MIN>
+static F64Fn whole_fn(int logg) {
+    if constexpr (LOGG > F64_WHOLE_MAX) return nullptr;
+    else return logg == LOGG ? k64_whole<LOGG, MODE> : whole_fn<MODE, LOGG + 1>(logg);
+}
+static F64Fn mid_fn(bool whole, int mode, int logg) {
+    switch (mode) {
+        case F64_SQUARE: return whole ? whole_fn<F64_SQUARE>(logg) : row_fn<F64_SQUARE>(logg);
+        case F64_MUL: return whole ? whole_fn<F64_MUL>(logg) : row_fn<F64_MUL>(logg);
+        case F64_FWD: return whole ? whole_fn<F64_FWD>(logg) : row_fn<F64_FWD>(logg);
+        default: return whole ? whole_fn<F64_EITHER>(logg) : row_fn<F64_EITHER>(logg);
+    }
+}
+
+// Workgroups of a launch of `per` a slot (f64_job).
+static dim3 f64_grid(const F64Args &A, uint32_t per) {
+    return dim3(A.pin ? 8 * per * ((A.nslots + 7) / 8) : per * A.nslots);
+}
+
+void f64_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream) {
+    const unsigned nb = 1u << (A.tn - S.a - 4), T = 16u << (S.a - F64_COL_E);
+    hipLaunchKernelGGL(fwd_fn(S.a), f64_grid(A, S.split ? 3 * nb : nb), dim3(T), (size_t)128 << S.a, stream, A, S.split);
+}
+
+void f64_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream) {
+    if (S.whole) {
+        hipLaunchKernelGGL(mid_fn(true, mode, A.tn), f64_grid(A, 3), dim3(1u << (A.tn - 4)), (size_t)8 * f64_row_words(A.tn), stream, A);
+        return;
+    }
+    const int L = A.tn - S.a;
+    hipLaunchKernelGGL(mid_fn(false, mode, L), f64_grid(A, 3 * ((1u << S.a) / S.row_ng)), dim3((unsigned)S.row_ng << (L - 4)),
+                       (size_t)8 * S.row_ng * f64_row_words(L), stream, A);
+}
+
+void f64_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream) {
+    if (S.whole) {
+        hipLaunchKernelGGL(k64_norm, f64_grid(A, (1u << A.tn) / F64_NORM_RANGE), dim3(F64_NORM_T), 0, stream, A);
+        return;
+    }
+    const unsigned T = 16u << (S.a - F64_COL_E);
+    hipLaunchKernelGGL(inv_fn(S.a), f64_grid(A, 1u << (A.tn - S.a - 4)), dim3(T), (size_t)128 << S.a, stream, A);
+}
+
+void f64_launch_flush(const F64Args &A, hipStream_t stream) {
+    const dim3 grid(((1u << (A.tn - 4)) + 255) / 256, A.nslots);
+    hipLaunchKernelGGL(k64_flush, grid, dim3(256), 0, stream, A);
+    hipLaunchKernelGGL(k64_carry, grid, dim3(256), 0, stream, A);
+}
+
+void f64_set_lds_attributes() {
+    static std::once_flag once;
+    std::call_once(once, []() {
+        auto set = [](const void *f) {
+            if (f) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        };
+        for (int a = F64_COL_MIN; a <= F64_COL_MAX; ++a) {
+            set((const void *)fwd_fn(a));
+            set((const void *)inv_fn(a));
+        }
+        for (int m = 0; m < 4; ++m) {
+            for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, l));
+            for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, l));
+        }
+        (void)hipGetLastError();
+    });
+}
+
+}  // namespace gfe

@@ -79,7 +79,7 @@ int gfe_load(gfe_engine *e, uint32_t num_regs, const void *buf, size_t size);
 /* transform::getError, src/transform.h:71 -- always 0: the arithmetic is exact. */
 double gfe_get_error(const gfe_engine *e);
 /* transform::info, src/transform.h:72 -- prime set computed in (and the reference's set when it
- * differs) and pass plan as text. */
+ * differs), pass plan and, while the engine squares in doubles, that transform's shape as text. */
 int gfe_info(const gfe_engine *e, char *buf, size_t len);
 /* No counterpart in the reference (one candidate per process there): moves the engine to base b of
  * the same n, for servers that keep engines between candidates instead of building their twiddle
@@ -107,11 +107,16 @@ const char *gfe_last_error(void);
 int gfe_time_squarings(gfe_engine *e, uint32_t count, uint64_t dup_bits, double *ms, double *kernel_ms);
 
 /* Autotuner: times every admissible pass plan for this engine's n on the device and keeps the
- * fastest (the reference's splitter + engines::tune, src/ocl.h:31-90, src/transformGPU.h:851-900).
- * `reps` squarings per plan.  The chosen plan is reported by gfe_info. */
+ * fastest, or the double-precision transform where that is (the reference's splitter + engines::tune,
+ * src/ocl.h:31-90, src/transformGPU.h:851-900).  `reps` squarings per plan.  The chosen plan is reported by gfe_info. */
 int gfe_tune(gfe_engine *e, uint32_t reps);
 
-/* The pass plan as {a (column levels), column E log2, columns per workgroup, row E log2, rows per
+/* An engine squares, and forms multiplicands, in a double-precision limb transform (exact: integer
+ * residues of 49-bit primes in doubles) wherever that is exact for its (b, n), which leaves out only
+ * bases below 2,300 at n >= 21.  The plan below shapes the integer passes: they run where it is not,
+ * and from gfe_set_plan on (gfe_tune keeps whichever is faster, gfe_rebase goes back to the default).
+ *
+ * The pass plan as {a (column levels), column E log2, columns per workgroup, row E log2, rows per
  * workgroup, flags: bit 0 factored row twiddles, bit 1 all-prime column passes with the CRT and
  * carry fused into the inverse one, bit 2 persistent column passes, bit 3 compile-time passes,
  * bit 4 the squaring in one workgroup (n <= 13), bit 5 the two-digit-limb transform (see
@@ -130,7 +135,7 @@ int gfe_set_plan(gfe_engine *e, const int32_t plan[6]);
  * GFE_EINVAL; gfe_candidate_plans writes how many plans the autotuner times at n to *count and,
  * when plans is not null, the first min(max, count) of them (6 int32 each). */
 int gfe_default_plan(uint32_t n, uint32_t capacity, int32_t plan[6]);
-/* The plan gfe_create gives an engine of (b, n): gfe_default_plan(n, 0), or for the (b, n) the
+/* The (integer) plan gfe_create gives an engine of (b, n): gfe_default_plan(n, 0), or for the (b, n) the
  * two-digit-limb transform covers (flags bit 5: limbs d_2j + b d_2j+1 of base b^2, N/2-point
  * transforms over four 31-bit primes; a and the row fields then describe the N/2-point transform)
  * its default plan, with the inverse column pass fused to the normalisation (flags 42) where that

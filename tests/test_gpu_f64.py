@@ -1,0 +1,92 @@
+"""The double-precision limb transform (what an engine squares with unless gfe_set_plan selects the
+integer passes) against the oracle, and its digits against the integer passes' own: at every n's
+shape, at the bases where the prime count, the limb conversion or the rule changes, from extreme
+digits, and through every use of the registers that has to apply its pending carries."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def canon(O, d, n, b):
+    return O.unbalance(d, n, b)
+
+
+def largest_two_prime_base(n):
+    from test_f64 import bound
+    lo, hi = 1 << 17, 1 << 25
+    while hi - lo > 1:
+        m = (lo + hi) // 2
+        lo, hi = (m, hi) if bound(m, n, 2) else (lo, m)
+    return lo
+
+
+@pytest.mark.parametrize("n", range(12, 24))
+def test_digits_equal_the_integer_passes(gfe, n):
+    """Random and extreme digits, doubled or not: the digits read back are those of the integer
+    passes, bit for bit, at the edges of the two- and three-prime ranges."""
+    e = largest_two_prime_base(n)
+    bases = [{21: 1148, 22: 1622, 23: 2292}.get(n, 1026), e - (e & 1), e + 2 - (e & 1), 15300000, 31987654, 32200000, 1999999998]
+    for b in bases if n <= 17 else bases[::2]:
+        t, u = gfe.Transform(b, n), gfe.Transform(b, n)
+        u.set_plan(u.get_plan())
+        assert "in doubles" in t.info() and "in doubles" not in u.info()
+        rs = np.random.RandomState(n)
+        N, h = 1 << n, b // 2 + 4
+        for d in (rs.randint(-((b - 1) // 2), b // 2 + 1, N), np.full(N, -h), np.where(np.arange(N) % 2 == 0, h, -h)):
+            for x in (t, u):
+                x.set_digits(d.astype(np.int32))
+                for dup in (1, 0, 1, 1):
+                    x.square_dup(dup)
+            got = t.get_digits()
+            assert np.abs(got.astype(np.int64)).max() <= h
+            assert np.array_equal(got, u.get_digits()), (b, n)
+        t.close()
+        u.close()
+
+
+@pytest.mark.parametrize("b,n", [(1026, 12), (146950, 12), (1999999998, 12), (777777778, 13), (1999999266, 14),
+                                 (1619951882, 15), (333333334, 17)])
+def test_every_use_of_the_registers_matches_the_oracle(gfe, oracle, b, n):
+    rs = np.random.RandomState(n)
+    t, o = gfe.Transform(b, n), oracle.Engine(b, n)
+    t.set(3); o.set(3)
+    a = oracle.balance(rs.randint(0, b, 1 << n).astype(np.int32), n, b)
+    t.set_digits(a, 1); o.set_digits(a, 1)
+    for k in range(6):
+        t.square_dup(k & 1); o.square_dup(k & 1)
+    t.init_multiplicand(0); o.init_multiplicand(0)      # of register 0, its carries pending
+    t.square_dup(True); o.square_dup(True)
+    t.mul(); o.mul()
+    t.copy(2, 0); o.copy(2, 0)
+    t.mul(1); o.mul(1)                                   # another multiplicand
+    t.square_mul(7); o.square_mul(7)
+    plan = t.get_plan()
+    t.square_dup(False); o.square_dup(False)
+    t.set_plan(plan)                                     # the integer passes, carries pending
+    t.square_dup(True); o.square_dup(True)
+    t.mul(); o.mul()                                     # the multiplicand of the other transform
+    t.rebase(b)                                          # back to doubles
+    t.square_dup(False); o.square_dup(False)
+    data = t.save_context(3)
+    for r in (0, 1, 2):
+        assert np.array_equal(canon(oracle, t.get_digits(r), n, b), canon(oracle, o.get_digits(r), n, b)), r
+    u = gfe.Transform(b, n)
+    assert u.read_context(data, 3)
+    assert np.array_equal(canon(oracle, u.get_digits(0), n, b), canon(oracle, o.get_digits(0), n, b))
+    t.time_squarings(3, 0b101)
+    t.time_squarings(2, 0b1, per_kernel=True)
+    for dup in (1, 0, 1, 1, 0, 0):
+        o.square_dup(dup)
+    assert np.array_equal(canon(oracle, t.get_digits(0), n, b), canon(oracle, o.get_digits(0), n, b))
+
+
+def test_refused_bases_keep_the_integer_passes(gfe, oracle):
+    """b = 1024 at n = 23 is outside the rule (the last piece may exceed the limb's size)."""
+    n, b = 23, 1026
+    t, o = gfe.Transform(b, n), oracle.Engine(b, n)
+    assert "in doubles" not in t.info()
+    d = np.full(1 << n, b // 2, dtype=np.int32)
+    t.set_digits(d); o.set_digits(d, 0)
+    t.square_dup(True); o.square_dup(True)
+    assert np.array_equal(canon(oracle, t.get_digits(), n, b), canon(oracle, o.get_digits(0), n, b))
