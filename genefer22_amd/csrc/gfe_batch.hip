@@ -7,6 +7,9 @@
 //   carry : cap x N/8 int64 workgroup carries (or segment carries of fused plans)
 //   crt   : cap CrtConst, slots: cap SlotInfo (b, prime count, prime width)
 //   tw    : 2 x 3 x N uint32 twiddles (31-bit set, 32-bit set), shared by all slots
+//   crt64, tw64 : the same for the double-precision limb transform (gfe_f64.h), in which a batch squares
+//           unless gfe_batch_set_plan selects the integer passes; ws, zp and carry hold its residues
+//           and range carries then
 // Every kernel runs over grid.z = slot and exits at once for a slot that is not active in the
 // current round (per-round activity and dup flags are uploaded per 64-round block).  Each slot
 // runs its own program: squaring runs (the PRP loop, the Gerbicz-Li check's squarings) and
@@ -288,6 +291,7 @@ struct Slot {
     std::vector<Words> w;             // exponents w_j, j < 2^depth / 2
     std::vector<uint64_t> mu_hash;    // gethash64 of mu_0, mu_1, ...
     uint64_t pkey = 0;                // proof key: gethash64 of v1 (after the last phase)
+    bool zp64 = false;                // the multiplicand is the double-precision transform's
     std::deque<Item> q;
     uint64_t pos = 0;                 // progress inside the head run
     uint64_t res64 = 0, old64 = 0, hash64 = 0, h1 = 0;
@@ -357,12 +361,13 @@ struct Batch {
     // destroyed only after the stream has drained: a launch of it may still be queued.  Captured
     // kernels record no memset (fill kernels only).
     static constexpr size_t MAX_GRAPHS = 16;
+    // (key: the plan, or the double-precision transform with or without multiplying rounds)
     struct BlockGraph { int rounds; uint32_t zl; uint64_t key; hipGraphExec_t exec; uint64_t last_use; };
     std::vector<BlockGraph> graphs;
     uint64_t graph_uses = 0;
     bool use_graphs = true;
     uint64_t plan_key() const;
-    hipGraphExec_t block_graph(int rounds);
+    hipGraphExec_t block_graph(int rounds, bool has_mul = false);
     void drop_graphs();
     int run_block(int rounds, uint32_t nact, bool has_mul = false, uint32_t nbig = 0);
     // The single-workgroup squaring at n = 13 pays off once 128 or more slots are active: with
@@ -383,6 +388,16 @@ struct Batch {
     // 512 slots, measured on MI355X: 0.367 ms per round either way; n = 20, one slot: 52.9 us against
     // 54.8 us with the carry kernel).
     bool carries_pending = false;
+    // The double-precision limb transform: selected until gfe_batch_set_plan (n <= F64_ALL_BASES_N), and
+    // in use while a power run holds a multiplicand in it.  Its range carries stay pending from round
+    // to round in every shape.  carry64: the form `carry` holds.
+    bool f64 = false, carry64 = false;
+    F64Shape shape;
+    double *tw64 = nullptr;
+    F64Crt *crt64 = nullptr, *crt64_host = nullptr;
+    bool mode64() const;
+    int use_mode(bool m);
+    F64Args args64(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf) const;
     bool defer_carry() const { return plan.spec && !plan.pipe && !plan.fused && (int)n - plan.a >= 11; }
     void flush_carries();
     int zero_carries();
@@ -418,7 +433,7 @@ struct Batch {
     void launch_row(const BArgs &A, int mode);
     void launch_col_inv(const BArgs &A);
     void launch_norm_carry(const BArgs &A);
-    void square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf = nullptr);
+    void square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf = nullptr, bool has_mul = true);
     void op_copy(const uint8_t *active, uint32_t dst, uint32_t src);
     void op_set(const uint8_t *active, uint32_t dst, int32_t value);
     void op_initmul(const uint8_t *active, uint32_t src);
@@ -461,8 +476,8 @@ void Batch::drop_graphs() {
 
 // The instantiated graph of a block of `rounds` squaring rounds at the current grid depth and plan
 // (captured on first use; null on failure).
-hipGraphExec_t Batch::block_graph(int rounds) {
-    const uint64_t key = plan_key();
+hipGraphExec_t Batch::block_graph(int rounds, bool has_mul) {
+    const uint64_t key = mode64() ? 1 + (has_mul ? 1 : 0) : plan_key();
     for (auto &g : graphs)
         if (g.rounds == rounds && g.zl == zdim() && g.key == key) {
             g.last_use = ++graph_uses;
@@ -471,7 +486,7 @@ hipGraphExec_t Batch::block_graph(int rounds) {
     hipGraph_t graph = nullptr;
     if (hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal) != hipSuccess) return nullptr;
     for (int r = 0; r < rounds; ++r)
-        square(act_dev + (size_t)r * cap, dup_dev + (size_t)r * cap, mul_dev + (size_t)r * cap);
+        square(act_dev + (size_t)r * cap, dup_dev + (size_t)r * cap, mul_dev + (size_t)r * cap, has_mul);
     if (hipStreamEndCapture(stream, &graph) != hipSuccess || !graph) {
         (void)hipGetLastError();
         return nullptr;
@@ -501,6 +516,21 @@ hipGraphExec_t Batch::block_graph(int rounds) {
 // the same launch when 128 or more of them are active (nbig), otherwise on the four-step passes of
 // n = 13 after it (fused_block's rule for one n).
 int Batch::run_block(int rounds, uint32_t nact, bool has_mul, uint32_t nbig) {
+    const int rc = use_mode(mode64());
+    if (rc != GFE_OK) return rc;
+    if (mode64()) {
+        if (use_graphs) {
+            if (hipGraphExec_t g = block_graph(rounds, has_mul)) {
+                carries_pending = true;
+                return check_hip(hipGraphLaunch(g, stream), "graph launch");
+            }
+            return set_error(GFE_EHIP, "squaring block graph capture failed");
+        }
+        for (int r = 0; r < rounds; ++r)
+            square(act_dev + (size_t)r * cap, dup_dev + (size_t)r * cap, mul_dev + (size_t)r * cap, has_mul);
+        carries_pending = true;
+        return check("square block");
+    }
     const bool mixed_fused = mixed && (nbig == 0 || nbig >= 128u);
     if (mixed || fused_block(nact, has_mul)) {  // one launch runs the whole block, one workgroup per slot
         flush_carries();
@@ -537,6 +567,8 @@ Batch::~Batch() {
     (void)hipFree(regs); (void)hipFree(ws); (void)hipFree(zp); (void)hipFree(tw); (void)hipFree(carry);
     (void)hipFree(crt); (void)hipFree(slots_dev); (void)hipFree(act_dev); (void)hipFree(dup_dev);
     (void)hipFree(mul_dev);
+    (void)hipFree(tw64); (void)hipFree(crt64);
+    if (crt64_host) (void)hipHostFree(crt64_host);
     for (int i = 0; i < NSTAGE; ++i) {
         if (stage[i]) (void)hipHostFree(stage[i]);
         if (stage_ev[i]) (void)hipEventDestroy(stage_ev[i]);
@@ -587,7 +619,9 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
         hipMalloc(&carry, (size_t)cap * (NA >> 3) * 8) != hipSuccess || hipMalloc(&crt, (size_t)cap * sizeof(CrtConst)) != hipSuccess ||
         hipMalloc(&slots_dev, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
         hipMalloc(&act_dev, (size_t)64 * cap) != hipSuccess || hipMalloc(&dup_dev, (size_t)64 * cap) != hipSuccess ||
-        hipMalloc(&mul_dev, (size_t)64 * cap) != hipSuccess)
+        hipMalloc(&mul_dev, (size_t)64 * cap) != hipSuccess ||
+        hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess ||
+        hipMalloc(&crt64, (size_t)cap * sizeof(F64Crt)) != hipSuccess)
         return set_error(GFE_ENOMEM, "device allocation failed");
     for (int i = 0; i < NSTAGE; ++i) {
         if (hipHostMalloc((void **)&stage[i], (size_t)3 * 64 * cap) != hipSuccess) return set_error(GFE_ENOMEM, "pinned");
@@ -600,7 +634,8 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     }
     for (int i = 0; i < NBLK; ++i)
         if (hipEventCreateWithFlags(&blk_ev[i], hipEventDisableTiming) != hipSuccess) return set_error(GFE_EHIP, "event");
-    if (hipHostMalloc((void **)&slot_host, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
+    if (hipHostMalloc((void **)&crt64_host, (size_t)cap * sizeof(F64Crt)) != hipSuccess ||
+        hipHostMalloc((void **)&slot_host, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
         hipHostMalloc((void **)&crt_host, (size_t)cap * sizeof(CrtConst)) != hipSuccess)
         return set_error(GFE_ENOMEM, "pinned");
     if (hipHostMalloc((void **)&readback, NA * 4) != hipSuccess) return set_error(GFE_ENOMEM, "pinned");
@@ -623,6 +658,7 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
         return set_error(GFE_EHIP, "slot upload");
     if (hipMemsetAsync(regs, 0, (size_t)cap * nregs * NA * 4, stream) != hipSuccess ||
         hipMemsetAsync(mul_dev, 0, (size_t)64 * cap, stream) != hipSuccess ||
+        hipMemsetAsync(crt64, 0, (size_t)cap * sizeof(F64Crt), stream) != hipSuccess ||
         hipMemsetAsync(carry, 0, (size_t)cap * (NA >> 3) * 8, stream) != hipSuccess ||
         hipMemsetAsync(act_dev, 0, (size_t)64 * cap, stream) != hipSuccess ||
         hipMemsetAsync(dup_dev, 0, (size_t)64 * cap, stream) != hipSuccess)
@@ -631,6 +667,10 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     set_lds_attr((const void *)kb_col_inv<3>); set_lds_attr((const void *)kb_col_inv<4>); set_lds_attr((const void *)kb_col_inv<5>);
     set_row_attrs<0>();
     set_row_attrs<1>();
+    f64_set_lds_attributes();
+    f64 = carry64 = n <= F64_ALL_BASES_N;
+    shape = f64_shape(n);
+    if (f64 && f64_build_twiddles(n, tw64, stream) != 0) return set_error(GFE_EHIP, "twiddles");
     spec_batch_set_lds_attributes();
     fused_set_lds_attributes();
     set_lds_attr((const void *)kb_col_fwd_p<3>); set_lds_attr((const void *)kb_col_fwd_p<4>); set_lds_attr((const void *)kb_col_fwd_p<5>);
@@ -647,6 +687,35 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     return check_hip(hipStreamSynchronize(stream), "init");
 }
 
+
+F64Args Batch::args64(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf) const {
+    F64Args A;
+    memset(&A, 0, sizeof(A));
+    A.regs = regs; A.ws = reinterpret_cast<double *>(ws); A.zp = reinterpret_cast<const double *>(zp);
+    A.tw = tw64; A.tws = (uint32_t)f64_tw_words(nalloc); A.slots = reinterpret_cast<int4 *>(carry); A.crt = crt64;
+    A.active = active; A.dupf = dup; A.mulf = mulf;
+    A.reg_stride = (long long)(nregs * NA); A.ws_stride = (long long)(3 * NA / 2); A.slot_stride = (long long)(NA / 16);
+    A.nslots = zdim(); A.tn = (int)nalloc - 1; A.a = shape.a; A.ng = shape.row_ng; A.mixed = mixed;
+    return A;
+}
+
+// Whether squarings and products run in doubles: selected, or a power run's multiplicand is in them.
+bool Batch::mode64() const {
+    if (f64) return true;
+    for (uint32_t s = 0; s < cap; ++s)
+        if (slots[s].busy && slots[s].zp64 && !slots[s].q.empty() && slots[s].q.front().kind == IT_RUN &&
+            slots[s].q.front().run == RUN_POW)
+            return true;
+    return false;
+}
+
+// `carry` in the form of the transform about to run: pending carries of the other are applied first.
+int Batch::use_mode(bool m) {
+    if (m == carry64) return GFE_OK;
+    flush_carries();
+    carry64 = m;
+    return zero_carries();
+}
 
 BArgs Batch::args(const uint8_t *active, const uint8_t *dup) const {
     BArgs A;
@@ -785,6 +854,10 @@ void Batch::launch_norm_carry(const BArgs &A0) {
 void Batch::flush_carries() {
     if (!carries_pending) return;
     carries_pending = false;
+    if (carry64) {
+        f64_launch_flush(args64(nullptr, nullptr, nullptr), stream);
+        return;
+    }
     const BArgs A = args(nullptr, nullptr);
     const unsigned nwg = (unsigned)(N >> 11);
     hipLaunchKernelGGL(kb_carry_wg, dim3((nwg + 255) / 256, 1, zdim()), dim3(256), 0, stream, A);
@@ -796,7 +869,15 @@ int Batch::zero_carries() {
     return check_hip(hipMemsetAsync(carry, 0, (size_t)cap * (NA >> 3) * 8, stream), "carry clear");
 }
 
-void Batch::square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf) {
+void Batch::square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf, bool has_mul) {
+    if (mode64()) {
+        F64Args A = args64(active, dup, mulf);
+        A.absorb = 1;
+        if (!shape.whole) f64_launch_fwd(A, shape, stream);
+        f64_launch_mid(A, shape, has_mul ? F64_EITHER : F64_SQUARE, stream);
+        f64_launch_inv(A, shape, stream);
+        return;
+    }
     BArgs A = args(active, dup);
     A.mulf = mulf;
     A.src_reg = 0;
@@ -820,6 +901,14 @@ void Batch::op_set(const uint8_t *active, uint32_t dst, int32_t value) {
 }
 
 void Batch::op_initmul(const uint8_t *active, uint32_t src) {
+    if (mode64()) {
+        F64Args A = args64(active, nullptr, nullptr);
+        A.src_reg = src;
+        A.ws = reinterpret_cast<double *>(zp);
+        if (!shape.whole) f64_launch_fwd(A, shape, stream);
+        f64_launch_mid(A, shape, F64_FWD, stream);
+        return;
+    }
     BArgs A = args(active, nullptr);
     A.src_reg = src;
     launch_col_fwd(A, 1);
@@ -827,6 +916,14 @@ void Batch::op_initmul(const uint8_t *active, uint32_t src) {
 }
 
 void Batch::op_mul(const uint8_t *active) {
+    if (mode64()) {
+        const F64Args A = args64(active, nullptr, nullptr);
+        if (!shape.whole) f64_launch_fwd(A, shape, stream);
+        f64_launch_mid(A, shape, F64_MUL, stream);
+        f64_launch_inv(A, shape, stream);
+        f64_launch_flush(A, stream);
+        return;
+    }
     BArgs A = args(active, nullptr);
     A.src_reg = 0;
     launch_col_fwd(A, 0);
@@ -980,6 +1077,8 @@ int Batch::submit(uint32_t b, uint64_t iters, uint64_t tag, int32_t *slot_out, u
     zl = std::max(zl, (uint32_t)s + 1);
     int rc = check_hip(hipMemcpyAsync(slots_dev + s, &si, sizeof(si), hipMemcpyHostToDevice, stream), "slot");
     if (rc == GFE_OK) rc = check_hip(hipMemcpyAsync(crt + s, crt_host + s, sizeof(CrtConst), hipMemcpyHostToDevice, stream), "crt");
+    crt64_host[s] = make_f64_crt(S.n, b, f64_primes(b, S.n));
+    if (rc == GFE_OK) rc = check_hip(hipMemcpyAsync(crt64 + s, crt64_host + s, sizeof(F64Crt), hipMemcpyHostToDevice, stream), "crt");
     if (rc != GFE_OK) return rc;
     std::vector<uint8_t> one(cap, 0);
     one[s] = 1;
@@ -1176,6 +1275,9 @@ int Batch::step(int32_t *active_out) {
         }
         if (groups.empty()) break;
         flush_carries();
+        const bool m64 = mode64();
+        rc0 = use_mode(m64);
+        if (rc0 != GFE_OK) return rc0;
         for (auto &kv : groups) {
             const int kind = std::get<0>(kv.first);
             const uint32_t a = std::get<1>(kv.first), b2 = std::get<2>(kv.first);
@@ -1206,7 +1308,10 @@ int Batch::step(int32_t *active_out) {
             });
             rc = check("op");
             if (rc != GFE_OK) return rc;
-            for (int s : kv.second) slots[s].q.pop_front();
+            for (int s : kv.second) {
+                if (kind == IT_INITMUL) slots[s].zp64 = m64;
+                slots[s].q.pop_front();
+            }
         }
     }
     // 2. one block of up to 64 squaring rounds
@@ -1305,7 +1410,7 @@ size_t gfe_batch_slot_bytes(uint32_t n) { return gfe_batch_proof_slot_bytes(n, 0
 size_t gfe_batch_proof_slot_bytes(uint32_t n, uint32_t depth) {
     const size_t N = (size_t)1 << n;
     const size_t regs = depth > 0 ? 3 + ((size_t)1 << depth) : 3;
-    return (regs + 6) * N * 4 + (N >> 3) * 8 + sizeof(gfe::CrtConst) + sizeof(gfe::SlotInfo);
+    return (regs + 6) * N * 4 + (N >> 3) * 8 + sizeof(gfe::CrtConst) + sizeof(gfe::F64Crt) + sizeof(gfe::SlotInfo);
 }
 
 
@@ -1347,6 +1452,7 @@ int gfe_batch_info(const gfe_batch *b, char *buf, size_t len) {
     if (!b || !buf || len == 0) return set_error(GFE_EINVAL, "info");
     std::ostringstream ss;
     ss << "batch n=" << b->bt.n << " capacity=" << b->bt.cap << "; " << gfe::plan_str(b->bt.plan, b->bt.n);
+    if (b->bt.f64) ss << "; " << gfe::f64_str(b->bt.n, 0, b->bt.shape);
     snprintf(buf, len, "%s", ss.str().c_str());
     return GFE_OK;
 }
@@ -1408,6 +1514,7 @@ int gfe_batch_set_plan(gfe_batch *b, const int32_t plan[6]) {
     if (b->bt.zero_carries() != GFE_OK || hipStreamSynchronize(b->bt.stream) != hipSuccess)
         return set_error(GFE_EHIP, "set_plan sync");
     b->bt.plan = P;
+    b->bt.f64 = false;
     b->bt.drop_graphs();
     return GFE_OK;
 }
@@ -1431,13 +1538,14 @@ size_t gfe_batch_device_bytes(uint32_t n, uint32_t capacity) { return gfe_batch_
 
 size_t gfe_batch_proof_device_bytes(uint32_t n, uint32_t capacity, uint32_t depth) {
     const size_t N = (size_t)1 << n;
-    return (size_t)capacity * (gfe_batch_proof_slot_bytes(n, depth) + 3 * 64) + 6 * N * 4;
+    return (size_t)capacity * (gfe_batch_proof_slot_bytes(n, depth) + 3 * 64) + 6 * N * 4 + gfe::F64_PRIMES * gfe::f64_tw_words(n) * 8;
 }
 
 int gfe_batch_get_digits(gfe_batch *b, int32_t slot, uint32_t reg, int32_t *out) {
     if (!b || !out || slot < 0 || (uint32_t)slot >= b->bt.cap || reg >= b->bt.nregs) return set_error(GFE_EINVAL, "get_digits");
     if (hipSetDevice(b->bt.device) != hipSuccess) return set_error(GFE_EHIP, "hipSetDevice");
     gfe::gint g(b->bt.slot_N(slot), b->bt.slots[slot].busy ? b->bt.slots[slot].b : 2);
+    b->bt.flush_carries();
     const int rc = b->bt.read_residue(slot, reg, g);
     if (rc != GFE_OK) return rc;
     memcpy(out, g.data(), b->bt.slot_N(slot) * 4);
@@ -1466,8 +1574,11 @@ int gfe_batch_time_rounds(gfe_batch *b, uint32_t rounds, double *ms) {
     B.stage_release();
     if (rc != GFE_OK) return rc;
     // captured blocks are built before the timed region
-    const bool four_step = B.mixed ? (nbig > 0 && nbig < 128) : !B.fused_block(nact);
-    if (B.use_graphs && !B.plan.pipe && four_step) {
+    const bool m64 = B.mode64();
+    rc = B.use_mode(m64);
+    if (rc != GFE_OK) return rc;
+    const bool four_step = m64 ? true : B.mixed ? (nbig > 0 && nbig < 128) : !B.fused_block(nact);
+    if (B.use_graphs && (m64 || !B.plan.pipe) && four_step) {
         if (rounds >= 64 && !B.block_graph(64)) return set_error(GFE_EHIP, "squaring block graph capture failed");
         if ((rounds % 64) && !B.block_graph((int)(rounds % 64))) return set_error(GFE_EHIP, "squaring block graph capture failed");
     }
@@ -1504,6 +1615,8 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
     if (hipMalloc(&save, (size_t)B.cap * row) != hipSuccess) return set_error(GFE_ENOMEM, "tune save");
     (void)hipMemcpy2DAsync(save, row, B.regs, pitch, row, B.cap, hipMemcpyDeviceToDevice, B.stream);
     const gfe::Plan orig = B.plan;
+    const bool f64_was = B.f64;
+    B.f64 = false;
     gfe::Plan best = orig;
     double best_ms = 1e30;
     const bool graphs = B.use_graphs;
@@ -1556,6 +1669,19 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
     B.use_graphs = graphs;
     B.drop_graphs();
     (void)B.zero_carries();
+    if (f64_was) {  // the double-precision transform against the chosen plan, as blocks run
+        double t[2] = {1e30, 1e30};
+        for (int pass = 0; pass < 4; ++pass) {
+            B.f64 = (pass & 1) != 0;
+            double ms = 0;
+            if (gfe_batch_time_rounds(b, 64, &ms) != GFE_OK || gfe_batch_time_rounds(b, 128, &ms) != GFE_OK) continue;
+            t[pass & 1] = std::min(t[pass & 1], ms);
+        }
+        B.f64 = t[1] < t[0];
+        B.drop_graphs();
+        (void)B.zero_carries();
+        B.carry64 = B.f64;
+    }
     (void)hipMemcpy2DAsync(B.regs, pitch, save, row, row, B.cap, hipMemcpyDeviceToDevice, B.stream);
     (void)hipStreamSynchronize(B.stream);
     (void)hipFree(save);

@@ -1073,7 +1073,7 @@ int Engine::f64_select() {
     f64 = zp_f64 = f64_k != 0;
     if (!f64) return GFE_OK;
     const F64Crt c = make_f64_crt(n, b, f64_k);
-    shape = f64_shape(n, 1);
+    shape = f64_shape(n);
     return hipMemcpy(crt64, &c, sizeof(c), hipMemcpyHostToDevice) == hipSuccess ? GFE_OK : set_error(GFE_EHIP, "crt upload");
 }
 
@@ -1091,7 +1091,7 @@ F64Args Engine::f64_args(int dup) const {
 void Engine::f64_run(uint32_t src, uint32_t *out, int mode) {
     if (carry_pending && (src != 0 || pend_kind != 3)) flush_carry();
     F64Args A = f64_args(0);
-    A.reg_off = src * (uint32_t)N;
+    A.src_reg = src;
     A.ws = reinterpret_cast<double *>(out);
     A.absorb = carry_pending;
     if (!shape.whole) f64_launch_fwd(A, shape, stream);

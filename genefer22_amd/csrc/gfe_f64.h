@@ -47,7 +47,7 @@ constexpr uint64_t F64_P[F64_PRIMES] = {562949869535233ull, 562949517213697ull, 
 constexpr uint32_t F64_G[F64_PRIMES] = {5, 10, 3};
 constexpr int F64_NG = 16;       // columns per workgroup: one 16-lane DPP row of limbs
 constexpr int F64_ROW_MIN = 6, F64_ROW_MAX = 14, F64_COL_MIN = 5, F64_COL_MAX = 8;
-constexpr int F64_WHOLE_MIN = 11, F64_WHOLE_MAX = 14;           // log2 limbs of a one-workgroup transform
+constexpr int F64_WHOLE_MIN = 11, F64_WHOLE_MAX = 12;           // log2 limbs of a one-workgroup transform
 constexpr uint32_t F64_NORM_T = 64, F64_NORM_PER = 1, F64_NORM_RANGE = F64_NORM_T * F64_NORM_PER;  // its normalisation
 constexpr int F64_COL_E = 3;     // log2 of the residues per thread in the column passes
 

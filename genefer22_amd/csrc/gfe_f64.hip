@@ -1,8 +1,8 @@
 // gfe_f64.hip -- kernels and host constants of the double-precision limb transform (gfe_f64.h).
 //
 // One squaring is three launches: forward column pass (digits -> residues of every prime), row pass
-// (forward, square, inverse), inverse column pass with the CRT and the carry; or, where a prime's
-// transform fits one workgroup's LDS (2^14 limbs), two: the whole transform of each prime, then the CRT
+// (forward, square, inverse), inverse column pass with the CRT and the carry; or, up to 2^12
+// limbs, two: the whole transform of each prime, then the CRT
 // and the carry.
 #include "gfe_f64_host.h"
 
@@ -37,7 +37,6 @@ __device__ __forceinline__ F64Job f64_job(const F64Args &A, uint32_t per) {
     }
     J.run = J.slot < A.nslots && !(A.active && !A.active[J.slot]);
     J.c = (F64CrtP)(A.crt + (J.run ? J.slot : 0));
-    J.run = J.run && J.c->n == A.tn + 1;  // a mixed batch's slots of another n
     J.K = J.c->K;
     return J;
 }
@@ -58,7 +57,7 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_fwd(F64Args 
     if (k0 >= K) return;
     const unsigned blk = f64_block(A, split ? J.w - k0 * nb : J.w, nb);
     int2 d[1 << LOGE];
-    f64_load_digits<LOGE, LOGG>(d, A.regs + J.slot * A.reg_stride + A.reg_off,
+    f64_load_digits<LOGE, LOGG>(d, A.regs + J.slot * A.reg_stride + (size_t)A.src_reg * (2u << A.tn),
                                 A.absorb ? A.slots + J.slot * A.slot_stride : nullptr, C, blk, t);
     const double bd = c->bd;
     const bool reduce = c->big == 2;
@@ -93,22 +92,17 @@ __global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
         for (int rr = 0; rr < 16; ++rr) x[rr] = md.red(x[rr]);
     };
     f64_row_pass<LOGG, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s, lds64 + q * f64_row_words(LOGG),
-                             MODE == F64_EITHER && A.mulf[J.slot]);
+                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
-// 3 workgroups a slot, 2^LOGG / 16 threads: a prime's whole transform, from the digits.
+// A prime's whole transform, from the digits, in one workgroup; thread s of 2^LOGG / 16.
 template <int LOGG, int MODE>
-__global__ void __launch_bounds__(1 << (LOGG - 4)) k64_whole(F64Args A) {
-    extern __shared__ double lds64[];
-    const F64Job J = f64_job(A, 3);
-    const int k = (int)J.w;
-    if (!J.run || k >= J.K) return;
+__device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J, int k, uint32_t s, double *lds) {
     const F64CrtP c = J.c;
-    const uint32_t s = threadIdx.x;
     const F64Mod md{c->p[k], c->pinv[k]};
     const double bd = c->bd;
     const bool reduce = c->big != 0;
-    const int2 *src = reinterpret_cast<const int2 *>(A.regs + J.slot * A.reg_stride + A.reg_off);
+    const int2 *src = reinterpret_cast<const int2 *>(A.regs + J.slot * A.reg_stride + (size_t)A.src_reg * (2u << LOGG));
     const int4 *ls = A.absorb ? A.slots + J.slot * A.slot_stride : nullptr;
     const size_t at = J.slot * A.ws_stride + ((size_t)k << LOGG);
     const auto load = [&](double (&x)[16], uint32_t base, auto yl) {
@@ -130,8 +124,27 @@ __global__ void __launch_bounds__(1 << (LOGG - 4)) k64_whole(F64Args A) {
 #pragma unroll
         for (int rr = 0; rr < 16; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
     };
-    f64_row_pass<LOGG, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds64,
-                             MODE == F64_EITHER && A.mulf[J.slot]);
+    f64_row_pass<LOGG, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
+                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
+}
+
+// 3 workgroups a slot.
+template <int LOGG, int MODE>
+__global__ void __launch_bounds__(1 << (LOGG - 4)) k64_whole(F64Args A) {
+    extern __shared__ double lds64[];
+    const F64Job J = f64_job(A, 3);
+    if (J.run && (int)J.w < J.K) f64_whole_body<LOGG, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+}
+
+// A mixed batch: each workgroup at its slot's n, 12 or 13 (of the 256 threads n = 12 takes two whole
+// waves; the others end before any barrier).
+template <int MODE>
+__global__ void __launch_bounds__(256) k64_whole_mixed(F64Args A) {
+    extern __shared__ double lds64[];
+    const F64Job J = f64_job(A, 3);
+    if (!J.run || (int)J.w >= J.K) return;
+    if (J.c->n == 13) f64_whole_body<12, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    else if (threadIdx.x < 128) f64_whole_body<11, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
 }
 
 template <int K, int LOGG>
@@ -146,7 +159,7 @@ __device__ __forceinline__ void f64_inv_body(const F64Args &A, const F64Job &J, 
 #pragma unroll
     for (int k = 0; k < K; ++k)
         f64_col_inv<LOGE, LOGG>(F64Mod{J.c->p[k], J.c->pinv[k]}, x[k], A.tw + (size_t)k * A.tws, t, lds);
-    f64_norm_store<K, LOGE, LOGG>(J.c, x, C, blk, t, dup, A.regs + J.slot * A.reg_stride + A.reg_off,
+    f64_norm_store<K, LOGE, LOGG>(J.c, x, C, blk, t, dup, A.regs + J.slot * A.reg_stride,
                                   A.slots + J.slot * A.slot_stride);
 }
 
@@ -162,8 +175,8 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_inv(F64Args 
 }
 
 template <int K>
-__device__ __forceinline__ void f64_norm_body(const F64Args &A, const F64Job &J, int dup) {
-    const uint32_t M = 1u << A.tn, i0 = J.w * F64_NORM_RANGE + threadIdx.x;
+__device__ __forceinline__ void f64_norm_body(const F64Args &A, const F64Job &J, uint32_t M, int dup) {
+    const uint32_t i0 = J.w * F64_NORM_RANGE + threadIdx.x;
     const double *ws = A.ws + J.slot * A.ws_stride;
     double r[F64_NORM_PER][K];
 #pragma unroll
@@ -172,17 +185,19 @@ __device__ __forceinline__ void f64_norm_body(const F64Args &A, const F64Job &J,
         for (int k = 0; k < K; ++k) r[j][k] = ws[(size_t)k * M + i0 + j * F64_NORM_T];
 #pragma unroll
     for (int j = 0; j < F64_NORM_PER; ++j)
-        f64_norm_limb<K>(J.c, r[j], dup, i0 + j * F64_NORM_T, M, A.regs + J.slot * A.reg_stride + A.reg_off,
-                         A.slots + J.slot * A.slot_stride);
+        f64_norm_limb<K>(J.c, r[j], dup, i0 + j * F64_NORM_T, M, A.regs + J.slot * A.reg_stride, A.slots + J.slot * A.slot_stride);
 }
 
-// The normalisation after k64_whole: M / F64_NORM_RANGE workgroups a slot.
+// The normalisation after k64_whole: M / F64_NORM_RANGE workgroups a slot (a mixed batch's slots of the
+// smaller n leave the rest idle).
 __global__ void __launch_bounds__(F64_NORM_T) k64_norm(F64Args A) {
     const F64Job J = f64_job(A, (1u << A.tn) / F64_NORM_RANGE);
     if (!J.run) return;
+    const uint32_t M = A.K ? 1u << A.tn : 1u << (J.c->n - 1);
+    if (J.w * F64_NORM_RANGE >= M) return;
     const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
-    if (J.K == 2) f64_norm_body<2>(A, J, dup);
-    else f64_norm_body<3>(A, J, dup);
+    if (J.K == 2) f64_norm_body<2>(A, J, M, dup);
+    else f64_norm_body<3>(A, J, M, dup);
 }
 
 // Register 0 of the slots in grid.y with its pending range carries, balanced (f64_flush_body).
@@ -329,7 +344,8 @@ int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
 
 // One candidate, timed on MI355X (us per squaring, three primes unless said).  Up to 2^12 limbs the
 // two launches with a prime's transform in one workgroup beat the three (2^11 limbs 9.3 against
-// 13.1, 2^12 11.0 against 13.4; at 2^13 one workgroup's arithmetic takes longer, 16.8 against 14.0).
+// 13.1, 2^12 11.0 against 13.4; at 2^13 one workgroup's arithmetic takes longer, 16.8 against 14.0;
+// in batches 100 candidates of 2^13 limbs 32.8 against 31.6, 512 of 2^14 230 against 228).
 // With three passes, up to 2^19 limbs each is bound by latency, so the shapes that win are those with
 // the most workgroups: short columns, one wave per row workgroup, a workgroup per prime in the
 // forward column pass (2^15 limbs: 15.0 with 2^5-point columns, 15.5 with 2^6, 16.3 with all primes
@@ -338,10 +354,10 @@ int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
 // (2^21 limbs: 81.8 with 2^8-point columns, 89.6 with 2^7).  The integer passes at the same sizes:
 // 14.5, 15.6, 15.9, 16.5, 18.8, 20.0, 25.8, 36.9, 41.8, 57.8, 89.3 at n = 12, 13, .., 22 (the last
 // eight limbs of two digits where those are exact).
-F64Shape f64_shape(uint32_t n, uint32_t slots) {
+F64Shape f64_shape(uint32_t n) {
     F64Shape S;
     const int tn = (int)n - 1;
-    S.whole = n <= 13;
+    S.whole = tn <= F64_WHOLE_MAX;
     S.a = tn <= 15 ? 5 : tn <= 18 ? 6 : tn == 19 ? 7 : 8;
     S.split = tn <= 19;
     const int spr = 1 << (tn - S.a - 4);
@@ -387,33 +403,53 @@ static F64Fn mid_fn(bool whole, int mode, int logg) {
     }
 }
 
+// Slots are pinned to XCDs (slot s on XCD s mod 8) where that leaves at most an eighth of the XCDs'
+// time idle: what one pass leaves in the XCD's L2 the next one finds there.  us per round of a
+// batch, pinned and not: 301 slots of n = 12 19.9 and 29.5, 32 slots 9.7 and 10.9, 7 slots of n = 18
+// 40.8 and 44.4, 512 of n = 15 (4 MiB of L2 hold 1 % of an XCD's share) 228 and 229; 3 slots of n = 20
+// would use 3 of the 8 XCDs: 118 and 63.
+static bool f64_pin(uint32_t slots) { return slots >= 7 && 7 * ((slots + 7) / 8) <= slots; }
+
 // Workgroups of a launch of `per` a slot (f64_job).
-static dim3 f64_grid(const F64Args &A, uint32_t per) {
+static dim3 f64_grid(F64Args &A, uint32_t per) {
+    A.pin = !A.K && f64_pin(A.nslots);
     return dim3(A.pin ? 8 * per * ((A.nslots + 7) / 8) : per * A.nslots);
 }
 
-void f64_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream) {
+void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream) {
     const unsigned nb = 1u << (A.tn - S.a - 4), T = 16u << (S.a - F64_COL_E);
-    hipLaunchKernelGGL(fwd_fn(S.a), f64_grid(A, S.split ? 3 * nb : nb), dim3(T), (size_t)128 << S.a, stream, A, S.split);
+    const dim3 grid = f64_grid(A, S.split ? 3 * nb : nb);
+    hipLaunchKernelGGL(fwd_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A, S.split);
 }
 
-void f64_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream) {
+void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) {
+    if (A.mixed) {
+        const F64Fn f = mode == F64_SQUARE ? k64_whole_mixed<F64_SQUARE> : mode == F64_MUL ? k64_whole_mixed<F64_MUL>
+                                                                                         : k64_whole_mixed<F64_FWD>;
+        const dim3 grid = f64_grid(A, 3);
+        hipLaunchKernelGGL(f, grid, dim3(256), (size_t)8 * f64_row_words(12), stream, A);
+        return;
+    }
     if (S.whole) {
-        hipLaunchKernelGGL(mid_fn(true, mode, A.tn), f64_grid(A, 3), dim3(1u << (A.tn - 4)), (size_t)8 * f64_row_words(A.tn), stream, A);
+        const dim3 grid = f64_grid(A, 3);
+        hipLaunchKernelGGL(mid_fn(true, mode, A.tn), grid, dim3(1u << (A.tn - 4)), (size_t)8 * f64_row_words(A.tn), stream, A);
         return;
     }
     const int L = A.tn - S.a;
-    hipLaunchKernelGGL(mid_fn(false, mode, L), f64_grid(A, 3 * ((1u << S.a) / S.row_ng)), dim3((unsigned)S.row_ng << (L - 4)),
+    const dim3 grid = f64_grid(A, 3 * ((1u << S.a) / S.row_ng));
+    hipLaunchKernelGGL(mid_fn(false, mode, L), grid, dim3((unsigned)S.row_ng << (L - 4)),
                        (size_t)8 * S.row_ng * f64_row_words(L), stream, A);
 }
 
-void f64_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream) {
+void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
     if (S.whole) {
-        hipLaunchKernelGGL(k64_norm, f64_grid(A, (1u << A.tn) / F64_NORM_RANGE), dim3(F64_NORM_T), 0, stream, A);
+        const dim3 grid = f64_grid(A, (1u << A.tn) / F64_NORM_RANGE);
+        hipLaunchKernelGGL(k64_norm, grid, dim3(F64_NORM_T), 0, stream, A);
         return;
     }
     const unsigned T = 16u << (S.a - F64_COL_E);
-    hipLaunchKernelGGL(inv_fn(S.a), f64_grid(A, 1u << (A.tn - S.a - 4)), dim3(T), (size_t)128 << S.a, stream, A);
+    const dim3 grid = f64_grid(A, 1u << (A.tn - S.a - 4));
+    hipLaunchKernelGGL(inv_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A);
 }
 
 void f64_launch_flush(const F64Args &A, hipStream_t stream) {

@@ -12,25 +12,24 @@
 namespace gfe {
 
 // Shape of the passes at one n.  whole: a prime's transform in one workgroup and the normalisation
-// after it (n <= 15); else three passes over 2^a rows of 2^(n-1-a) limbs, row_ng rows per
-// workgroup, the forward column pass with one prime per workgroup (split) instead of all.
-// pin: a slot's workgroups all on one XCD.
+// after it; else three passes over 2^a rows of 2^(n-1-a) limbs, row_ng rows per workgroup, the
+// forward column pass with one prime per workgroup (split) instead of all.
 struct F64Shape {
-    int whole = 0, a = 0, row_ng = 1, split = 0, pin = 0;
+    int whole = 0, a = 0, row_ng = 1, split = 0;
 };
 
 // Primes the transform needs for (b, n): 2 or 3, or 0 where it is not exact (or out of range).
 int f64_primes(uint32_t b, uint32_t n);
 // Largest n at which it is exact for every base.
 constexpr uint32_t F64_ALL_BASES_N = 20;
-F64Shape f64_shape(uint32_t n, uint32_t slots);
+F64Shape f64_shape(uint32_t n);
 std::string f64_str(uint32_t n, int K, const F64Shape &S);  // K = 0: by the slot
 F64Crt make_f64_crt(uint32_t n, uint32_t b, int K);
 // Table words of one prime: entries psi^bitrev(j), j < M / 4 (those of a smaller n are its first ones).
 inline size_t f64_tw_words(uint32_t n) { return ((size_t)1 << n) / 8; }
 int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream);
 
-// Slot s of a launch: registers at regs + s reg_stride (the pass's at + reg_off), residues at
+// Slot s of a launch: registers at regs + s reg_stride (2^n digits each), residues at
 // ws / zp + s ws_stride, range carries at slots + s slot_stride, constants crt[s].  One candidate is slot
 // 0 with K set: its kernels then wait for no per-slot table before their first loads (0.3-0.5 us a
 // launch).
@@ -43,16 +42,18 @@ struct F64Args {
     const F64Crt *crt;
     const uint8_t *active, *dupf, *mulf;  // per slot, or null (all, dup, none)
     long long reg_stride, ws_stride, slot_stride;
-    uint32_t reg_off, tws, nslots;
-    int tn, a, ng, dup, absorb, pin;
+    uint32_t src_reg, tws, nslots;
+    int tn, a, ng, dup, absorb;
+    int pin;                // slot s on XCD s mod 8 (set by the launches)
+    int mixed;              // slots of n = 12 beside those of n = 13 (tn = 12, whole)
     int K;                  // one candidate's primes, or 0: slots, each with its own
 };
 
-// Register at regs + reg_off -> residues in ws (col_fwd then row, or whole_fwd), the square or product
-// (row or whole in the same mode), ws -> register at regs + reg_off (inv).
-void f64_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream);           // three passes only
-void f64_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream); // row, or whole
-void f64_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream);           // with the carry
+// Register src_reg -> (fwd and) mid -> ws, and ws -> register 0 with the carry (inv).
+void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream);           // three passes only
+void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream); // row, or whole
+void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream);
+// Adds the pending range carries of register 0 and balances it.
 void f64_launch_flush(const F64Args &A, hipStream_t stream);
 void f64_set_lds_attributes();
 

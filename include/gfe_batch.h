@@ -70,13 +70,15 @@ size_t gfe_batch_slot_bytes(uint32_t n);
 size_t gfe_batch_proof_slot_bytes(uint32_t n, uint32_t depth);
 /* Chooses the pass plan by timing the admissible ones on `reps` rounds of the batch's busy slots,
  * the fastest eight again on 8 x reps and, when the batch runs its blocks as graphs, the fastest
- * three on captured 64-round blocks (their registers are saved and restored, so their programs
- * continue unchanged); returns
+ * three on captured 64-round blocks, and last the fastest against the double-precision transform
+ * (their registers are saved and restored, so their programs continue unchanged); returns
  * GFE_EINVAL when no slot is busy: submit the candidates first.  The reference's tune,
  * src/transformGPU.h:851-900. */
 int gfe_batch_tune(gfe_batch *bt, uint32_t reps);
 int gfe_batch_info(const gfe_batch *bt, char *buf, size_t len);
-/* The batch's pass plan, as gfe_get_plan / gfe_set_plan of gfe.h. */
+/* The batch's pass plan, as gfe_get_plan / gfe_set_plan of gfe.h: up to n = 20 a batch squares in the
+ * double-precision limb transform until gfe_batch_set_plan selects the integer passes (power runs
+ * under way then end in the transform that holds their multiplicand). */
 int gfe_batch_get_plan(const gfe_batch *bt, int32_t plan[6]);
 int gfe_batch_set_plan(gfe_batch *bt, const int32_t plan[6]);
 

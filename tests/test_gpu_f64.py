@@ -90,3 +90,58 @@ def test_refused_bases_keep_the_integer_passes(gfe, oracle):
     t.set_digits(d); o.set_digits(d, 0)
     t.square_dup(True); o.square_dup(True)
     assert np.array_equal(canon(oracle, t.get_digits(), n, b), canon(oracle, o.get_digits(0), n, b))
+
+
+def run_batch(gfe, n, bases, iters, integer=False, graphs=True, mixed=False):
+    bt = gfe.Batch(n, len(bases), mixed=mixed)
+    assert "in doubles" in bt.info()
+    bt.set_graphs(graphs)
+    if integer:
+        bt.set_plan(bt.get_plan()[:5] + (24,) if mixed else bt.get_plan())
+        assert "in doubles" not in bt.info()
+    for i, b in enumerate(bases):
+        assert bt.submit(b, iters + 3 * i, i, n=12 + i % 2 if mixed else None) is not None
+    got = []
+    while len(got) < len(bases):
+        bt.step()
+        got += bt.poll()
+    bt.close()
+    return sorted((r["tag"], r["res64"], r["old64"], r["hash64"]) for r in got)
+
+
+@pytest.mark.parametrize("n,count", [(12, 9), (12, 8), (13, 15), (14, 3), (15, 7), (17, 8), (19, 2), (20, 1)])
+def test_batches_equal_the_integer_passes(gfe, n, count):
+    """Slots spread over the XCDs or pinned to one each, two and three primes side by side, slots that
+    end rounds before others, graphs and single launches."""
+    e = largest_two_prime_base(n)
+    bases = [(1026, 1999999898, e & ~1, (e & ~1) + 2, 146950, 20204692)[i % 6] + 2 * (i // 6) for i in range(count)]
+    want = run_batch(gfe, n, bases, 70, integer=True)
+    assert run_batch(gfe, n, bases, 70) == want
+    assert run_batch(gfe, n, bases, 70, graphs=False) == want
+
+
+def test_mixed_batch_equals_the_integer_passes(gfe):
+    bases = [1026, 1999999998, 146950, 20204692, 50000000, 4098, 999999618]
+    assert run_batch(gfe, 13, bases, 70, mixed=True) == run_batch(gfe, 13, bases, 70, mixed=True, integer=True)
+
+
+@pytest.mark.parametrize("at", [10, 17, 24, 31])
+def test_plan_change_during_a_proofs_powers(gfe, at):
+    """gfe_batch_set_plan while power runs hold their multiplicand in doubles: those runs end in
+    doubles, what follows is in the integer passes, and the proof is the same."""
+    b, n, depth = 1026, 12, 3
+    want = gfe.run_proof(b, n, depth)
+    bt = gfe.Batch(n, 2, depth=depth)
+    for tag in (0, 1):
+        bt.submit(b, 0, tag)
+    got, steps, prp = [], 0, want["esize"] // 64
+    while len(got) < 2:
+        bt.step()
+        steps += 1
+        if steps == prp + at:
+            bt.set_plan(bt.get_plan())
+        got += bt.poll()
+    assert steps > prp + at
+    bt.close()
+    for r in got:
+        assert (r["res64"], r["pkey"], r["mu_hash64"], r["gl_ok"]) == (want["res64"], want["pkey"], want["mu_hash64"], 1)
