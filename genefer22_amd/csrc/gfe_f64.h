@@ -238,6 +238,20 @@ enum { F64_SQUARE = 0, F64_MUL = 1, F64_FWD = 2, F64_EITHER = 3 };
 
 __host__ __device__ constexpr uint32_t f64_row_words(int logg) { return (1u << logg) + (1u << (logg - 4)); }
 
+// Between the LDS writes of a chunk and the next chunk's reads, YL the larger of their strides' logs: a
+// sub-transform then spans 2^(YL + 4) consecutive residues, and up to 1024 of them belong to one
+// wave, whose own accesses stay in order; beyond that the workgroup's threads meet.  (A thread writes
+// back the very elements it has read, so nothing is needed between its reads and its writes.)
+template <int YL>
+__device__ __forceinline__ void f64_exchange() {
+    if constexpr (YL <= 6) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        __syncthreads();
+    }
+}
+
 __device__ __forceinline__ constexpr uint32_t f64_off(uint32_t rr, int YL) { return (rr << YL) + ((rr << YL) >> 4); }
 
 // (a0..a3)^2 mod X^4 - w, operands reduced; results below 1.8 p.
@@ -285,14 +299,13 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
         if constexpr (ci == 0) {
             load(x, base, std::integral_constant<int, YL>{});
         } else {
-            __syncthreads();
+            f64_exchange<GM::ylog(ci - 1)>();
             const double *p = L + base + (base >> 4);
 #pragma unroll
             for (int rr = 0; rr < 16; ++rr) x[rr] = p[f64_off(rr, YL)];
         }
         f64_fwd_chunk<4, NE>(md, x, w);
         if constexpr (ci != LAST) {
-            if constexpr (ci > 0) __syncthreads();
             double *p = L + base + (base >> 4);
 #pragma unroll
             for (int rr = 0; rr < 16; ++rr) p[f64_off(rr, YL)] = x[rr];
@@ -330,7 +343,7 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
             const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
             f64_inv_tw<4, UNI>(w, tw, (uint32_t)(a + lam0), (row << lam0) + hi, NE);
             if constexpr (ci != LAST) {
-                __syncthreads();
+                f64_exchange<YL>();
                 const double *p = L + base + (base >> 4);
 #pragma unroll
                 for (int rr = 0; rr < 16; ++rr) x[rr] = p[f64_off(rr, YL)];
@@ -340,7 +353,6 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
 #pragma unroll
                 for (int rr = 0; rr < 16; ++rr) data[base + (rr << YL)] = x[rr];
             } else {
-                __syncthreads();
                 double *p = L + base + (base >> 4);
 #pragma unroll
                 for (int rr = 0; rr < 16; ++rr) p[f64_off(rr, YL)] = x[rr];
@@ -414,7 +426,7 @@ __device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const int2 (&d)[1 
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) o[(size_t)(base + ((uint32_t)rr << YL)) * C] = x[rr];
         } else {
-            __syncthreads();  // the previous chunk's (or prime's) reads
+            if constexpr (ci == 0) __syncthreads();  // the previous prime's last reads
             double *p = lds + base * 16 + q;
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) p[(uint32_t)rr << (YL + 4)] = x[rr];
@@ -456,7 +468,7 @@ __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << L
         }
         f64_inv_chunk<LOGE, NE, (ci != 0)>(md, x, w);
         if constexpr (ci != 0) {
-            __syncthreads();
+            if constexpr (ci == GM::NCH - 1) __syncthreads();  // the previous prime's last reads
             double *p = lds + base * 16 + q;
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) p[(uint32_t)rr << (YL + 4)] = x[rr];
