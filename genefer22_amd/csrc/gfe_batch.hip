@@ -395,6 +395,7 @@ struct Batch {
     F64Shape shape;
     double *tw64 = nullptr;
     F64Crt *crt64 = nullptr, *crt64_host = nullptr;
+    int int_tables();
     bool mode64() const;
     int use_mode(bool m);
     F64Args args64(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf) const;
@@ -615,7 +616,7 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) cus = 256;
     plan = default_batch_plan(n, cap);
     if (hipMalloc(&regs, (size_t)cap * nregs * NA * 4) != hipSuccess || hipMalloc(&ws, (size_t)cap * 3 * NA * 4) != hipSuccess ||
-        hipMalloc(&zp, (size_t)cap * 3 * NA * 4) != hipSuccess || hipMalloc(&tw, (size_t)6 * NA * 4) != hipSuccess ||
+        hipMalloc(&zp, (size_t)cap * 3 * NA * 4) != hipSuccess ||
         hipMalloc(&carry, (size_t)cap * (NA >> 3) * 8) != hipSuccess || hipMalloc(&crt, (size_t)cap * sizeof(CrtConst)) != hipSuccess ||
         hipMalloc(&slots_dev, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
         hipMalloc(&act_dev, (size_t)64 * cap) != hipSuccess || hipMalloc(&dup_dev, (size_t)64 * cap) != hipSuccess ||
@@ -640,13 +641,6 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
         return set_error(GFE_ENOMEM, "pinned");
     if (hipHostMalloc((void **)&readback, NA * 4) != hipSuccess) return set_error(GFE_ENOMEM, "pinned");
     if (hipEventCreate(&ev0) != hipSuccess || hipEventCreate(&ev1) != hipSuccess) return set_error(GFE_EHIP, "event");
-    {
-        std::vector<uint32_t> h(6 * N);
-        const int sets[6] = {0, 0, 0, 1, 1, 1}, primes[6] = {0, 1, 2, 0, 1, 2};
-        make_twiddle_tables(sets, primes, 6, n, h.data());
-        if (hipMemcpy(tw, h.data(), 6 * N * 4, hipMemcpyHostToDevice) != hipSuccess)
-            return set_error(GFE_EHIP, "twiddle upload");
-    }
     for (int k = 0; k < 3; ++k) {
         prS.p[k] = prime_of(0, k); prU.p[k] = prime_of(1, k);
         CrtConst c0 = make_crt(3, 0, n), c1 = make_crt(3, 1, n);
@@ -671,6 +665,10 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     f64 = carry64 = n <= F64_ALL_BASES_N;
     shape = f64_shape(n);
     if (f64 && f64_build_twiddles(n, tw64, stream) != 0) return set_error(GFE_EHIP, "twiddles");
+    if (!f64) {
+        const int rc = int_tables();
+        if (rc != GFE_OK) return rc;
+    }
     spec_batch_set_lds_attributes();
     fused_set_lds_attributes();
     set_lds_attr((const void *)kb_col_fwd_p<3>); set_lds_attr((const void *)kb_col_fwd_p<4>); set_lds_attr((const void *)kb_col_fwd_p<5>);
@@ -687,6 +685,22 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     return check_hip(hipStreamSynchronize(stream), "init");
 }
 
+
+// The integer passes' twiddle tables, made when those passes are first selected.
+int Batch::int_tables() {
+    if (tw) return GFE_OK;
+    std::vector<uint32_t> h(6 * NA);
+    const int sets[6] = {0, 0, 0, 1, 1, 1}, primes[6] = {0, 1, 2, 0, 1, 2};
+    make_twiddle_tables(sets, primes, 6, nalloc, h.data());
+    uint32_t *t = nullptr;
+    if (hipMalloc(&t, (size_t)6 * NA * 4) != hipSuccess) return set_error(GFE_ENOMEM, "device allocation failed");
+    if (hipMemcpy(t, h.data(), 6 * NA * 4, hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(t);
+        return set_error(GFE_EHIP, "twiddle upload");
+    }
+    tw = t;
+    return GFE_OK;
+}
 
 F64Args Batch::args64(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf) const {
     F64Args A;
@@ -1510,6 +1524,8 @@ int gfe_batch_set_plan(gfe_batch *b, const int32_t plan[6]) {
     if (b->bt.mixed && (!P.spec || !P.fuse_sq))
         return set_error(GFE_EINVAL, "a mixed batch keeps compile-time passes and the single-workgroup squaring");
     if (hipSetDevice(b->bt.device) != hipSuccess) return set_error(GFE_EHIP, "hipSetDevice");
+    const int rc = b->bt.int_tables();
+    if (rc != GFE_OK) return rc;
     b->bt.flush_carries();
     if (b->bt.zero_carries() != GFE_OK || hipStreamSynchronize(b->bt.stream) != hipSuccess)
         return set_error(GFE_EHIP, "set_plan sync");
@@ -1607,6 +1623,8 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
     bool any = false;
     for (auto &S : B.slots) any |= S.busy;
     if (!any) return set_error(GFE_EINVAL, "tune needs busy slots");
+    const int rct = B.int_tables();
+    if (rct != GFE_OK) return rct;
     const std::vector<gfe::Plan> plans = gfe::candidate_plans(B.n);
     B.flush_carries();
     // squarings on the busy slots' r0: save and restore register 0 of every slot

@@ -86,12 +86,15 @@ struct Engine {
     uint32_t *tw = nullptr;
     CrtConst *crt = nullptr;
     // two-digit-limb transform (limb_ok): four twiddle tables of N/2 entries, its CRT constants,
-    // its primes and b 2^32 mod p of each
+    // its primes and b 2^32 mod p of each (tw and tw_limb: int_tables)
     uint32_t *tw_limb = nullptr;
     void *limb_crt = nullptr;
     PrimeArgs pr4;
     uint32_t bm4[4] = {0, 0, 0, 0};
-    bool can_limb = false;
+    LimbCrt limb_crt_host;
+    bool can_limb = false, limb_made = false;  // exact for b; for the b the engine was created with
+    void limb_constants();
+    int int_tables();
     int tn() const { return plan.limb ? (int)n - 1 : (int)n; }   // log2 of the transform length
     int tp() const { return plan.limb ? 4 : rns; }               // primes of the transform
     const uint32_t *cur_tw() const { return plan.limb ? tw_limb : tw; }

@@ -749,52 +749,78 @@ int Engine::init(uint32_t b_, uint32_t n_, uint32_t num_regs_, int device_) {
     const size_t wb = work_bytes(N);
     if (hipMalloc(&regs, (size_t)num_regs * N * 4) != hipSuccess || hipMalloc(&ws, wb) != hipSuccess ||
         hipMalloc(&zp, wb) != hipSuccess || hipMalloc(&carry, (N / 8) * 8) != hipSuccess ||
-        hipMalloc(&tw, (size_t)rns * N * 4) != hipSuccess || hipMalloc(&crt, sizeof(CrtConst)) != hipSuccess) {
+        hipMalloc(&crt, sizeof(CrtConst)) != hipSuccess) {
         dev_ok = true;
         return set_error(GFE_ENOMEM, "device allocation failed");
     }
     dev_ok = true;
-    {
-        std::vector<uint32_t> htw((size_t)rns * N);
-        const int sets[3] = {is32, is32, is32}, primes[3] = {0, 1, 2};
-        make_twiddle_tables(sets, primes, rns, n, htw.data());
-        if (hipMemcpy(tw, htw.data(), (size_t)rns * N * 4, hipMemcpyHostToDevice) != hipSuccess)
-            return set_error(GFE_EHIP, "twiddle upload");
-    }
     const CrtConst c = make_crt(rns, is32, n, b);
     if (hipMemcpy(crt, &c, sizeof(c), hipMemcpyHostToDevice) != hipSuccess) return set_error(GFE_EHIP, "crt upload");
     for (int k = 0; k < 3; ++k) { pr.p[k] = prime_of(is32, k); pr.q[k] = pinv32(pr.p[k]); }
     pr.p[3] = pr.q[3] = 0;
-    can_limb = limb_ok(b, n) && default_limb_plan(n).limb;
+    for (int k = 0; k < 4; ++k) {
+        pr4.p[k] = prime_of(LIMB_SET, k);
+        pr4.q[k] = pinv32(pr4.p[k]);
+    }
+    can_limb = limb_made = limb_ok(b, n) && default_limb_plan(n).limb;
     if (can_limb) {
-        // the two-digit-limb transform: four tables of N/2 twiddles and its CRT constants
-        const size_t M = N / 2;
-        if (hipMalloc(&tw_limb, 4 * M * 4) != hipSuccess || hipMalloc(&limb_crt, sizeof(LimbCrt)) != hipSuccess)
-            return set_error(GFE_ENOMEM, "device allocation failed");
-        std::vector<uint32_t> htw(4 * M);
-        const int sets[4] = {LIMB_SET, LIMB_SET, LIMB_SET, LIMB_SET}, primes[4] = {0, 1, 2, 3};
-        make_twiddle_tables(sets, primes, 4, n - 1, htw.data());
-        if (hipMemcpy(tw_limb, htw.data(), 4 * M * 4, hipMemcpyHostToDevice) != hipSuccess)
-            return set_error(GFE_EHIP, "twiddle upload");
-        const LimbCrt lc = make_limb_crt(n, b);
-        if (hipMemcpy(limb_crt, &lc, sizeof(lc), hipMemcpyHostToDevice) != hipSuccess)
-            return set_error(GFE_EHIP, "crt upload");
-        for (int k = 0; k < 4; ++k) {
-            pr4.p[k] = prime_of(LIMB_SET, k);
-            pr4.q[k] = pinv32(pr4.p[k]);
-            bm4[k] = mulw_const(b % pr4.p[k], pr4.p[k]);
-        }
+        limb_constants();
         plan = engine_plan_for(b, n);
     }
     // the double-precision transform's tables, of three primes whatever b needs: a rebase may need them
     if (hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess || hipMalloc(&crt64, sizeof(F64Crt)) != hipSuccess)
         return set_error(GFE_ENOMEM, "device allocation failed");
     if (f64_build_twiddles(n, tw64, stream) != 0) return set_error(GFE_EHIP, "twiddles");
-    const int rc = f64_select();
+    int rc = f64_select();
+    if (rc == GFE_OK && !f64) rc = int_tables();
     if (rc != GFE_OK) return rc;
     if (hipMemsetAsync(regs, 0, (size_t)num_regs * N * 4, stream) != hipSuccess) return set_error(GFE_EHIP, "memset");
     for (int i = 0; i < 12; ++i) { hipEvent_t ev; if (hipEventCreate(&ev) != hipSuccess) return set_error(GFE_EHIP, "event"); events.push_back(ev); }
     if (hipStreamSynchronize(stream) != hipSuccess) return set_error(GFE_EHIP, "init sync");
+    return GFE_OK;
+}
+
+// The limb transform's constants for b.
+void Engine::limb_constants() {
+    for (int k = 0; k < 4; ++k) bm4[k] = mulw_const(b % pr4.p[k], pr4.p[k]);
+    limb_crt_host = make_limb_crt(n, b);
+}
+
+// The integer passes' twiddle tables and the limb transform's constants on the device: made when
+// those passes are first selected (their tables take most of an engine's set-up, 0.2 s at n = 23).
+int Engine::int_tables() {
+    if (!tw) {
+        uint32_t *t = nullptr;
+        if (hipMalloc(&t, (size_t)rns * N * 4) != hipSuccess) return set_error(GFE_ENOMEM, "device allocation failed");
+        std::vector<uint32_t> htw((size_t)rns * N);
+        const int sets[3] = {is32, is32, is32}, primes[3] = {0, 1, 2};
+        make_twiddle_tables(sets, primes, rns, n, htw.data());
+        if (hipMemcpy(t, htw.data(), (size_t)rns * N * 4, hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(t);
+            return set_error(GFE_EHIP, "twiddle upload");
+        }
+        tw = t;
+    }
+    if (!can_limb) return GFE_OK;
+    if (!tw_limb) {
+        // the two-digit-limb transform: four tables of N/2 twiddles
+        const size_t M = N / 2;
+        uint32_t *t = nullptr;
+        if (hipMalloc(&t, 4 * M * 4) != hipSuccess || (!limb_crt && hipMalloc(&limb_crt, sizeof(LimbCrt)) != hipSuccess)) {
+            (void)hipFree(t);
+            return set_error(GFE_ENOMEM, "device allocation failed");
+        }
+        std::vector<uint32_t> htw(4 * M);
+        const int sets[4] = {LIMB_SET, LIMB_SET, LIMB_SET, LIMB_SET}, primes[4] = {0, 1, 2, 3};
+        make_twiddle_tables(sets, primes, 4, n - 1, htw.data());
+        if (hipMemcpy(t, htw.data(), 4 * M * 4, hipMemcpyHostToDevice) != hipSuccess) {
+            (void)hipFree(t);
+            return set_error(GFE_EHIP, "twiddle upload");
+        }
+        tw_limb = t;
+    }
+    if (hipMemcpy(limb_crt, &limb_crt_host, sizeof(LimbCrt), hipMemcpyHostToDevice) != hipSuccess)
+        return set_error(GFE_EHIP, "crt upload");
     return GFE_OK;
 }
 
@@ -1305,7 +1331,7 @@ int gfe_set_digits(gfe_engine *e, uint32_t reg, const int32_t *in) {
 size_t gfe_mem_size(const gfe_engine *e) {
     if (!e) return 0;
     const Engine &g = e->eng;
-    return gfe::engine_bytes(g.rns, g.N, g.num_regs, g.tw_limb != nullptr);
+    return gfe::engine_bytes(g.rns, g.N, g.num_regs, g.limb_made);
 }
 
 size_t gfe_cache_size(const gfe_engine *e) {
@@ -1508,6 +1534,8 @@ int gfe_tune(gfe_engine *e, uint32_t reps) {
     GFE_GUARD(e);
     e->eng.flush_carry();
     Engine &g = e->eng;
+    const int rc = g.int_tables();
+    if (rc != GFE_OK) return rc;
     if (reps == 0) reps = 8;
     std::vector<int32_t> saved(g.N), trial(g.N);
     if (hipMemcpyAsync(saved.data(), g.regs, g.N * 4, hipMemcpyDeviceToHost, g.stream) != hipSuccess ||
@@ -1632,15 +1660,11 @@ int gfe_rebase(gfe_engine *e, uint32_t b) {
     g.rounds = gfe::carry_rounds(b, g.n);
     const gfe::CrtConst c = gfe::make_crt(g.rns, g.is32, g.n, b);
     if (hipMemcpy(g.crt, &c, sizeof(c), hipMemcpyHostToDevice) != hipSuccess) return set_error(GFE_EHIP, "crt upload");
-    g.can_limb = g.tw_limb != nullptr && gfe::limb_ok(b, g.n) && gfe::default_limb_plan(g.n).limb;
-    if (g.can_limb) {
-        const gfe::LimbCrt lc = gfe::make_limb_crt(g.n, b);
-        if (hipMemcpy(g.limb_crt, &lc, sizeof(lc), hipMemcpyHostToDevice) != hipSuccess)
-            return set_error(GFE_EHIP, "crt upload");
-        for (int k = 0; k < 4; ++k) g.bm4[k] = gfe::mulw_const(b % g.pr4.p[k], g.pr4.p[k]);
-    }
+    g.can_limb = g.limb_made && gfe::limb_ok(b, g.n) && gfe::default_limb_plan(g.n).limb;
+    if (g.can_limb) g.limb_constants();
     g.plan = g.can_limb ? gfe::engine_plan_for(b, g.n) : gfe::default_plan(g.n);
-    const int rc = g.f64_select();
+    int rc = g.f64_select();
+    if (rc == GFE_OK && !g.f64) rc = g.int_tables();
     return rc != GFE_OK ? rc : g.check("rebase");
 }
 
@@ -1652,6 +1676,8 @@ int gfe_set_plan(gfe_engine *e, const int32_t plan[6]) {
     if (P.limb && !e->eng.can_limb) return set_error(GFE_EINVAL, "the limb transform is not exact for this (b, n)");
     if (P.limb && P.fused && !gfe::limb_fused_ok(e->eng.b, e->eng.n, P.col_ng))
         return set_error(GFE_EINVAL, "the fused limb normalisation is not exact for this (b, n) and column group");
+    const int rc = e->eng.int_tables();
+    if (rc != GFE_OK) return rc;
     e->eng.flush_carry();
     if (hipStreamSynchronize(e->eng.stream) != hipSuccess) return set_error(GFE_EHIP, "set_plan sync");
     e->eng.plan = P;
