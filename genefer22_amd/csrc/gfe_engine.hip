@@ -147,13 +147,6 @@ static uint32_t pinv32(uint32_t p) {
 // Operand of ModS::mulw / ModU::mulw for the constant w: its Montgomery form w 2^32 mod p.
 uint32_t mulw_const(uint32_t w, uint32_t p) { return (uint32_t)((((uint64_t)w) << 32) % p); }
 
-uint32_t psi_mont(int is32, int k, uint32_t n) {
-    const uint32_t p = prime_of(is32, k), g = gen_of(is32, k);
-    return mulw_const(hpow(g, (p - 1) >> (n + 1), p), p);
-}
-
-uint32_t prime_qinv(uint32_t p) { return pinv32(p); }
-
 // create_ocl's rule, src/transform_ocl.cpp:35-50.
 void select_primes(uint32_t b, uint32_t n, int *rns, int *is32) {
     const uint64_t bb = (uint64_t)b * b, N = (uint64_t)1 << n;
@@ -824,18 +817,16 @@ int Engine::int_tables() {
     return GFE_OK;
 }
 
-void Engine::bind(uint32_t b_, uint32_t n_, int device_, hipStream_t stream_, int32_t *digits, uint32_t *ws_,
-                  uint32_t *tw_, int64_t *carry_, CrtConst *crt_, const Plan &plan_) {
+void Engine::bind(uint32_t b_, uint32_t n_, int device_, hipStream_t stream_, int32_t *digits, void *ws_, double *tw_,
+                  int64_t *carry_, F64Crt *crt_) {
     b = b_; n = n_; num_regs = 1; device = device_;
     N = (size_t)1 << n;
-    select_primes(b, n, &rns, &ref_is32);
-    is32 = transform_is32(rns, ref_is32);
     stream = stream_;
-    regs = digits; ws = ws_; zp = nullptr; tw = tw_; carry = carry_; crt = crt_;
-    plan = plan_;
-    rounds = carry_rounds(b, n);
-    cus = 256;
-    for (int k = 0; k < 3; ++k) { pr.p[k] = prime_of(is32, k); pr.q[k] = pinv32(pr.p[k]); }
+    regs = digits; ws = static_cast<uint32_t *>(ws_); zp = nullptr; carry = carry_;
+    tw64 = tw_; crt64 = crt_;
+    f64_k = f64_primes(b, n);
+    shape = f64_shape(n);
+    f64 = true;
     carry_pending = false;
     dev_ok = false;  // nothing here is the engine's to free
 }

@@ -156,11 +156,10 @@ int gfe_host_twiddles(uint32_t n, int is32, int max_threads, uint32_t *out);
  * Squares the N = 2^n balanced digits at `digits` -- device memory of `device`, read and written in
  * place, digits as gfe_get_digits returns them (|d| <= b/2 + 4) -- `count` times, squaring i
  * doubled when bit i mod 64 of dup_bits is set, queued on `stream` (a hipStream_t; NULL = the null
- * stream), and returns without waiting.  The squarings run the digit transform's default plan
- * (gfe_default_plan(n, 0)): the digits equal those of `count` gfe_square_dup calls on an engine of
- * the same (b, n) on that plan followed by gfe_get_digits, and their value equals the engine's on
- * any plan (where an engine starts on the two-digit-limb transform, its balanced digits may differ
- * from these while the residue is the same).  The transform work space, twiddles,
+ * stream), and returns without waiting.  The squarings run in the double-precision limb transform, as
+ * an engine's do: the digits equal those of `count` gfe_square_dup calls on an engine of the same (b, n)
+ * followed by gfe_get_digits (an engine on a plan set by gfe_set_plan has the same residue; its
+ * balanced digits may differ in a carry left at b/2).  The transform work space, twiddles,
  * carries and CRT constants live in one static device array of GFE_NOALLOC_BYTES that the library
  * holds on every device it runs on until the process ends, which limits n to
  * 12 <= n <= GFE_NOALLOC_MAX_N (GFE_EINVAL beyond); no device or host memory is allocated or freed.

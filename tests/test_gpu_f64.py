@@ -145,3 +145,27 @@ def test_plan_change_during_a_proofs_powers(gfe, at):
     bt.close()
     for r in got:
         assert (r["res64"], r["pkey"], r["mu_hash64"], r["gl_ok"]) == (want["res64"], want["pkey"], want["mu_hash64"], 1)
+
+
+@pytest.mark.parametrize("b,n", [(1026, 12), (1999999998, 13), (15300000, 14), (1999999998, 16)])
+def test_noalloc_digits_equal_the_engines(gfe, b, n):
+    """gfe_square_noalloc from extreme digits, one squaring and 65 (the doubling pattern's period and one)."""
+    from test_zz_no_alloc import Hip
+    h, hip, t = b // 2 + 4, Hip(), gfe.Transform(b, n)
+    hip.ck(hip.h.hipSetDevice(0), "hipSetDevice")
+    buf, got, dup = hip.malloc(4 << n), np.empty(1 << n, dtype=np.int32), 0x8000000000000003
+    try:
+        for d in (np.full(1 << n, -h), np.random.RandomState(n).randint(-h, h + 1, 1 << n)):
+            for count in (1, 65):
+                d = np.ascontiguousarray(d, dtype=np.int32)
+                hip.to_device(buf, d)
+                rc = gfe.lib().gfe_square_noalloc(b, n, 0, buf, count, dup, None)
+                assert rc == 0, gfe.lib().gfe_last_error()
+                hip.ck(hip.h.hipDeviceSynchronize(), "hipDeviceSynchronize")
+                hip.to_host(got, buf)
+                t.set_digits(d)
+                for i in range(count):
+                    t.square_dup((dup >> (i % 64)) & 1)
+                assert np.array_equal(got, t.get_digits()), count
+    finally:
+        hip.h.hipFree(buf)
