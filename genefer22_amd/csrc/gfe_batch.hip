@@ -709,7 +709,7 @@ F64Args Batch::args64(const uint8_t *active, const uint8_t *dup, const uint8_t *
     A.tw = tw64; A.tws = (uint32_t)f64_tw_words(nalloc); A.slots = reinterpret_cast<int4 *>(carry); A.crt = crt64;
     A.active = active; A.dupf = dup; A.mulf = mulf;
     A.reg_stride = (long long)(nregs * NA); A.ws_stride = (long long)(3 * NA / 2); A.slot_stride = (long long)(NA / 16);
-    A.nslots = zdim(); A.tn = (int)nalloc - 1; A.a = shape.a; A.ng = shape.row_ng; A.mixed = mixed;
+    A.nslots = zdim(); A.tn = (int)nalloc - 1; A.a = shape.a; A.mixed = mixed;
     return A;
 }
 

@@ -1099,7 +1099,7 @@ F64Args Engine::f64_args(int dup) const {
     memset(&A, 0, sizeof(A));
     A.regs = regs; A.ws = reinterpret_cast<double *>(ws); A.zp = reinterpret_cast<const double *>(zp);
     A.tw = tw64; A.tws = (uint32_t)f64_tw_words(n); A.slots = reinterpret_cast<int4 *>(carry); A.crt = crt64;
-    A.nslots = 1; A.K = f64_k; A.tn = (int)n - 1; A.a = shape.a; A.ng = shape.row_ng; A.dup = dup;
+    A.nslots = 1; A.K = f64_k; A.tn = (int)n - 1; A.a = shape.a; A.dup = dup;
     return A;
 }
 

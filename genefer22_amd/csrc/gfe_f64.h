@@ -46,7 +46,8 @@ constexpr int F64_PRIMES = 3;
 constexpr uint64_t F64_P[F64_PRIMES] = {562949869535233ull, 562949517213697ull, 562949282332673ull};
 constexpr uint32_t F64_G[F64_PRIMES] = {5, 10, 3};
 constexpr int F64_NG = 16;       // columns per workgroup: one 16-lane DPP row of limbs
-constexpr int F64_ROW_MIN = 6, F64_ROW_MAX = 14, F64_COL_MIN = 5, F64_COL_MAX = 8;
+constexpr int F64_ROW_MIN = 6, F64_ROW_MAX = 14, F64_ROW8_MAX = 13, F64_COL_MIN = 5, F64_COL_MAX = 8,
+              F64_SPLIT_MAX = 7;
 constexpr int F64_WHOLE_MIN = 11, F64_WHOLE_MAX = 12;           // log2 limbs of a one-workgroup transform
 constexpr uint32_t F64_NORM_T = 64, F64_NORM_PER = 1, F64_NORM_RANGE = F64_NORM_T * F64_NORM_PER;  // its normalisation
 constexpr int F64_COL_E = 3;     // log2 of the residues per thread in the column passes
@@ -228,19 +229,19 @@ struct F64Geo {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Row pass: rows of 2^LOGG contiguous residues, 16 per thread, thread s of a row.  Exchanges through
-// LDS at k + (k >> 4) (64-bit accesses of 16 consecutive lanes fall in distinct banks in every
-// chunk).  MODE as in gfe_kernels.h: square, product by zp, or forward only.
+// Row pass: rows of 2^LOGG contiguous residues, 2^LOGE per thread, thread s of a row.  Exchanges through
+// LDS at k + (k >> LOGE) (64-bit accesses of 16 consecutive lanes fall in distinct banks in every
+// chunk with 16 residues per thread, and with 8 but for one lane of 16).  MODE as in gfe_kernels.h: square, product by zp, or forward only.
 
 // F64_EITHER: a square, or the product where `mul` (uniform over the workgroup): rounds of batched powers.
 
 enum { F64_SQUARE = 0, F64_MUL = 1, F64_FWD = 2, F64_EITHER = 3 };
 
-__host__ __device__ constexpr uint32_t f64_row_words(int logg) { return (1u << logg) + (1u << (logg - 4)); }
+__host__ __device__ constexpr uint32_t f64_row_words(int logg, int loge) { return (1u << logg) + (1u << (logg - loge)); }
 
-// Between the LDS writes of a chunk and the next chunk's reads, YL the larger of their strides' logs: a
-// sub-transform then spans 2^(YL + 4) consecutive residues, and up to 1024 of them belong to one
-// wave, whose own accesses stay in order; beyond that the workgroup's threads meet.  (A thread writes
+// Between the LDS writes of a chunk and the next chunk's reads, YL the larger of their strides' logs: up
+// to 6 the elements of a wave's 64 threads are the same run of residues in both chunks, and a
+// wave's own accesses stay in order; beyond that the workgroup's threads meet.  (A thread writes
 // back the very elements it has read, so nothing is needed between its reads and its writes.)
 template <int YL>
 __device__ __forceinline__ void f64_exchange() {
@@ -252,7 +253,8 @@ __device__ __forceinline__ void f64_exchange() {
     }
 }
 
-__device__ __forceinline__ constexpr uint32_t f64_off(uint32_t rr, int YL) { return (rr << YL) + ((rr << YL) >> 4); }
+template <int LOGE>
+__device__ __forceinline__ constexpr uint32_t f64_off(uint32_t rr, int YL) { return (rr << YL) + ((rr << YL) >> LOGE); }
 
 // (a0..a3)^2 mod X^4 - w, operands reduced; results below 1.8 p.
 __device__ __forceinline__ void f64_quad_square(const F64Mod &md, double &a0, double &a1, double &a2, double &a3, double w) {
@@ -281,81 +283,102 @@ __device__ __forceinline__ void f64_quad_mul(const F64Mod &md, double &a0, doubl
 
 // load(x, base, YL): the first chunk's elements base + rr 2^YL, at most 0.52 p.  `data` / `zp` at the
 // row's first residue, `row` its index among the 2^a rows, L its LDS words.
-template <int LOGG, int MODE, class LD>
+template <int LOGG, int LOGE, int MODE, class LD>
 __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, double *__restrict__ data,
                                              const double *__restrict__ zp, const double *__restrict__ tw, int a,
                                              uint32_t row, uint32_t s, double *L, bool mul) {
-    using GM = F64Geo<LOGG, 4>;
-    constexpr int LAST = GM::NCH - 1;
-    static_assert(LOGG >= 6, "two chunks at least");
-    double x[16], w[16];
-    f64_for<0, GM::NCH>([&](auto cc) {
+    using GM = F64Geo<LOGG, LOGE>;
+    constexpr int E = 1 << LOGE, LAST = GM::NCH - 1;
+    static_assert(GM::NCH >= 2, "two chunks at least");
+    // With 8 residues per thread a pass is bound by latency: a chunk's twiddles are on their way while the
+    // chunk before it is computed (with 16 the registers go to more waves).
+    constexpr bool AHEAD = LOGE <= 3;
+    double x[E], w[E], wn[E];
+    const auto twiddles = [&](auto cc, auto inv, double (&v)[E]) {
         constexpr int ci = decltype(cc)::value;
-        constexpr int lam0 = GM::lam0(ci), NE = ci == LAST ? 2 : GM::ne(ci), YL = GM::ylog(ci);
+        constexpr int lam0 = GM::lam0(ci), NE = ci == LAST ? LOGE - 2 : GM::ne(ci), YL = GM::ylog(ci);
         // a wave's 64 threads lie in one sub-transform of this level (and in one row)
         constexpr bool UNI = YL >= 6;
+        const uint32_t J = (row << lam0) + (s >> YL);
+        if constexpr (decltype(inv)::value) f64_inv_tw<LOGE, UNI>(v, tw, (uint32_t)(a + lam0), J, NE);
+        else f64_fwd_tw<LOGE, UNI>(v, tw, (uint32_t)(a + lam0), J, NE);
+    };
+    const auto next = [&]() {
+#pragma unroll
+        for (int i = 0; i < E; ++i) w[i] = wn[i];
+    };
+    if constexpr (AHEAD) twiddles(std::integral_constant<int, 0>{}, std::false_type{}, w);
+    f64_for<0, GM::NCH>([&](auto cc) {
+        constexpr int ci = decltype(cc)::value;
+        constexpr int lam0 = GM::lam0(ci), NE = ci == LAST ? LOGE - 2 : GM::ne(ci), YL = GM::ylog(ci);
         const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
-        f64_fwd_tw<4, UNI>(w, tw, (uint32_t)(a + lam0), (row << lam0) + hi, NE);
+        if constexpr (!AHEAD) twiddles(cc, std::false_type{}, w);
+        else if constexpr (ci != LAST) twiddles(std::integral_constant<int, ci + 1>{}, std::false_type{}, wn);
+        else twiddles(cc, std::true_type{}, wn);
         if constexpr (ci == 0) {
             load(x, base, std::integral_constant<int, YL>{});
         } else {
             f64_exchange<GM::ylog(ci - 1)>();
-            const double *p = L + base + (base >> 4);
+            const double *p = L + base + (base >> LOGE);
 #pragma unroll
-            for (int rr = 0; rr < 16; ++rr) x[rr] = p[f64_off(rr, YL)];
+            for (int rr = 0; rr < E; ++rr) x[rr] = p[f64_off<LOGE>(rr, YL)];
         }
-        f64_fwd_chunk<4, NE>(md, x, w);
+        f64_fwd_chunk<LOGE, NE>(md, x, w);
         if constexpr (ci != LAST) {
-            double *p = L + base + (base >> 4);
+            double *p = L + base + (base >> LOGE);
 #pragma unroll
-            for (int rr = 0; rr < 16; ++rr) p[f64_off(rr, YL)] = x[rr];
+            for (int rr = 0; rr < E; ++rr) p[f64_off<LOGE>(rr, YL)] = x[rr];
+            if constexpr (AHEAD) next();
         }
     });
 #pragma unroll
-    for (int rr = 0; rr < 16; ++rr) x[rr] = md.red(x[rr]);
-    const uint32_t base_last = s << 4;
+    for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
+    const uint32_t base_last = s << LOGE;
     if constexpr (MODE == F64_FWD) {
 #pragma unroll
-        for (int rr = 0; rr < 16; rr += 2)
+        for (int rr = 0; rr < E; rr += 2)
             *reinterpret_cast<double2 *>(data + base_last + rr) = make_double2(x[rr], x[rr + 1]);
         return;
     } else {
         if (MODE == F64_SQUARE || (MODE == F64_EITHER && !mul)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                f64_quad_square(md, x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3], (i & 1) ? -w[2 + i / 2] : w[2 + i / 2]);
+            for (int i = 0; i < E / 4; ++i)
+                f64_quad_square(md, x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3], (i & 1) ? -w[E / 8 + i / 2] : w[E / 8 + i / 2]);
         } else {
             const double2 *z = reinterpret_cast<const double2 *>(zp + base_last);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < E / 4; ++i) {
                 const double2 za = z[2 * i], zb = z[2 * i + 1];
                 f64_quad_mul(md, x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3], za.x, za.y, zb.x, zb.y,
-                             (i & 1) ? -w[2 + i / 2] : w[2 + i / 2]);
+                             (i & 1) ? -w[E / 8 + i / 2] : w[E / 8 + i / 2]);
             }
             // a product's coefficients reach 2.4 p: back to F64_KEEP
 #pragma unroll
-            for (int rr = 0; rr < 16; ++rr) x[rr] = md.red(x[rr]);
+            for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
         }
         f64_for_down<0, GM::NCH>([&](auto cc) {
             constexpr int ci = decltype(cc)::value;
-            constexpr int lam0 = GM::lam0(ci), NE = ci == LAST ? 2 : GM::ne(ci), YL = GM::ylog(ci);
-            constexpr bool UNI = YL >= 6;
+            constexpr int lam0 = GM::lam0(ci), NE = ci == LAST ? LOGE - 2 : GM::ne(ci), YL = GM::ylog(ci);
             const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
-            f64_inv_tw<4, UNI>(w, tw, (uint32_t)(a + lam0), (row << lam0) + hi, NE);
+            if constexpr (!AHEAD) twiddles(cc, std::true_type{}, w);
+            else {
+                next();
+                if constexpr (ci > 0) twiddles(std::integral_constant<int, ci - 1>{}, std::true_type{}, wn);
+            }
             if constexpr (ci != LAST) {
                 f64_exchange<YL>();
-                const double *p = L + base + (base >> 4);
+                const double *p = L + base + (base >> LOGE);
 #pragma unroll
-                for (int rr = 0; rr < 16; ++rr) x[rr] = p[f64_off(rr, YL)];
+                for (int rr = 0; rr < E; ++rr) x[rr] = p[f64_off<LOGE>(rr, YL)];
             }
-            f64_inv_chunk<4, NE, true>(md, x, w);
+            f64_inv_chunk<LOGE, NE, true>(md, x, w);
             if constexpr (ci == 0) {
 #pragma unroll
-                for (int rr = 0; rr < 16; ++rr) data[base + (rr << YL)] = x[rr];
+                for (int rr = 0; rr < E; ++rr) data[base + (rr << YL)] = x[rr];
             } else {
-                double *p = L + base + (base >> 4);
+                double *p = L + base + (base >> LOGE);
 #pragma unroll
-                for (int rr = 0; rr < 16; ++rr) p[f64_off(rr, YL)] = x[rr];
+                for (int rr = 0; rr < E; ++rr) p[f64_off<LOGE>(rr, YL)] = x[rr];
             }
         });
     }
@@ -404,13 +427,18 @@ __device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const int2 (&d)[1 
     using GM = F64Geo<LOGG, LOGE>;
     constexpr int E = 1 << LOGE;
     const uint32_t q = t & 15u, s = t >> 4;
-    double x[E], w[E];
+    double x[E], w[E], wn[E];
+    const auto twiddles = [&](auto cc, double (&v)[E]) {
+        constexpr int ci = decltype(cc)::value;
+        constexpr bool UNI = GM::ylog(ci) >= 2;  // a wave holds four consecutive s
+        f64_fwd_tw<LOGE, UNI>(v, tw, (uint32_t)GM::lam0(ci), s >> GM::ylog(ci), GM::ne(ci));
+    };
+    twiddles(std::integral_constant<int, 0>{}, w);
     f64_for<0, GM::NCH>([&](auto cc) {
         constexpr int ci = decltype(cc)::value;
         constexpr int lam0 = GM::lam0(ci), NE = GM::ne(ci), YL = GM::ylog(ci);
-        constexpr bool UNI = YL >= 2;  // a wave holds four consecutive s
         const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
-        f64_fwd_tw<LOGE, UNI>(w, tw, (uint32_t)lam0, hi, NE);
+        if constexpr (ci + 1 < GM::NCH) twiddles(std::integral_constant<int, ci + 1>{}, wn);
         if constexpr (ci == 0) {
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
@@ -430,6 +458,8 @@ __device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const int2 (&d)[1 
             double *p = lds + base * 16 + q;
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) p[(uint32_t)rr << (YL + 4)] = x[rr];
+#pragma unroll
+            for (int i = 0; i < E; ++i) w[i] = wn[i];
         }
     });
 }
@@ -453,13 +483,17 @@ __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << L
     using GM = F64Geo<LOGG, LOGE>;
     constexpr int E = 1 << LOGE;
     const uint32_t q = t & 15u, s = t >> 4;
-    double w[E];
+    double w[E], wn[E];
+    const auto twiddles = [&](auto cc, double (&v)[E]) {
+        constexpr int ci = decltype(cc)::value;
+        f64_inv_tw<LOGE, (GM::ylog(ci) >= 2)>(v, tw, (uint32_t)GM::lam0(ci), s >> GM::ylog(ci), GM::ne(ci));
+    };
+    twiddles(std::integral_constant<int, GM::NCH - 1>{}, w);
     f64_for_down<0, GM::NCH>([&](auto cc) {
         constexpr int ci = decltype(cc)::value;
         constexpr int lam0 = GM::lam0(ci), NE = GM::ne(ci), YL = GM::ylog(ci);
-        constexpr bool UNI = YL >= 2;
         const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
-        f64_inv_tw<LOGE, UNI>(w, tw, (uint32_t)lam0, hi, NE);
+        if constexpr (ci > 0) twiddles(std::integral_constant<int, ci - 1>{}, wn);
         if constexpr (ci != GM::NCH - 1) {
             __syncthreads();
             const double *p = lds + base * 16 + q;
@@ -472,6 +506,8 @@ __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << L
             double *p = lds + base * 16 + q;
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) p[(uint32_t)rr << (YL + 4)] = x[rr];
+#pragma unroll
+            for (int i = 0; i < E; ++i) w[i] = wn[i];
         }
     });
 }

@@ -68,13 +68,13 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_fwd(F64Args 
                                 lds64, bd, reduce);
 }
 
-constexpr int f64_row_threads(int logg) { return logg > 12 ? 1 << (logg - 4) : 256; }
+constexpr int f64_row_threads(int logg, int loge) { return logg - loge > 8 ? 1 << (logg - loge) : 256; }
 
 // 3 2^a / ng workgroups a slot.
-template <int LOGG, int MODE>
-__global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
+template <int LOGG, int LOGE, int MODE>
+__global__ void __launch_bounds__(f64_row_threads(LOGG, LOGE)) k64_row(F64Args A) {
     extern __shared__ double lds64[];
-    constexpr uint32_t SPR = 1u << (LOGG - 4);
+    constexpr uint32_t SPR = 1u << (LOGG - LOGE);
     const uint32_t nb = (1u << A.a) / (uint32_t)A.ng;
     const F64Job J = f64_job(A, 3 * nb);
     const int k = (int)(J.w / nb);
@@ -85,19 +85,22 @@ __global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
     const size_t at = J.slot * A.ws_stride + ((size_t)k << A.tn) + ((size_t)row << LOGG);
     const F64Mod md{J.c->p[k], J.c->pinv[k]};
     double *data = A.ws + at;
-    const auto load = [&](double (&x)[16], uint32_t base, auto yl) {
+    const auto load = [&](double (&x)[1 << LOGE], uint32_t base, auto yl) {
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) x[rr] = data[base + ((uint32_t)rr << decltype(yl)::value)];
+        for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = data[base + ((uint32_t)rr << decltype(yl)::value)];
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) x[rr] = md.red(x[rr]);
+        for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = md.red(x[rr]);
     };
-    f64_row_pass<LOGG, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s, lds64 + q * f64_row_words(LOGG),
+    f64_row_pass<LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
+                                   lds64 + q * f64_row_words(LOGG, LOGE),
                              MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
-// A prime's whole transform, from the digits, in one workgroup; thread s of 2^LOGG / 16.
-template <int LOGG, int MODE>
+// A prime's whole transform, from the digits, in one workgroup; thread s of
+// 2^(LOGG - LOGE).
+template <int LOGG, int LOGE, int MODE>
 __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J, int k, uint32_t s, double *lds) {
+    constexpr int E = 1 << LOGE;
     const F64CrtP c = J.c;
     const F64Mod md{c->p[k], c->pinv[k]};
     const double bd = c->bd;
@@ -105,35 +108,35 @@ __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J
     const int2 *src = reinterpret_cast<const int2 *>(A.regs + J.slot * A.reg_stride + (size_t)A.src_reg * (2u << LOGG));
     const int4 *ls = A.absorb ? A.slots + J.slot * A.slot_stride : nullptr;
     const size_t at = J.slot * A.ws_stride + ((size_t)k << LOGG);
-    const auto load = [&](double (&x)[16], uint32_t base, auto yl) {
+    const auto load = [&](double (&x)[E], uint32_t base, auto yl) {
         constexpr int YL = decltype(yl)::value;
-        int2 d[16];
+        int2 d[E];
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) d[rr] = src[base + ((uint32_t)rr << YL)];
+        for (int rr = 0; rr < E; ++rr) d[rr] = src[base + ((uint32_t)rr << YL)];
         if (ls && (base & 15u) < 2) {  // as f64_load_digits
             const uint32_t q = base & 1u;
-            int2 e[16];
+            int2 e[E];
 #pragma unroll
-            for (int rr = 0; rr < 16; ++rr) e[rr] = reinterpret_cast<const int2 *>(ls + ((base + ((uint32_t)rr << YL)) >> 4))[q];
+            for (int rr = 0; rr < E; ++rr) e[rr] = reinterpret_cast<const int2 *>(ls + ((base + ((uint32_t)rr << YL)) >> 4))[q];
 #pragma unroll
-            for (int rr = 0; rr < 16; ++rr) {
+            for (int rr = 0; rr < E; ++rr) {
                 d[rr].x += e[rr].x;
                 d[rr].y += q == 0 ? e[rr].y : 0;
             }
         }
 #pragma unroll
-        for (int rr = 0; rr < 16; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
+        for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
     };
-    f64_row_pass<LOGG, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
+    f64_row_pass<LOGG, LOGE, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
                              MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
 // 3 workgroups a slot.
-template <int LOGG, int MODE>
-__global__ void __launch_bounds__(1 << (LOGG - 4)) k64_whole(F64Args A) {
+template <int LOGG, int LOGE, int MODE>
+__global__ void __launch_bounds__(1 << (LOGG - LOGE)) k64_whole(F64Args A) {
     extern __shared__ double lds64[];
     const F64Job J = f64_job(A, 3);
-    if (J.run && (int)J.w < J.K) f64_whole_body<LOGG, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    if (J.run && (int)J.w < J.K) f64_whole_body<LOGG, LOGE, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
 }
 
 // A mixed batch: each workgroup at its slot's n, 12 or 13 (of the 256 threads n = 12 takes two whole
@@ -143,8 +146,8 @@ __global__ void __launch_bounds__(256) k64_whole_mixed(F64Args A) {
     extern __shared__ double lds64[];
     const F64Job J = f64_job(A, 3);
     if (!J.run || (int)J.w >= J.K) return;
-    if (J.c->n == 13) f64_whole_body<12, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
-    else if (threadIdx.x < 128) f64_whole_body<11, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    if (J.c->n == 13) f64_whole_body<12, 4, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    else if (threadIdx.x < 128) f64_whole_body<11, 4, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
 }
 
 template <int K, int LOGG>
@@ -172,6 +175,35 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_inv(F64Args 
     const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
     if (J.K == 2) f64_inv_body<2, LOGG>(A, J, dup, lds64);
     else f64_inv_body<3, LOGG>(A, J, dup, lds64);
+}
+
+// One candidate's inverse column pass with its primes side by side: K groups of 16 2^(LOGG - LOGE) threads,
+// one prime each, then all threads over the limbs.  C / 16 workgroups.
+template <int K, int LOGG>
+__global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_split(F64Args A) {
+    extern __shared__ double lds64[];
+    constexpr int LOGE = F64_COL_E, E = 1 << LOGE;
+    constexpr uint32_t T = 16u << (LOGG - LOGE), LIMBS = 16u << LOGG;
+    const F64CrtP c = (F64CrtP)A.crt;
+    const uint32_t M = 1u << A.tn, C = M >> LOGG;
+    const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / T);
+    const uint32_t t = threadIdx.x % T;
+    const unsigned blk = xcd_block(blockIdx.x, C / 16);
+    double x[E], *L = lds64 + k * LIMBS;
+    f64_col_load<LOGE, LOGG>(x, A.ws + (size_t)k * M, C, blk, t);
+    f64_col_inv<LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, x, A.tw + (size_t)k * A.tws, t, L);
+#pragma unroll
+    for (int rr = 0; rr < E; ++rr) L[((t >> 4) + ((uint32_t)rr << (LOGG - LOGE))) * 16 + (t & 15u)] = x[rr];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t j = 0; j < (LIMBS + K * T - 1) / (K * T); ++j) {
+        const uint32_t i = threadIdx.x + j * K * T;
+        if (i >= LIMBS) break;  // whole waves
+        double r[K];
+#pragma unroll
+        for (int m = 0; m < K; ++m) r[m] = lds64[m * LIMBS + i];
+        f64_norm_limb<K>(c, r, A.dup, (i >> 4) * C + blk * 16 + (i & 15u), M, A.regs, A.slots);
+    }
 }
 
 template <int K>
@@ -343,25 +375,26 @@ int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
 
 
 // One candidate, timed on MI355X (us per squaring, three primes unless said).  Up to 2^12 limbs the
-// two launches with a prime's transform in one workgroup beat the three (2^11 limbs 9.3 against
-// 13.1, 2^12 11.0 against 13.4; at 2^13 one workgroup's arithmetic takes longer, 16.8 against 14.0;
+// two launches with a prime's transform in one workgroup beat the three (2^11 limbs 7.6 against
+// 10.1, 2^12 9.7 against 10.6; at 2^13 one workgroup's arithmetic takes longer, 16.8 against 14.0;
 // in batches 100 candidates of 2^13 limbs 32.8 against 31.6, 512 of 2^14 230 against 228).
-// With three passes, up to 2^19 limbs each is bound by latency, so the shapes that win are those with
-// the most workgroups: short columns, one wave per row workgroup, a workgroup per prime in the
-// forward column pass (2^15 limbs: 15.0 with 2^5-point columns, 15.5 with 2^6, 16.3 with all primes
-// in one workgroup; 2^18: 23.5 with 2^6, 25.3 with 2^7).  From 2^20 limbs the passes are bound by
-// memory and fp64 issue and longer columns pay, the digits then being read once for all primes
-// (2^21 limbs: 81.8 with 2^8-point columns, 89.6 with 2^7).  The integer passes at the same sizes:
-// 14.5, 15.6, 15.9, 16.5, 18.8, 20.0, 25.8, 36.9, 41.8, 57.8, 89.3 at n = 12, 13, .., 22 (the last
-// eight limbs of two digits where those are exact).
+// With three passes, up to 2^19 limbs each is bound by latency: a wave issues one instruction in four
+// clocks, and with 16 residues a thread the row pass of 2^14 limbs was 5.2 us in a few waves.  So the
+// shapes that win there have many workgroups and short threads (`few`: 8 residues per thread in the
+// rows, the primes side by side in the inverse column pass; 2^14 limbs 14.7 -> 11.0, 2^16 16.5 ->
+// 12.9, 2^17 19.1 -> 16.4, 2^18 23.4 -> 21.1, 2^19 36.3 -> 34.0) and short columns (2^14 limbs: 11.4
+// with 2^5-point columns, 11.9 with 2^6; 2^16: 13.0 and 13.6; 2^17 16.7 and 15.9).  From 2^20 limbs
+// the passes are bound by memory and fp64 issue and longer columns pay, the digits then being read
+// once for all primes (2^21 limbs: 81.8 with 2^8-point columns, 89.6 with 2^7).  The integer passes at
+// the same sizes: 14.5, 15.6, 15.9, 16.5, 18.8, 20.0, 25.8, 36.9, 41.8, 57.8, 89.3 at n = 12, 13, .., 22
+// (the last eight limbs of two digits where those are exact).
 F64Shape f64_shape(uint32_t n) {
     F64Shape S;
     const int tn = (int)n - 1;
     S.whole = tn <= F64_WHOLE_MAX;
-    S.a = tn <= 15 ? 5 : tn <= 18 ? 6 : tn == 19 ? 7 : 8;
+    S.a = tn <= 16 ? 5 : tn <= 18 ? 6 : tn == 19 ? 7 : 8;
     S.split = tn <= 19;
-    const int spr = 1 << (tn - S.a - 4);
-    S.row_ng = spr >= 64 ? 1 : 64 / spr;
+    S.few = tn <= 19;
     return S;
 }
 
@@ -384,22 +417,33 @@ static F64Fn inv_fn(int a) {
     if constexpr (LOGG > F64_COL_MAX) return nullptr;
     else return a == LOGG ? k64_col_inv<LOGG> : inv_fn<LOGG + 1>(a);
 }
-template <int MODE, int LOGG = F64_ROW_MIN>
-static F64Fn row_fn(int logg) {
-    if constexpr (LOGG > F64_ROW_MAX) return nullptr;
-    else return logg == LOGG ? k64_row<LOGG, MODE> : row_fn<MODE, LOGG + 1>(logg);
+template <int K, int LOGG = F64_COL_MIN>
+static F64Fn split_fn(int a) {
+    if constexpr (LOGG > F64_SPLIT_MAX) return nullptr;
+    else return a == LOGG ? k64_col_inv_split<K, LOGG> : split_fn<K, LOGG + 1>(a);
 }
-template <int MODE, int LOGG = F64_WHOLE_MIN>
+template <int MODE, int LOGE, int LOGG = F64_ROW_MIN>
+static F64Fn row_fn(int logg) {
+    if constexpr (LOGG > (LOGE == 3 ? F64_ROW8_MAX : F64_ROW_MAX)) return nullptr;
+    else return logg == LOGG ? k64_row<LOGG, LOGE, MODE> : row_fn<MODE, LOGE, LOGG + 1>(logg);
+}
+template <int MODE, int LOGE, int LOGG = F64_WHOLE_MIN>
 static F64Fn whole_fn(int logg) {
     if constexpr (LOGG > F64_WHOLE_MAX) return nullptr;
-    else return logg == LOGG ? k64_whole<LOGG, MODE> : whole_fn<MODE, LOGG + 1>(logg);
+    else return logg == LOGG ? k64_whole<LOGG, LOGE, MODE> : whole_fn<MODE, LOGE, LOGG + 1>(logg);
 }
-static F64Fn mid_fn(bool whole, int mode, int logg) {
+template <int MODE>
+static F64Fn mid_mode(bool whole, int loge, int logg) {
+    if (loge == 4) return whole ? whole_fn<MODE, 4>(logg) : row_fn<MODE, 4>(logg);
+    if constexpr (MODE == F64_EITHER) return nullptr;  // one candidate's passes have no per-slot kind
+    else return whole ? whole_fn<MODE, 3>(logg) : row_fn<MODE, 3>(logg);
+}
+static F64Fn mid_fn(bool whole, int mode, int loge, int logg) {
     switch (mode) {
-        case F64_SQUARE: return whole ? whole_fn<F64_SQUARE>(logg) : row_fn<F64_SQUARE>(logg);
-        case F64_MUL: return whole ? whole_fn<F64_MUL>(logg) : row_fn<F64_MUL>(logg);
-        case F64_FWD: return whole ? whole_fn<F64_FWD>(logg) : row_fn<F64_FWD>(logg);
-        default: return whole ? whole_fn<F64_EITHER>(logg) : row_fn<F64_EITHER>(logg);
+        case F64_SQUARE: return mid_mode<F64_SQUARE>(whole, loge, logg);
+        case F64_MUL: return mid_mode<F64_MUL>(whole, loge, logg);
+        case F64_FWD: return mid_mode<F64_FWD>(whole, loge, logg);
+        default: return mid_mode<F64_EITHER>(whole, loge, logg);
     }
 }
 
@@ -423,22 +467,24 @@ void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream) {
 }
 
 void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) {
+    const int L = S.whole ? A.tn : A.tn - S.a;
     if (A.mixed) {
         const F64Fn f = mode == F64_SQUARE ? k64_whole_mixed<F64_SQUARE> : mode == F64_MUL ? k64_whole_mixed<F64_MUL>
                                                                                          : k64_whole_mixed<F64_FWD>;
         const dim3 grid = f64_grid(A, 3);
-        hipLaunchKernelGGL(f, grid, dim3(256), (size_t)8 * f64_row_words(12), stream, A);
+        hipLaunchKernelGGL(f, grid, dim3(256), (size_t)8 * f64_row_words(12, 4), stream, A);
         return;
     }
+    const int loge = A.K && S.few ? 3 : 4;
     if (S.whole) {
         const dim3 grid = f64_grid(A, 3);
-        hipLaunchKernelGGL(mid_fn(true, mode, A.tn), grid, dim3(1u << (A.tn - 4)), (size_t)8 * f64_row_words(A.tn), stream, A);
+        hipLaunchKernelGGL(mid_fn(true, mode, loge, L), grid, dim3(1u << (L - loge)), (size_t)8 * f64_row_words(L, loge), stream, A);
         return;
     }
-    const int L = A.tn - S.a;
-    const dim3 grid = f64_grid(A, 3 * ((1u << S.a) / S.row_ng));
-    hipLaunchKernelGGL(mid_fn(false, mode, L), grid, dim3((unsigned)S.row_ng << (L - 4)),
-                       (size_t)8 * S.row_ng * f64_row_words(L), stream, A);
+    A.ng = L - loge >= 6 ? 1 : 64 >> (L - loge);  // rows per workgroup: one wave at least
+    const dim3 grid = f64_grid(A, 3 * ((1u << S.a) / A.ng));
+    hipLaunchKernelGGL(mid_fn(false, mode, loge, L), grid, dim3((unsigned)A.ng << (L - loge)),
+                       (size_t)8 * A.ng * f64_row_words(L, loge), stream, A);
 }
 
 void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
@@ -447,8 +493,12 @@ void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
         hipLaunchKernelGGL(k64_norm, grid, dim3(F64_NORM_T), 0, stream, A);
         return;
     }
-    const unsigned T = 16u << (S.a - F64_COL_E);
-    const dim3 grid = f64_grid(A, 1u << (A.tn - S.a - 4));
+    const unsigned T = 16u << (S.a - F64_COL_E), nb = 1u << (A.tn - S.a - 4);
+    if (A.K && S.few) {
+        hipLaunchKernelGGL(A.K == 2 ? split_fn<2>(S.a) : split_fn<3>(S.a), dim3(nb), dim3(A.K * T), (size_t)A.K * 128 << S.a, stream, A);
+        return;
+    }
+    const dim3 grid = f64_grid(A, nb);
     hipLaunchKernelGGL(inv_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A);
 }
 
@@ -468,10 +518,15 @@ void f64_set_lds_attributes() {
             set((const void *)fwd_fn(a));
             set((const void *)inv_fn(a));
         }
-        for (int m = 0; m < 4; ++m) {
-            for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, l));
-            for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, l));
+        for (int a = F64_COL_MIN; a <= F64_SPLIT_MAX; ++a) {
+            set((const void *)split_fn<2>(a));
+            set((const void *)split_fn<3>(a));
         }
+        for (int m = 0; m < 4; ++m)
+            for (int e = 3; e <= 4; ++e) {
+                for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, e, l));
+                for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, e, l));
+            }
         (void)hipGetLastError();
     });
 }

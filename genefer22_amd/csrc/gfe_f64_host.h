@@ -12,10 +12,11 @@
 namespace gfe {
 
 // Shape of the passes at one n.  whole: a prime's transform in one workgroup and the normalisation
-// after it; else three passes over 2^a rows of 2^(n-1-a) limbs, row_ng rows per workgroup, the
-// forward column pass with one prime per workgroup (split) instead of all.
+// after it; else three passes over 2^a rows of 2^(n-1-a) limbs, the forward column pass with one prime
+// per workgroup (split) instead of all.  few: one candidate's work is too little for the chip, so its
+// passes take fewer residues per thread.
 struct F64Shape {
-    int whole = 0, a = 0, row_ng = 1, split = 0;
+    int whole = 0, a = 0, split = 0, few = 0;
 };
 
 // Primes the transform needs for (b, n): 2 or 3, or 0 where it is not exact (or out of range).
@@ -43,7 +44,8 @@ struct F64Args {
     const uint8_t *active, *dupf, *mulf;  // per slot, or null (all, dup, none)
     long long reg_stride, ws_stride, slot_stride;
     uint32_t src_reg, tws, nslots;
-    int tn, a, ng, dup, absorb;
+    int tn, a, dup, absorb;
+    int ng;                 // rows per workgroup (set by the launches)
     int pin;                // slot s on XCD s mod 8 (set by the launches)
     int mixed;              // slots of n = 12 beside those of n = 13 (tn = 12, whole)
     int K;                  // one candidate's primes, or 0: slots, each with its own
