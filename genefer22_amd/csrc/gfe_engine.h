@@ -95,14 +95,15 @@ struct Engine {
     int tp() const { return plan.limb ? 4 : rns; }               // primes of the transform
     const uint32_t *cur_tw() const { return plan.limb ? tw_limb : tw; }
     const PrimeArgs &cur_pr() const { return plan.limb ? pr4 : pr; }
-    // Double-precision limb transform (gfe_f64.h).  An engine squares with it from its creation where
+    // Double-precision limb transform (gfe_f64.h, gfe_f64q.h).  An engine squares with it from its creation where
     // it is exact (f64_k primes, 0: it is not); gfe_set_plan selects the integer passes instead.
     // Products run in the transform that holds the multiplicand (zp_f64).
     bool f64 = false, zp_f64 = false;
     int f64_k = 0;
     F64Shape shape;
-    double *tw64 = nullptr;
-    F64Crt *crt64 = nullptr;
+    double *tw64 = nullptr, *twq = nullptr;
+    void *crt64 = nullptr, *crtq = nullptr;  // F64Crt, F64QCrt
+    int tables_for(uint32_t b);
     int f64_select();
     F64Args f64_args(int dup) const;
     void f64_run(uint32_t src, uint32_t *out, int mode);

@@ -414,7 +414,7 @@ static size_t work_bytes(size_t N) { return 4 * (size_t)F64_PRIMES * N; }
 // double-precision transform's (3 x N/8 doubles).
 size_t engine_bytes(int rns, size_t N, uint32_t num_regs, bool limb_tables) {
     return (size_t)num_regs * N * 4 + 2 * work_bytes(N) + (size_t)rns * N * 4 + N + (limb_tables ? 8 * N : 0) +
-           (size_t)F64_PRIMES * N;
+           (size_t)F64_PRIMES * N;  // four-digit limbs: less
 }
 
 // An engine's first plan: the limb transform where it is exact (with the inverse column pass and
@@ -715,6 +715,8 @@ Engine::~Engine() {
         (void)hipFree(tw); (void)hipFree(crt);
         if (tw64) (void)hipFree(tw64);
         if (crt64) (void)hipFree(crt64);
+        if (twq) (void)hipFree(twq);
+        if (crtq) (void)hipFree(crtq);
         if (tw_limb) (void)hipFree(tw_limb);
         if (limb_crt) (void)hipFree(limb_crt);
         if (stream) (void)hipStreamDestroy(stream);
@@ -760,12 +762,8 @@ int Engine::init(uint32_t b_, uint32_t n_, uint32_t num_regs_, int device_) {
         limb_constants();
         plan = engine_plan_for(b, n);
     }
-    // the double-precision transform's tables, of three primes whatever b needs: a rebase may need them
-    if (hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess || hipMalloc(&crt64, sizeof(F64Crt)) != hipSuccess)
-        return set_error(GFE_ENOMEM, "device allocation failed");
-    if (f64_build_twiddles(n, tw64, stream) != 0) return set_error(GFE_EHIP, "twiddles");
-    int rc = f64_select();
-    if (rc == GFE_OK && !f64) rc = int_tables();
+    int rc = tables_for(b);
+    if (rc == GFE_OK) rc = f64_select();
     if (rc != GFE_OK) return rc;
     if (hipMemsetAsync(regs, 0, (size_t)num_regs * N * 4, stream) != hipSuccess) return set_error(GFE_EHIP, "memset");
     for (int i = 0; i < 12; ++i) { hipEvent_t ev; if (hipEventCreate(&ev) != hipSuccess) return set_error(GFE_EHIP, "event"); events.push_back(ev); }
@@ -1051,7 +1049,8 @@ void Engine::flush_carry() {
 }
 
 void Engine::launch_carry() {
-    if (pend_kind == 3) f64_launch_flush(f64_args(0), stream);
+    if (pend_kind == 3 && shape.quad) f64q_launch_flush(f64_args(0), b, stream);
+    else if (pend_kind == 3) f64_launch_flush(f64_args(0), stream);
     else if (pend_kind == 2) launch_carry_slots();
     else if (pend_kind == 1) launch_carry_limbs();
     else launch_carry_digits();
@@ -1084,22 +1083,56 @@ void Engine::launch_fused(int dup) {
     hipLaunchKernelGGL(fused_square_fn((int)n), dim3(1), dim3(fused_threads((int)n)), fused_lds_bytes((int)n), stream, A);
 }
 
-// The double-precision transform for the engine's (b, n), where it is exact.
+static bool f64_quad(uint32_t b, uint32_t n) { return f64_primes(b, n) == 3 && f64q_ok(b, n); }
+
+// The tables base b squares with, made when one first needs them: three primes', the five primes' of
+// four-digit limbs, or the integer passes'.  Leaves the engine as it was where that fails.
+int Engine::tables_for(uint32_t b) {
+    if (f64_primes(b, n) == 0) return int_tables();
+    const bool quad = f64_quad(b, n);
+    double *&table = quad ? twq : tw64;
+    void *&consts = quad ? crtq : crt64;
+    if (table) return GFE_OK;
+    if (!consts && hipMalloc(&consts, quad ? f64q_crt_bytes() : sizeof(F64Crt)) != hipSuccess)
+        return set_error(GFE_ENOMEM, "device allocation failed");
+    double *t = nullptr;
+    if (hipMalloc(&t, (quad ? F64Q_PRIMES * f64q_tw_words(n) : F64_PRIMES * f64_tw_words(n)) * 8) != hipSuccess)
+        return set_error(GFE_ENOMEM, "device allocation failed");
+    if ((quad ? f64q_build_twiddles(n, t, stream) : f64_build_twiddles(n, t, stream)) != 0) {
+        (void)hipFree(t);
+        return set_error(GFE_EHIP, "twiddles");
+    }
+    table = t;
+    return GFE_OK;
+}
+
+// The double-precision transform for the engine's (b, n), where it is exact; its tables are there.
 int Engine::f64_select() {
     f64_k = f64_primes(b, n);
     f64 = zp_f64 = f64_k != 0;
     if (!f64) return GFE_OK;
-    const F64Crt c = make_f64_crt(n, b, f64_k);
-    shape = f64_shape(n);
-    return hipMemcpy(crt64, &c, sizeof(c), hipMemcpyHostToDevice) == hipSuccess ? GFE_OK : set_error(GFE_EHIP, "crt upload");
+    const bool quad = f64_quad(b, n);
+    shape = quad ? f64q_shape(n) : f64_shape(n);
+    hipError_t rc;
+    if (quad) {
+        f64_k = F64Q_PRIMES;
+        F64QCrt c;
+        make_f64q_crt(n, b, &c);
+        rc = hipMemcpy(crtq, &c, sizeof(c), hipMemcpyHostToDevice);
+    } else {
+        const F64Crt c = make_f64_crt(n, b, f64_k);
+        rc = hipMemcpy(crt64, &c, sizeof(c), hipMemcpyHostToDevice);
+    }
+    return rc == hipSuccess ? GFE_OK : set_error(GFE_EHIP, "crt upload");
 }
 
 F64Args Engine::f64_args(int dup) const {
     F64Args A;
     memset(&A, 0, sizeof(A));
     A.regs = regs; A.ws = reinterpret_cast<double *>(ws); A.zp = reinterpret_cast<const double *>(zp);
-    A.tw = tw64; A.tws = (uint32_t)f64_tw_words(n); A.slots = reinterpret_cast<int4 *>(carry); A.crt = crt64;
-    A.nslots = 1; A.K = f64_k; A.tn = (int)n - 1; A.a = shape.a; A.dup = dup;
+    A.tw = shape.quad ? twq : tw64; A.tws = (uint32_t)(shape.quad ? f64q_tw_words(n) : f64_tw_words(n));
+    A.slots = reinterpret_cast<int4 *>(carry); A.crt = shape.quad ? crtq : crt64;
+    A.nslots = 1; A.K = f64_k; A.tn = (int)n - (shape.quad ? 2 : 1); A.a = shape.a; A.dup = dup;
     return A;
 }
 
@@ -1644,6 +1677,8 @@ int gfe_rebase(gfe_engine *e, uint32_t b) {
     gfe::select_primes(b, g.n, &rns, &ref_is32);
     if (rns != g.rns || gfe::transform_is32(rns, ref_is32) != g.is32)
         return set_error(GFE_EKIND, "rebase: b selects another prime set at this n");
+    int rc = g.tables_for(b);
+    if (rc != GFE_OK) return rc;
     g.flush_carry();  // register 0's pending carries, in the old base
     if (hipStreamSynchronize(g.stream) != hipSuccess) return set_error(GFE_EHIP, "rebase sync");
     g.b = b;
@@ -1654,8 +1689,8 @@ int gfe_rebase(gfe_engine *e, uint32_t b) {
     g.can_limb = g.limb_made && gfe::limb_ok(b, g.n) && gfe::default_limb_plan(g.n).limb;
     if (g.can_limb) g.limb_constants();
     g.plan = g.can_limb ? gfe::engine_plan_for(b, g.n) : gfe::default_plan(g.n);
-    int rc = g.f64_select();
-    if (rc == GFE_OK && !g.f64) rc = g.int_tables();
+    rc = g.f64_select();
+    if (rc == GFE_OK && !g.f64) rc = g.int_tables();  // limbs of two digits, if this base allows them
     return rc != GFE_OK ? rc : g.check("rebase");
 }
 

@@ -15,7 +15,7 @@
 //
 // Sizes in units of p (p < 2^49, so 2^53 > 16 p).  The rounding of q costs at most
 // 3 2^-53 |a w| / p <= 0.094 B for |a| = B p, |w| <= 0.51 p, so a product is below 0.52 + 0.096 B
-// (prod_bound).  Forward levels add one product per level, so they run unreduced from 2 p through a
+// (F64Wide).  Forward levels add one product per level, so they run unreduced from 2 p through a
 // whole column pass and, from a reduced start, through a whole row pass.  The inverse sums double
 // per level: its reductions are placed at compile time from the same bounds (InvSched).
 //
@@ -97,36 +97,40 @@ __device__ __forceinline__ void f64_for_down(const F &f) {
 // ---------------------------------------------------------------------------------------------
 // Bounds and chunks
 
-constexpr double prod_bound(double B) { return 0.52 + 0.096 * B; }
-constexpr double F64_LIM = 15.0;   // largest operand a butterfly may form (16 p > 2^53 - p)
-constexpr double F64_KEEP = 1.8;   // what an inverse chunk starts from and leaves
+// Bounds of a prime size, in units of p: lim the largest operand a butterfly may form, start what the
+// inverse transform starts from, keep what an inverse chunk leaves, a product of B p by a constant
+// at most 0.52 + slope B; reduce: rows reduce on the way in and before the pointwise products.
+struct F64Wide {  // p < 2^49
+    static constexpr double lim = 15.0, start = 1.8, keep = 1.8, slope = 0.096;
+    static constexpr bool reduce = true;
+};
 
-// Where the inverse chunk of NE levels on 2^LOGE elements, all at most F64_KEEP p, reduces: pre[mu]
-// bit i before level mu, post bit i after the last.
-template <int LOGE, int NE>
+// Where the inverse chunk of NE levels on 2^LOGE elements, all at most B0 p, reduces: pre[mu] bit i
+// before level mu, post bit i after the last.
+template <class SZ, int LOGE, int NE>
 struct InvSched {
     uint32_t pre[NE > 0 ? NE : 1] = {};
     uint32_t post = 0;
-    constexpr InvSched() {
+    constexpr explicit InvSched(double B0) {
         constexpr int E = 1 << LOGE;
         double B[E] = {};
-        for (int i = 0; i < E; ++i) B[i] = F64_KEEP;
+        for (int i = 0; i < E; ++i) B[i] = B0;
         for (int mu = NE - 1; mu >= 0; --mu) {
             const int h = E >> (mu + 1);
             for (int bi = 0; bi < (1 << mu); ++bi)
                 for (int i = 0; i < h; ++i) {
                     const int i0 = bi * 2 * h + i, i1 = i0 + h;
-                    if (B[i0] + B[i1] > F64_LIM) {
-                        if (B[i0] > F64_KEEP) { pre[mu] |= 1u << i0; B[i0] = 0.51; }
-                        if (B[i1] > F64_KEEP) { pre[mu] |= 1u << i1; B[i1] = 0.51; }
+                    if (B[i0] + B[i1] > SZ::lim) {
+                        if (B[i0] > SZ::keep) { pre[mu] |= 1u << i0; B[i0] = 0.51; }
+                        if (B[i1] > SZ::keep) { pre[mu] |= 1u << i1; B[i1] = 0.51; }
                     }
                     const double s = B[i0] + B[i1];
                     B[i0] = s;
-                    B[i1] = prod_bound(s);
+                    B[i1] = 0.52 + SZ::slope * s;
                 }
         }
         for (int i = 0; i < E; ++i)
-            if (B[i] > F64_KEEP) post |= 1u << i;
+            if (B[i] > SZ::keep) post |= 1u << i;
     }
 };
 
@@ -152,11 +156,12 @@ __device__ __forceinline__ void f64_fwd_chunk(const F64Mod &md, double (&x)[1 <<
 }
 
 // Inverse levels NE-1..0: the twiddle of block bi, level mu is -1 / w[2^mu + bi]'s mirror (f64_inv_tw),
-// so the difference enters as v - u.  POST: bring every element back to F64_KEEP.
-template <int LOGE, int NE, bool POST, class W>
+// so the difference enters as v - u.  FIRST: of the inverse transform; POST: bring every element back to
+// SZ::keep.
+template <class SZ, int LOGE, int NE, bool FIRST, bool POST, class W>
 __device__ __forceinline__ void f64_inv_chunk(const F64Mod &md, double (&x)[1 << LOGE], const W &w) {
     constexpr int E = 1 << LOGE;
-    constexpr InvSched<LOGE, NE> S{};
+    constexpr InvSched<SZ, LOGE, NE> S{FIRST ? SZ::start : SZ::keep};
 #pragma unroll
     for (int mu = NE - 1; mu >= 0; --mu) {
         const int h = E >> (mu + 1);
@@ -283,7 +288,7 @@ __device__ __forceinline__ void f64_quad_mul(const F64Mod &md, double &a0, doubl
 
 // load(x, base, YL): the first chunk's elements base + rr 2^YL, at most 0.52 p.  `data` / `zp` at the
 // row's first residue, `row` its index among the 2^a rows, L its LDS words.
-template <int LOGG, int LOGE, int MODE, class LD>
+template <class SZ, int LOGG, int LOGE, int MODE, class LD>
 __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, double *__restrict__ data,
                                              const double *__restrict__ zp, const double *__restrict__ tw, int a,
                                              uint32_t row, uint32_t s, double *L, bool mul) {
@@ -331,8 +336,10 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
             if constexpr (AHEAD) next();
         }
     });
+    if constexpr (SZ::reduce || MODE == F64_FWD) {
 #pragma unroll
-    for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
+        for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
+    }
     const uint32_t base_last = s << LOGE;
     if constexpr (MODE == F64_FWD) {
 #pragma unroll
@@ -352,9 +359,11 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
                 f64_quad_mul(md, x[4 * i], x[4 * i + 1], x[4 * i + 2], x[4 * i + 3], za.x, za.y, zb.x, zb.y,
                              (i & 1) ? -w[E / 8 + i / 2] : w[E / 8 + i / 2]);
             }
-            // a product's coefficients reach 2.4 p: back to F64_KEEP
+            // a product's coefficients reach 2.4 p
+            if constexpr (SZ::reduce) {
 #pragma unroll
-            for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
+                for (int rr = 0; rr < E; ++rr) x[rr] = md.red(x[rr]);
+            }
         }
         f64_for_down<0, GM::NCH>([&](auto cc) {
             constexpr int ci = decltype(cc)::value;
@@ -371,7 +380,7 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
 #pragma unroll
                 for (int rr = 0; rr < E; ++rr) x[rr] = p[f64_off<LOGE>(rr, YL)];
             }
-            f64_inv_chunk<LOGE, NE, true>(md, x, w);
+            f64_inv_chunk<SZ, LOGE, NE, ci == LAST, true>(md, x, w);
             if constexpr (ci == 0) {
 #pragma unroll
                 for (int rr = 0; rr < E; ++rr) data[base + (rr << YL)] = x[rr];
@@ -420,10 +429,11 @@ __device__ __forceinline__ void f64_load_digits(int2 (&d)[1 << LOGE], const int3
     }
 }
 
-template <int LOGE, int LOGG>
-__device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const int2 (&d)[1 << LOGE], double *__restrict__ dst,
+// limb(rr): residue of the limb in row s + rr 2^(LOGG - LOGE).
+template <int LOGE, int LOGG, class LD>
+__device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const LD &limb, double *__restrict__ dst,
                                             const double *__restrict__ tw, uint32_t C, unsigned blk, uint32_t t,
-                                            double *lds, double bd, bool reduce) {
+                                            double *lds) {
     using GM = F64Geo<LOGG, LOGE>;
     constexpr int E = 1 << LOGE;
     const uint32_t q = t & 15u, s = t >> 4;
@@ -441,7 +451,7 @@ __device__ __forceinline__ void f64_col_fwd(const F64Mod &md, const int2 (&d)[1 
         if constexpr (ci + 1 < GM::NCH) twiddles(std::integral_constant<int, ci + 1>{}, wn);
         if constexpr (ci == 0) {
 #pragma unroll
-            for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
+            for (int rr = 0; rr < E; ++rr) x[rr] = limb(rr);
         } else {
             __syncthreads();
             const double *p = lds + base * 16 + q;
@@ -477,7 +487,7 @@ __device__ __forceinline__ void f64_col_load(double (&x)[1 << LOGE], const doubl
 
 // Inverse column levels on x (f64_col_load's layout in, the first forward chunk's out: rows
 // s + rr 2^(LOGG - LOGE)).
-template <int LOGE, int LOGG>
+template <class SZ, int LOGE, int LOGG>
 __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << LOGE], const double *__restrict__ tw,
                                             uint32_t t, double *lds) {
     using GM = F64Geo<LOGG, LOGE>;
@@ -500,7 +510,7 @@ __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << L
 #pragma unroll
             for (int rr = 0; rr < E; ++rr) x[rr] = p[(uint32_t)rr << (YL + 4)];
         }
-        f64_inv_chunk<LOGE, NE, (ci != 0)>(md, x, w);
+        f64_inv_chunk<SZ, LOGE, NE, false, (ci != 0)>(md, x, w);
         if constexpr (ci != 0) {
             if constexpr (ci == GM::NCH - 1) __syncthreads();  // the previous prime's last reads
             double *p = lds + base * 16 + q;
@@ -509,6 +519,60 @@ __device__ __forceinline__ void f64_col_inv(const F64Mod &md, double (&x)[1 << L
 #pragma unroll
             for (int i = 0; i < E; ++i) w[i] = wn[i];
         }
+    });
+}
+
+template <bool FIRST, class T>
+__device__ __forceinline__ T &f64_either(T &a, T &b) {
+    if constexpr (FIRST) return a;
+    else return b;
+}
+
+// f64_col_load and f64_col_inv on x[k] of prime k, mod(k), for K primes as a pipeline: step d runs chunk
+// NCH - 1 - i of prime d - i for every i, from LDS buffer (prime mod NCH), and one barrier ends
+// the step.  (A buffer's last reads, in a prime's last chunk, are a step before the writes of
+// the prime that takes it over.)  K + NCH - 2 barriers instead of 2 K (NCH - 1), and up to NCH
+// independent chains between them; residues at ws + k M, twiddles at tw + k tws.  The first chunk's twiddles
+// differ within a wave and are vector loads, each prime's before its residues': a wait for them
+// would else include the residues of all.
+template <class SZ, int K, int LOGE, int LOGG, class MD>
+__device__ __forceinline__ void f64_cols_inv(const MD &mod, double (&x)[K][1 << LOGE], const double *__restrict__ ws,
+                                             size_t M, const double *__restrict__ tw, size_t tws, uint32_t C,
+                                             unsigned blk, uint32_t t, double *lds) {
+    using GM = F64Geo<LOGG, LOGE>;
+    constexpr int E = 1 << LOGE, NCH = GM::NCH;
+    const uint32_t q = t & 15u, s = t >> 4;
+    double wl[K][E];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        f64_inv_tw<LOGE, false>(wl[k], tw + k * tws, (uint32_t)GM::lam0(NCH - 1), s, GM::ne(NCH - 1));
+        f64_col_load<LOGE, LOGG>(x[k], ws + k * M, C, blk, t);
+    }
+    f64_for<0, K + NCH - 1>([&](auto dd) {
+        constexpr int d = decltype(dd)::value;
+        f64_for<0, NCH>([&](auto cc) {
+            constexpr int ci = decltype(cc)::value, k = d - (NCH - 1 - ci);
+            if constexpr (k >= 0 && k < K) {
+                constexpr int lam0 = GM::lam0(ci), NE = GM::ne(ci), YL = GM::ylog(ci);
+                const uint32_t hi = s >> YL, base = (hi << (LOGG - lam0)) + (s & ((1u << YL) - 1u));
+                double v[E], *p = lds + (k % NCH) * (16u << LOGG) + base * 16 + q;
+                constexpr bool UNI = YL >= 2;
+                if constexpr (UNI) {
+                    f64_inv_tw<LOGE, UNI>(v, tw + k * tws, (uint32_t)lam0, hi, NE);
+                }
+                auto &w = f64_either<UNI>(v, wl[k]);
+                if constexpr (ci != NCH - 1) {
+#pragma unroll
+                    for (int rr = 0; rr < E; ++rr) x[k][rr] = p[(uint32_t)rr << (YL + 4)];
+                }
+                f64_inv_chunk<SZ, LOGE, NE, false, (ci != 0)>(mod(k), x[k], w);
+                if constexpr (ci != 0) {
+#pragma unroll
+                    for (int rr = 0; rr < E; ++rr) p[(uint32_t)rr << (YL + 4)] = x[k][rr];
+                }
+            }
+        });
+        if constexpr (d < K + NCH - 2) __syncthreads();
     });
 }
 
@@ -641,17 +705,21 @@ __device__ __forceinline__ void f64_flush_body(int32_t *dst, int4 *slots, uint32
     slots[w] = make_int4(0, 0, 0, (int32_t)c);
 }
 
-__device__ __forceinline__ void f64_carry_body(int32_t *dst, const int4 *slots, uint32_t nrange, uint32_t b, uint32_t w) {
-    int32_t c = w == 0 ? -slots[nrange - 1].w : slots[w - 1].w;
+// A carry c into balanced digits p[0..N-1], N digits of a range.
+template <int N>
+__device__ __forceinline__ void f64_carry_digits(int32_t *p, int32_t c, uint32_t b) {
     if (c == 0) return;
     const int32_t hi = (int32_t)(b / 2), lo = -(int32_t)((b - 1) / 2);
-    int32_t *p = dst + (size_t)w * 32;
-    for (int i = 0; i < 31 && c != 0; ++i) {
+    for (int i = 0; i < N - 1 && c != 0; ++i) {
         int32_t d = p[i] + c;
         c = (d > hi) - (d < lo);
         p[i] = d - c * (int32_t)b;
     }
-    if (c) p[31] += c;
+    if (c) p[N - 1] += c;
+}
+
+__device__ __forceinline__ void f64_carry_body(int32_t *dst, const int4 *slots, uint32_t nrange, uint32_t b, uint32_t w) {
+    f64_carry_digits<32>(dst + (size_t)w * 32, w == 0 ? -slots[nrange - 1].w : slots[w - 1].w, b);
 }
 
 }  // namespace gfe

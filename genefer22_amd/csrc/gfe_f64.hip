@@ -36,7 +36,7 @@ __device__ __forceinline__ F64Job f64_job(const F64Args &A, uint32_t per) {
         J.w = id - J.slot * per;
     }
     J.run = J.slot < A.nslots && !(A.active && !A.active[J.slot]);
-    J.c = (F64CrtP)(A.crt + (J.run ? J.slot : 0));
+    J.c = (F64CrtP)A.crt + (J.run ? J.slot : 0);
     J.K = J.c->K;
     return J;
 }
@@ -63,9 +63,11 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_fwd(F64Args 
     const bool reduce = c->big == 2;
     double *ws = A.ws + J.slot * A.ws_stride;
 #pragma unroll 1
-    for (int k = k0; k < k1; ++k)
-        f64_col_fwd<LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, d, ws + (size_t)k * M, A.tw + (size_t)k * A.tws, C, blk, t,
-                                lds64, bd, reduce);
+    for (int k = k0; k < k1; ++k) {
+        const F64Mod md{c->p[k], c->pinv[k]};
+        const auto limb = [&](int rr) { return f64_limb(md, d[rr].x, d[rr].y, bd, reduce); };
+        f64_col_fwd<LOGE, LOGG>(md, limb, ws + (size_t)k * M, A.tw + (size_t)k * A.tws, C, blk, t, lds64);
+    }
 }
 
 constexpr int f64_row_threads(int logg, int loge) { return logg - loge > 8 ? 1 << (logg - loge) : 256; }
@@ -91,7 +93,7 @@ __global__ void __launch_bounds__(f64_row_threads(LOGG, LOGE)) k64_row(F64Args A
 #pragma unroll
         for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = md.red(x[rr]);
     };
-    f64_row_pass<LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
+    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
                                    lds64 + q * f64_row_words(LOGG, LOGE),
                              MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
@@ -127,7 +129,7 @@ __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J
 #pragma unroll
         for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
     };
-    f64_row_pass<LOGG, LOGE, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
+    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
                              MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
@@ -161,7 +163,7 @@ __device__ __forceinline__ void f64_inv_body(const F64Args &A, const F64Job &J, 
     for (int k = 0; k < K; ++k) f64_col_load<LOGE, LOGG>(x[k], ws + (size_t)k * M, C, blk, t);
 #pragma unroll
     for (int k = 0; k < K; ++k)
-        f64_col_inv<LOGE, LOGG>(F64Mod{J.c->p[k], J.c->pinv[k]}, x[k], A.tw + (size_t)k * A.tws, t, lds);
+        f64_col_inv<F64Wide, LOGE, LOGG>(F64Mod{J.c->p[k], J.c->pinv[k]}, x[k], A.tw + (size_t)k * A.tws, t, lds);
     f64_norm_store<K, LOGE, LOGG>(J.c, x, C, blk, t, dup, A.regs + J.slot * A.reg_stride,
                                   A.slots + J.slot * A.slot_stride);
 }
@@ -191,7 +193,7 @@ __global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_sp
     const unsigned blk = xcd_block(blockIdx.x, C / 16);
     double x[E], *L = lds64 + k * LIMBS;
     f64_col_load<LOGE, LOGG>(x, A.ws + (size_t)k * M, C, blk, t);
-    f64_col_inv<LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, x, A.tw + (size_t)k * A.tws, t, L);
+    f64_col_inv<F64Wide, LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, x, A.tw + (size_t)k * A.tws, t, L);
 #pragma unroll
     for (int rr = 0; rr < E; ++rr) L[((t >> 4) + ((uint32_t)rr << (LOGG - LOGE))) * 16 + (t & 15u)] = x[rr];
     __syncthreads();
@@ -236,7 +238,7 @@ __global__ void __launch_bounds__(F64_NORM_T) k64_norm(F64Args A) {
 __global__ void __launch_bounds__(256) k64_flush(F64Args A) {
     const uint32_t s = blockIdx.y, w = blockIdx.x * 256u + threadIdx.x;
     if (A.active && !A.active[s]) return;
-    const F64CrtP c = (F64CrtP)(A.crt + s);
+    const F64CrtP c = (F64CrtP)A.crt + s;
     if (c->n == 0 || w >= (1u << c->n) / 32) return;
     f64_flush_body(A.regs + s * A.reg_stride, A.slots + s * A.slot_stride, c->b, w);
 }
@@ -244,7 +246,7 @@ __global__ void __launch_bounds__(256) k64_flush(F64Args A) {
 __global__ void __launch_bounds__(256) k64_carry(F64Args A) {
     const uint32_t s = blockIdx.y, w = blockIdx.x * 256u + threadIdx.x;
     if (A.active && !A.active[s]) return;
-    const F64CrtP c = (F64CrtP)(A.crt + s);
+    const F64CrtP c = (F64CrtP)A.crt + s;
     if (c->n == 0 || w >= (1u << c->n) / 32) return;
     f64_carry_body(A.regs + s * A.reg_stride, A.slots + s * A.slot_stride, (1u << c->n) / 32, c->b, w);
 }
@@ -253,8 +255,8 @@ struct F64TwArgs {
     double *tw;
     uint32_t words;                       // per prime
     int bits;                             // log2 M
-    double p[F64_PRIMES], pinv[F64_PRIMES];
-    double pw[F64_PRIMES][24];            // psi^(2^i)
+    double p[F64Q_PRIMES], pinv[F64Q_PRIMES];
+    double pw[F64Q_PRIMES][22];           // psi^(2^i)
 };
 
 // Psi[j] = psi^bitrev(j): bit i of j contributes psi^(2^(bits - 1 - i)).
@@ -279,8 +281,8 @@ static uint64_t pow64(uint64_t a, uint64_t e, uint64_t p) {
         if (e & 1) r = mul64(r, a, p);
     return r;
 }
-static uint64_t inv64(uint64_t a, uint64_t p) { return pow64(a % p, p - 2, p); }
-static double bal64(uint64_t a, uint64_t p) { return a > p / 2 ? -(double)(p - a) : (double)a; }
+uint64_t f64_inv_mod(uint64_t a, uint64_t p) { return pow64(a % p, p - 2, p); }
+double f64_balanced(uint64_t a, uint64_t p) { return a > p / 2 ? -(double)(p - a) : (double)a; }
 
 // Largest doubled coefficient against the primes' product.  Limbs are at most L = (b/2 + 4)(b + 1),
 // but for the first two of a range of 16, which enter with the range carry added: the first's
@@ -321,13 +323,13 @@ F64Crt make_f64_crt(uint32_t n, uint32_t b, int K) {
         c.p[k] = (double)p;
         c.pinv[k] = 1.0 / (double)p;
         // n - 3 of the transform's n - 1 levels are run and undone: 2^(n-3) comes out of the inverse
-        const uint64_t s = inv64((uint64_t)1 << (n - 3), p);
-        c.s[0][k] = bal64(s, p);
-        c.s[1][k] = bal64(mul64(s, 2, p), p);
+        const uint64_t s = f64_inv_mod((uint64_t)1 << (n - 3), p);
+        c.s[0][k] = f64_balanced(s, p);
+        c.s[1][k] = f64_balanced(mul64(s, 2, p), p);
     }
-    c.i12 = bal64(inv64(F64_P[0], F64_P[1]), F64_P[1]);
-    c.i13 = bal64(inv64(F64_P[0], F64_P[2]), F64_P[2]);
-    c.i23 = bal64(inv64(F64_P[1], F64_P[2]), F64_P[2]);
+    c.i12 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[1]), F64_P[1]);
+    c.i13 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[2]), F64_P[2]);
+    c.i23 = f64_balanced(f64_inv_mod(F64_P[1], F64_P[2]), F64_P[2]);
     auto split = [&](__int128 x, int pieces, double *w, uint32_t *wl) {
         for (int i = 0; i < pieces; ++i) {
             __int128 r = x;
@@ -353,21 +355,29 @@ F64Crt make_f64_crt(uint32_t n, uint32_t b, int K) {
     return c;
 }
 
-int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
+static int build_twiddles(const uint64_t *primes, const uint32_t *gen, int K, int bits, double *tw, hipStream_t stream) {
     F64TwArgs A;
     memset(&A, 0, sizeof(A));
     A.tw = tw;
-    A.words = (uint32_t)f64_tw_words(n);
-    A.bits = (int)n - 1;
-    for (int k = 0; k < F64_PRIMES; ++k) {
-        const uint64_t p = F64_P[k];
+    A.words = 1u << (bits - 2);
+    A.bits = bits;
+    for (int k = 0; k < K; ++k) {
+        const uint64_t p = primes[k];
         A.p[k] = (double)p;
         A.pinv[k] = 1.0 / (double)p;
-        uint64_t w = pow64(F64_G[k], (p - 1) >> n, p);  // a primitive 2M-th root, M = 2^(n-1)
-        for (int i = 0; i < A.bits; ++i, w = mul64(w, w, p)) A.pw[k][i] = bal64(w, p);
+        uint64_t w = pow64(gen[k], (p - 1) >> (bits + 1), p);  // a primitive 2M-th root, M = 2^bits
+        for (int i = 0; i < A.bits; ++i, w = mul64(w, w, p)) A.pw[k][i] = f64_balanced(w, p);
     }
-    hipLaunchKernelGGL(k64_twiddles, dim3((A.words + 255) / 256, F64_PRIMES, 1), dim3(256), 0, stream, A);
+    hipLaunchKernelGGL(k64_twiddles, dim3((A.words + 255) / 256, K, 1), dim3(256), 0, stream, A);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
+    return build_twiddles(F64_P, F64_G, F64_PRIMES, (int)n - 1, tw, stream);
+}
+
+int f64q_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
+    return build_twiddles(F64Q_P, F64Q_G, F64Q_PRIMES, (int)n - 2, tw, stream);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -399,6 +409,9 @@ F64Shape f64_shape(uint32_t n) {
 }
 
 std::string f64_str(uint32_t n, int K, const F64Shape &S) {
+    if (S.quad)
+        return "squares in doubles (limbs of four digits, 5 45-bit primes, cols 2^" + std::to_string(S.a) + " x rows 2^" +
+               std::to_string((int)n - 2 - S.a) + ")";
     std::string s = "squares in doubles (limbs of two digits, " + (K ? std::to_string(K) : std::string("2 or 3")) + " 49-bit primes, ";
     if (S.whole) return s + "a prime's 2^" + std::to_string(n - 1) + " limbs in one workgroup)";
     return s + "cols 2^" + std::to_string(S.a) + " x rows 2^" + std::to_string((int)n - 1 - S.a) + ")";
@@ -461,12 +474,14 @@ static dim3 f64_grid(F64Args &A, uint32_t per) {
 }
 
 void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream) {
+    if (S.quad) return f64q_launch_fwd(A, S, stream);
     const unsigned nb = 1u << (A.tn - S.a - 4), T = 16u << (S.a - F64_COL_E);
     const dim3 grid = f64_grid(A, S.split ? 3 * nb : nb);
     hipLaunchKernelGGL(fwd_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A, S.split);
 }
 
 void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) {
+    if (S.quad) return f64q_launch_mid(A, S, mode, stream);
     const int L = S.whole ? A.tn : A.tn - S.a;
     if (A.mixed) {
         const F64Fn f = mode == F64_SQUARE ? k64_whole_mixed<F64_SQUARE> : mode == F64_MUL ? k64_whole_mixed<F64_MUL>
@@ -488,6 +503,7 @@ void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) 
 }
 
 void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
+    if (S.quad) return f64q_launch_inv(A, S, stream);
     if (S.whole) {
         const dim3 grid = f64_grid(A, (1u << A.tn) / F64_NORM_RANGE);
         hipLaunchKernelGGL(k64_norm, grid, dim3(F64_NORM_T), 0, stream, A);
@@ -518,6 +534,7 @@ void f64_set_lds_attributes() {
             set((const void *)fwd_fn(a));
             set((const void *)inv_fn(a));
         }
+        f64q_set_lds_attributes();
         for (int a = F64_COL_MIN; a <= F64_SPLIT_MAX; ++a) {
             set((const void *)split_fn<2>(a));
             set((const void *)split_fn<3>(a));

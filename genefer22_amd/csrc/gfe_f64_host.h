@@ -7,16 +7,17 @@
 
 #include <string>
 
-#include "gfe_f64.h"
+#include "gfe_f64q.h"
 
 namespace gfe {
 
 // Shape of the passes at one n.  whole: a prime's transform in one workgroup and the normalisation
 // after it; else three passes over 2^a rows of 2^(n-1-a) limbs, the forward column pass with one prime
 // per workgroup (split) instead of all.  few: one candidate's work is too little for the chip, so its
-// passes take fewer residues per thread.
+// passes take fewer residues per thread.  quad: limbs of four digits (gfe_f64q.h), three passes over
+// 2^(n-2) of them.
 struct F64Shape {
-    int whole = 0, a = 0, split = 0, few = 0;
+    int whole = 0, a = 0, split = 0, few = 0, quad = 0;
 };
 
 // Primes the transform needs for (b, n): 2 or 3, or 0 where it is not exact (or out of range).
@@ -29,6 +30,16 @@ F64Crt make_f64_crt(uint32_t n, uint32_t b, int K);
 // Table words of one prime: entries psi^bitrev(j), j < M / 4 (those of a smaller n are its first ones).
 inline size_t f64_tw_words(uint32_t n) { return ((size_t)1 << n) / 8; }
 int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream);
+uint64_t f64_inv_mod(uint64_t a, uint64_t p);
+double f64_balanced(uint64_t a, uint64_t p);  // in (-p/2, p/2]
+
+// Limbs of four digits, for one candidate: where they are exact and pay, constants and tables.
+bool f64q_ok(uint32_t b, uint32_t n);
+void make_f64q_crt(uint32_t n, uint32_t b, F64QCrt *out);
+inline size_t f64q_crt_bytes() { return sizeof(F64QCrt); }
+inline size_t f64q_tw_words(uint32_t n) { return ((size_t)1 << n) / 16; }
+int f64q_build_twiddles(uint32_t n, double *tw, hipStream_t stream);
+F64Shape f64q_shape(uint32_t n);
 
 // Slot s of a launch: registers at regs + s reg_stride (2^n digits each), residues at
 // ws / zp + s ws_stride, range carries at slots + s slot_stride, constants crt[s].  One candidate is slot
@@ -40,7 +51,7 @@ struct F64Args {
     const double *zp;       // [K][M] multiplicand
     const double *tw;       // [3][tws] twiddles
     int4 *slots;            // M / 16 range carries
-    const F64Crt *crt;
+    const void *crt;        // F64Crt[nslots], or F64QCrt
     const uint8_t *active, *dupf, *mulf;  // per slot, or null (all, dup, none)
     long long reg_stride, ws_stride, slot_stride;
     uint32_t src_reg, tws, nslots;
@@ -58,5 +69,11 @@ void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream);
 // Adds the pending range carries of register 0 and balances it.
 void f64_launch_flush(const F64Args &A, hipStream_t stream);
 void f64_set_lds_attributes();
+// The same for limbs of four digits (called by the above where S.quad).
+void f64q_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream);
+void f64q_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream);
+void f64q_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream);
+void f64q_launch_flush(const F64Args &A, uint32_t b, hipStream_t stream);
+void f64q_set_lds_attributes();
 
 }  // namespace gfe

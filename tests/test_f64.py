@@ -173,3 +173,109 @@ def test_rule_covers_the_range_in_use():
             assert bound(b, n, 2) or (b >= 2**17 and bound(b, n, 3)), (b, n)
     for n, b in ((21, 1148), (22, 1622), (23, 2292)):  # the first base covered
         assert bound(b, n, 2) and not bound(b - 2, n, 2)
+
+
+# Limbs of four digits over five 45.5-bit primes (gfe_f64q.h)
+Q = [49757816881153, 49757632331777, 49757078683649, 49756457926657, 49756323708929]
+QPROD = Q[0] * Q[1] * Q[2] * Q[3] * Q[4]
+
+
+def qbound(b, n):
+    """The host's rule restated: the largest doubled coefficient, or None where (b, n) is refused."""
+    if not 20 <= n <= 23 or b < 2**20 or b * b > 1.5 * 2**52:
+        return None
+    M, up = 2 ** (n - 2), (b + 1) * (b * b + 1)
+    half = Fraction(b, 2)
+    L, g = (half + 4) * up, min(M, half) - 4
+    X = 2 * (M // 16) * (((Fraction(106, 100) * b + g + 8) * up) ** 2 + (L + g) ** 2 + 14 * L * L)
+    return X if 10 * X < 3 * QPROD and X / b**8 + 4 < g else None
+
+
+def qedges(n):
+    """Smallest and largest base of the rule at n."""
+    lo, hi = 2**20 - 1, 2**23
+    while hi - lo > 1:
+        m = (lo + hi) // 2
+        lo, hi = (lo, m) if qbound(m, n) else (m, hi)
+    lo2, hi2 = 2**23, 2**27
+    while hi2 - lo2 > 1:
+        m = (lo2 + hi2) // 2
+        lo2, hi2 = (m, hi2) if qbound(m, n) else (lo2, m)
+    return hi, lo2
+
+
+def base_pieces(x, b, count):
+    out = []
+    for _ in range(count):
+        r = x % b
+        if r > b // 2:
+            r -= b
+        out.append(r)
+        x = (x - r) // b
+    return out
+
+
+def qpieces(x, b, n, dup, rng):
+    """f64q_crt_pieces on raw residues of any representative up to 18 p; every sum has to be exact."""
+    v = []
+    for k, p in enumerate(Q):
+        pinv, s = 1.0 / p, pow(pow(2, n - 4, p), -1, p)
+        raw = float((x // (2 if dup else 1)) * pow(s, -1, p) % p + p * rng.randrange(-18, 18))
+        t = mul(raw, bal(s * (2 if dup else 1), p), p, pinv)
+        for j in range(k):
+            t = mul(t - v[j], bal(pow(Q[j], -1, p), p), p, pinv)
+        v.append(t)
+    hi = [rint(t * 2.0**-23) for t in v]
+    lo = [fma(-h, 2.0**23, t) for h, t in zip(hi, v)]
+    prod, w, u = 1, [], []
+    for j in range(4):
+        prod *= Q[j]
+        w.append(base_pieces(prod, b, 9))
+        u.append(base_pieces(prod << 23, b, 9))
+        assert not any(w[j][2 * j + 3:]) and (j >= 2 or not any(u[j][2 * j + 4:]))  # what the kernel leaves out
+    g, S = [], v[0]
+    for i in range(9):
+        exact = int(S) + sum(int(lo[j + 1]) * w[j][i] + int(hi[j + 1]) * u[j][i] for j in range(4))
+        for j in range(4):
+            S = fma(lo[j + 1], float(w[j][i]), S)
+            S = fma(hi[j + 1], float(u[j][i]), S)
+        assert int(S) == exact
+        q = rint(S * (1.0 / b))
+        g.append(int(fma(-q, float(b), S)))
+        assert g[-1] == exact - int(q) * b
+        S = q
+    return g
+
+
+def test_four_digit_primes():
+    for p, gen in zip(Q, (7, 5, 3, 5, 3)):
+        assert p < 2**45.5 and (p - 1) % 2**24 == 0
+        assert pow(gen, p - 1, p) == 1 and pow(gen, (p - 1) // 2, p) == p - 1
+        assert all(p % d for d in range(3, 100000, 2))
+
+
+def test_four_digit_product_is_bounded():
+    """|r| <= 0.52 + 0.0085 B by a constant, 0.5 + 0.0167 B B' (and 0.02 of slack) by a residue."""
+    rng = random.Random(5)
+    for i in range(6000):
+        p = Q[i % 5]
+        B, C = rng.choice([(1.0, 0.5), (14.0, 0.5), (146.0, 0.5), (14.0, 14.0), (28.0, 14.0), (4.0, 8.0)])
+        a, w = (float(rng.choice([-1, 1]) * (int(x * p) - rng.randrange(1000 if i % 2 else int(x * p)))) for x in (B, C))
+        r = mul(a, w, p, 1.0 / p)
+        assert (int(r) - int(a) * int(w)) % p == 0
+        assert abs(r) <= (0.52 + 0.0085 * abs(a) / p if C == 0.5 else 0.52 + 0.0167 * abs(a * w) / p / p) * p
+
+
+@pytest.mark.parametrize("n", range(20, 24))
+def test_four_digit_pieces_at_the_rules_edges(n):
+    for b in (*qedges(n), 2**23 + 2):
+        X, rng = int(qbound(b, n)), random.Random(b)
+        assert b * b * 1.07 < 2**53 and 1.07 * b * b < 146 * min(Q)
+        xs = [0, 1, -1, X, -X, b**8, -b**8 // 2] + [rng.randrange(-X, X) for _ in range(150)]
+        xs += [rng.choice([-1, 1]) * rng.randrange(1 << rng.randrange(1, X.bit_length() - 1)) for _ in range(150)]
+        for x in xs:
+            for dup in (0, 1):
+                x2 = x - (x & 1) if dup else x
+                g = qpieces(x2, b, n, dup, rng)
+                assert sum(gi * b**i for i, gi in enumerate(g)) == x2
+                assert all(abs(gi) <= 0.55 * b for gi in g)

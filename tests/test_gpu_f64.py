@@ -169,3 +169,48 @@ def test_noalloc_digits_equal_the_engines(gfe, b, n):
                 assert np.array_equal(got, t.get_digits()), count
     finally:
         hip.h.hipFree(buf)
+
+
+@pytest.mark.parametrize("n", range(19, 24))
+def test_four_digit_limbs_equal_the_integer_passes(gfe, n):
+    """At the edges of the rule of four-digit limbs and past them: extreme and random digits, products,
+    copies and a change of base and back (to two-digit limbs between), against the integer passes."""
+    from test_f64 import qbound, qedges
+    lo, hi = qedges(max(n, 20))
+    for b in (lo + (lo & 1), hi - (hi & 1), lo - 2 - (lo & 1), hi + 2 - (hi & 1)):
+        t, u = gfe.Transform(b, n), gfe.Transform(b, n)
+        u.set_plan(u.get_plan())
+        assert ("four digits" in t.info()) == (qbound(b, n) is not None) and "in doubles" not in u.info()
+        rs, N, h = np.random.RandomState(n), 1 << n, b // 2 + 4
+        d = rs.randint(-((b - 1) // 2), b // 2 + 1, N).astype(np.int32)
+        for x in (np.full(N, -h, np.int32), np.where(np.arange(N) % 2 == 0, h, -h).astype(np.int32), d):
+            for e in (t, u):
+                e.set_digits(x)
+                for dup in (1, 0, 1):
+                    e.square_dup(dup)
+            got = t.get_digits()
+            assert np.abs(got.astype(np.int64)).max() <= h
+            assert np.array_equal(got, u.get_digits()), (b, n)
+        for e in (t, u):
+            e.set_digits(d, 1)
+            e.init_multiplicand(1)
+            e.square_dup(False)
+            e.mul()
+            e.copy(2, 0)                    # carries pending
+            e.init_multiplicand(0)
+            e.square_dup(True)
+            e.mul()
+            e.square_mul(7)
+        assert np.array_equal(t.get_digits(0), u.get_digits(0)) and np.array_equal(t.get_digits(2), u.get_digits(2))
+        t.rebase(hi + 2 + (hi & 1) if b > 2**25 else lo - 4 - (lo & 1))
+        assert "two digits" in t.info()
+        t.set(3)
+        t.square_dup(True)
+        t.rebase(b)
+        u.copy(0, 1)
+        t.set_digits(d, 0)
+        for e in (t, u):
+            e.square_dup(True)
+        assert np.array_equal(t.get_digits(), u.get_digits())
+        t.close()
+        u.close()
