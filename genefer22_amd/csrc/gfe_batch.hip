@@ -240,6 +240,30 @@ __global__ void __launch_bounds__(256) kb_set(BArgs A) {
     if (i < N) A.regs[s * A.reg_stride + A.dst_reg * N + i] = (i == 0) ? A.value : 0;
 }
 
+// A slot taken by a candidate: its constants, and r0 = r1 = 1.  They come as arguments of the one launch:
+// four uploads and two kb_set launches over every slot's workgroups took 30-37 us a candidate.
+struct SlotInit {
+    SlotInfo si;
+    CrtConst c;
+    F64Crt d;
+    SlotInfo *slots;
+    CrtConst *crt;
+    F64Crt *crt64;
+    int4 *r0, *r1;
+    uint32_t n4;
+    int s;
+};
+__global__ void __launch_bounds__(256) kb_take_slot(SlotInit A) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= A.n4) return;
+    A.r0[i] = A.r1[i] = make_int4(i == 0, 0, 0, 0);
+    if (i == 0) {
+        A.slots[A.s] = A.si;
+        A.crt[A.s] = A.c;
+        A.crt64[A.s] = A.d;
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Host side
 
@@ -332,8 +356,6 @@ struct Batch {
     // Pinned mirrors of the per-slot tables.  Entry s is written only by submit() into a free
     // slot; the previous occupant's program ended with a read-back, whose completion the host
     // waited for, so no upload of entry s is still pending then.
-    SlotInfo *slot_host = nullptr;
-    CrtConst *crt_host = nullptr;
     int32_t *readback = nullptr;                      // pinned N int32 (synchronous reads)
     // Asynchronous result read-backs: pinned N-digit buffers, each with a completion event,
     // processed in stream order.
@@ -394,7 +416,7 @@ struct Batch {
     bool f64 = false, carry64 = false;
     F64Shape shape;
     double *tw64 = nullptr;
-    F64Crt *crt64 = nullptr, *crt64_host = nullptr;
+    F64Crt *crt64 = nullptr;
     int int_tables();
     bool mode64() const;
     int use_mode(bool m);
@@ -569,7 +591,6 @@ Batch::~Batch() {
     (void)hipFree(crt); (void)hipFree(slots_dev); (void)hipFree(act_dev); (void)hipFree(dup_dev);
     (void)hipFree(mul_dev);
     (void)hipFree(tw64); (void)hipFree(crt64);
-    if (crt64_host) (void)hipHostFree(crt64_host);
     for (int i = 0; i < NSTAGE; ++i) {
         if (stage[i]) (void)hipHostFree(stage[i]);
         if (stage_ev[i]) (void)hipEventDestroy(stage_ev[i]);
@@ -580,8 +601,6 @@ Batch::~Batch() {
     }
     for (int i = 0; i < NBLK; ++i)
         if (blk_ev[i]) (void)hipEventDestroy(blk_ev[i]);
-    if (slot_host) (void)hipHostFree(slot_host);
-    if (crt_host) (void)hipHostFree(crt_host);
     if (readback) (void)hipHostFree(readback);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -635,10 +654,6 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
     }
     for (int i = 0; i < NBLK; ++i)
         if (hipEventCreateWithFlags(&blk_ev[i], hipEventDisableTiming) != hipSuccess) return set_error(GFE_EHIP, "event");
-    if (hipHostMalloc((void **)&crt64_host, (size_t)cap * sizeof(F64Crt)) != hipSuccess ||
-        hipHostMalloc((void **)&slot_host, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
-        hipHostMalloc((void **)&crt_host, (size_t)cap * sizeof(CrtConst)) != hipSuccess)
-        return set_error(GFE_ENOMEM, "pinned");
     if (hipHostMalloc((void **)&readback, NA * 4) != hipSuccess) return set_error(GFE_ENOMEM, "pinned");
     if (hipEventCreate(&ev0) != hipSuccess || hipEventCreate(&ev1) != hipSuccess) return set_error(GFE_EHIP, "event");
     for (int k = 0; k < 3; ++k) {
@@ -1085,26 +1100,15 @@ int Batch::submit(uint32_t b, uint64_t iters, uint64_t tag, int32_t *slot_out, u
     }
     mpz_clear(E);
     // slot table and CRT constants; r0 = 1, r1 = 1 (prp: set(1); copy(1, 0))
-    SlotInfo &si = slot_host[s];
-    si.b = b; si.rns = S.rns; si.is32 = S.is32; si.rounds = carry_rounds(b, S.n); si.n = (int32_t)S.n;
-    crt_host[s] = make_crt(S.rns, S.is32, S.n, b);
+    SlotInit A;
+    A.si.b = b; A.si.rns = S.rns; A.si.is32 = S.is32; A.si.rounds = carry_rounds(b, S.n); A.si.n = (int32_t)S.n;
+    A.c = make_crt(S.rns, S.is32, S.n, b);
+    A.d = make_f64_crt(S.n, b, f64_primes(b, S.n));
+    A.slots = slots_dev; A.crt = crt; A.crt64 = crt64; A.s = s;
+    A.r0 = reinterpret_cast<int4 *>(reg(s, 0)); A.r1 = reinterpret_cast<int4 *>(reg(s, 1));
+    A.n4 = (uint32_t)(slot_N(s) / 4);
     zl = std::max(zl, (uint32_t)s + 1);
-    int rc = check_hip(hipMemcpyAsync(slots_dev + s, &si, sizeof(si), hipMemcpyHostToDevice, stream), "slot");
-    if (rc == GFE_OK) rc = check_hip(hipMemcpyAsync(crt + s, crt_host + s, sizeof(CrtConst), hipMemcpyHostToDevice, stream), "crt");
-    crt64_host[s] = make_f64_crt(S.n, b, f64_primes(b, S.n));
-    if (rc == GFE_OK) rc = check_hip(hipMemcpyAsync(crt64 + s, crt64_host + s, sizeof(F64Crt), hipMemcpyHostToDevice, stream), "crt");
-    if (rc != GFE_OK) return rc;
-    std::vector<uint8_t> one(cap, 0);
-    one[s] = 1;
-    uint8_t *st = stage_acquire();
-    memcpy(st, one.data(), cap);
-    rc = check_hip(hipMemcpyAsync(act_dev, st, cap, hipMemcpyHostToDevice, stream), "flags");
-    stage_release();
-    if (rc != GFE_OK) return rc;
-    with_n(S.n, [&]() {
-        op_set(act_dev, 0, 1);
-        op_set(act_dev, 1, 1);
-    });
+    hipLaunchKernelGGL(kb_take_slot, dim3((A.n4 + 255) / 256), dim3(256), 0, stream, A);
     if (slot_out) *slot_out = s;
     return check("submit");
 }
