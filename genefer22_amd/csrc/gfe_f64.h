@@ -46,7 +46,7 @@ constexpr int F64_PRIMES = 3;
 constexpr uint64_t F64_P[F64_PRIMES] = {562949869535233ull, 562949517213697ull, 562949282332673ull};
 constexpr uint32_t F64_G[F64_PRIMES] = {5, 10, 3};
 constexpr int F64_NG = 16;       // columns per workgroup: one 16-lane DPP row of limbs
-constexpr int F64_ROW_MIN = 6, F64_ROW_MAX = 14, F64_ROW8_MAX = 13, F64_COL_MIN = 5, F64_COL_MAX = 8,
+constexpr int F64_ROW_MIN = 8, F64_ROW_MAX = 14, F64_COL_MIN = 5, F64_COL_MAX = 8,
               F64_SPLIT_MAX = 7;
 constexpr int F64_WHOLE_MIN = 11, F64_WHOLE_MAX = 12;           // log2 limbs of a one-workgroup transform
 constexpr uint32_t F64_NORM_T = 64, F64_NORM_PER = 1, F64_NORM_RANGE = F64_NORM_T * F64_NORM_PER;  // its normalisation
@@ -242,7 +242,13 @@ struct F64Geo {
 
 enum { F64_SQUARE = 0, F64_MUL = 1, F64_FWD = 2, F64_EITHER = 3 };
 
-__host__ __device__ constexpr uint32_t f64_row_words(int logg, int loge) { return (1u << logg) + (1u << (logg - loge)); }
+// 8 residues a thread, 16 from 2^13 on (where 8 would be 1024 threads and gain nothing).  Twice the waves
+// outweigh one exchange more: us per round or squaring with 16 and with 8 a thread, 8 slots of n = 12
+// 9.1 and 7.7, 301 19.7 and 19.0, 1024 47.4 and 45.5; n = 13 64 slots 12.9 and 12.0, 301 32.9 and
+// 32.3; n = 15 64 slots 38.0 and 35.7, 512 226 and 222; 7 of n = 18 41.2 and 39.1; one candidate of
+// n = 18 19.1 and 16.4.
+__host__ __device__ constexpr int f64_row_loge(int logg) { return logg <= 12 ? 3 : 4; }
+__host__ __device__ constexpr uint32_t f64_row_words(int logg) { return (1u << logg) + (1u << (logg - f64_row_loge(logg))); }
 
 // Between the LDS writes of a chunk and the next chunk's reads, YL the larger of their strides' logs: up
 // to 6 the elements of a wave's 64 threads are the same run of residues in both chunks, and a

@@ -70,12 +70,13 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_fwd(F64Args 
     }
 }
 
-constexpr int f64_row_threads(int logg, int loge) { return logg - loge > 8 ? 1 << (logg - loge) : 256; }
+constexpr int f64_row_threads(int logg) { return logg > 11 ? 1 << (logg - f64_row_loge(logg)) : 256; }
 
 // 3 2^a / ng workgroups a slot.
-template <int LOGG, int LOGE, int MODE>
-__global__ void __launch_bounds__(f64_row_threads(LOGG, LOGE)) k64_row(F64Args A) {
+template <int LOGG, int MODE>
+__global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
     extern __shared__ double lds64[];
+    constexpr int LOGE = f64_row_loge(LOGG);
     constexpr uint32_t SPR = 1u << (LOGG - LOGE);
     const uint32_t nb = (1u << A.a) / (uint32_t)A.ng;
     const F64Job J = f64_job(A, 3 * nb);
@@ -94,15 +95,15 @@ __global__ void __launch_bounds__(f64_row_threads(LOGG, LOGE)) k64_row(F64Args A
         for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = md.red(x[rr]);
     };
     f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
-                                   lds64 + q * f64_row_words(LOGG, LOGE),
-                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
+                                            lds64 + q * f64_row_words(LOGG),
+                                            MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
 // A prime's whole transform, from the digits, in one workgroup; thread s of
-// 2^(LOGG - LOGE).
-template <int LOGG, int LOGE, int MODE>
+// 2^(LOGG - f64_row_loge(LOGG)).
+template <int LOGG, int MODE>
 __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J, int k, uint32_t s, double *lds) {
-    constexpr int E = 1 << LOGE;
+    constexpr int LOGE = f64_row_loge(LOGG), E = 1 << LOGE;
     const F64CrtP c = J.c;
     const F64Mod md{c->p[k], c->pinv[k]};
     const double bd = c->bd;
@@ -130,26 +131,26 @@ __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J
         for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
     };
     f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
-                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
+                                            MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
 // 3 workgroups a slot.
-template <int LOGG, int LOGE, int MODE>
-__global__ void __launch_bounds__(1 << (LOGG - LOGE)) k64_whole(F64Args A) {
+template <int LOGG, int MODE>
+__global__ void __launch_bounds__(1 << (LOGG - f64_row_loge(LOGG))) k64_whole(F64Args A) {
     extern __shared__ double lds64[];
     const F64Job J = f64_job(A, 3);
-    if (J.run && (int)J.w < J.K) f64_whole_body<LOGG, LOGE, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    if (J.run && (int)J.w < J.K) f64_whole_body<LOGG, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
 }
 
-// A mixed batch: each workgroup at its slot's n, 12 or 13 (of the 256 threads n = 12 takes two whole
+// A mixed batch: each workgroup at its slot's n, 12 or 13 (of the 512 threads n = 12 takes four whole
 // waves; the others end before any barrier).
 template <int MODE>
-__global__ void __launch_bounds__(256) k64_whole_mixed(F64Args A) {
+__global__ void __launch_bounds__(512) k64_whole_mixed(F64Args A) {
     extern __shared__ double lds64[];
     const F64Job J = f64_job(A, 3);
     if (!J.run || (int)J.w >= J.K) return;
-    if (J.c->n == 13) f64_whole_body<12, 4, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
-    else if (threadIdx.x < 128) f64_whole_body<11, 4, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    if (J.c->n == 13) f64_whole_body<12, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+    else if (threadIdx.x < 256) f64_whole_body<11, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
 }
 
 template <int K, int LOGG>
@@ -390,8 +391,8 @@ int f64q_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
 // in batches 100 candidates of 2^13 limbs 32.8 against 31.6, 512 of 2^14 230 against 228).
 // With three passes, up to 2^19 limbs each is bound by latency: a wave issues one instruction in four
 // clocks, and with 16 residues a thread the row pass of 2^14 limbs was 5.2 us in a few waves.  So the
-// shapes that win there have many workgroups and short threads (`few`: 8 residues per thread in the
-// rows, the primes side by side in the inverse column pass; 2^14 limbs 14.7 -> 11.0, 2^16 16.5 ->
+// shapes that win there have many workgroups and short threads (8 residues per thread in the rows, and
+// `few`: the primes side by side in the inverse column pass; 2^14 limbs 14.7 -> 11.0, 2^16 16.5 ->
 // 12.9, 2^17 19.1 -> 16.4, 2^18 23.4 -> 21.1, 2^19 36.3 -> 34.0) and short columns (2^14 limbs: 11.4
 // with 2^5-point columns, 11.9 with 2^6; 2^16: 13.0 and 13.6; 2^17 16.7 and 15.9).  From 2^20 limbs
 // the passes are bound by memory and fp64 issue and longer columns pay, the digits then being read
@@ -435,28 +436,22 @@ static F64Fn split_fn(int a) {
     if constexpr (LOGG > F64_SPLIT_MAX) return nullptr;
     else return a == LOGG ? k64_col_inv_split<K, LOGG> : split_fn<K, LOGG + 1>(a);
 }
-template <int MODE, int LOGE, int LOGG = F64_ROW_MIN>
+template <int MODE, int LOGG = F64_ROW_MIN>
 static F64Fn row_fn(int logg) {
-    if constexpr (LOGG > (LOGE == 3 ? F64_ROW8_MAX : F64_ROW_MAX)) return nullptr;
-    else return logg == LOGG ? k64_row<LOGG, LOGE, MODE> : row_fn<MODE, LOGE, LOGG + 1>(logg);
+    if constexpr (LOGG > F64_ROW_MAX) return nullptr;
+    else return logg == LOGG ? k64_row<LOGG, MODE> : row_fn<MODE, LOGG + 1>(logg);
 }
-template <int MODE, int LOGE, int LOGG = F64_WHOLE_MIN>
+template <int MODE, int LOGG = F64_WHOLE_MIN>
 static F64Fn whole_fn(int logg) {
     if constexpr (LOGG > F64_WHOLE_MAX) return nullptr;
-    else return logg == LOGG ? k64_whole<LOGG, LOGE, MODE> : whole_fn<MODE, LOGE, LOGG + 1>(logg);
+    else return logg == LOGG ? k64_whole<LOGG, MODE> : whole_fn<MODE, LOGG + 1>(logg);
 }
-template <int MODE>
-static F64Fn mid_mode(bool whole, int loge, int logg) {
-    if (loge == 4) return whole ? whole_fn<MODE, 4>(logg) : row_fn<MODE, 4>(logg);
-    if constexpr (MODE == F64_EITHER) return nullptr;  // one candidate's passes have no per-slot kind
-    else return whole ? whole_fn<MODE, 3>(logg) : row_fn<MODE, 3>(logg);
-}
-static F64Fn mid_fn(bool whole, int mode, int loge, int logg) {
+static F64Fn mid_fn(bool whole, int mode, int logg) {
     switch (mode) {
-        case F64_SQUARE: return mid_mode<F64_SQUARE>(whole, loge, logg);
-        case F64_MUL: return mid_mode<F64_MUL>(whole, loge, logg);
-        case F64_FWD: return mid_mode<F64_FWD>(whole, loge, logg);
-        default: return mid_mode<F64_EITHER>(whole, loge, logg);
+        case F64_SQUARE: return whole ? whole_fn<F64_SQUARE>(logg) : row_fn<F64_SQUARE>(logg);
+        case F64_MUL: return whole ? whole_fn<F64_MUL>(logg) : row_fn<F64_MUL>(logg);
+        case F64_FWD: return whole ? whole_fn<F64_FWD>(logg) : row_fn<F64_FWD>(logg);
+        default: return whole ? whole_fn<F64_EITHER>(logg) : row_fn<F64_EITHER>(logg);
     }
 }
 
@@ -487,19 +482,19 @@ void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) 
         const F64Fn f = mode == F64_SQUARE ? k64_whole_mixed<F64_SQUARE> : mode == F64_MUL ? k64_whole_mixed<F64_MUL>
                                                                                          : k64_whole_mixed<F64_FWD>;
         const dim3 grid = f64_grid(A, 3);
-        hipLaunchKernelGGL(f, grid, dim3(256), (size_t)8 * f64_row_words(12, 4), stream, A);
+        hipLaunchKernelGGL(f, grid, dim3(512), (size_t)8 * f64_row_words(12), stream, A);
         return;
     }
-    const int loge = A.K && S.few ? 3 : 4;
+    const int loge = f64_row_loge(L);
     if (S.whole) {
         const dim3 grid = f64_grid(A, 3);
-        hipLaunchKernelGGL(mid_fn(true, mode, loge, L), grid, dim3(1u << (L - loge)), (size_t)8 * f64_row_words(L, loge), stream, A);
+        hipLaunchKernelGGL(mid_fn(true, mode, L), grid, dim3(1u << (L - loge)), (size_t)8 * f64_row_words(L), stream, A);
         return;
     }
     A.ng = L - loge >= 6 ? 1 : 64 >> (L - loge);  // rows per workgroup: one wave at least
     const dim3 grid = f64_grid(A, 3 * ((1u << S.a) / A.ng));
-    hipLaunchKernelGGL(mid_fn(false, mode, loge, L), grid, dim3((unsigned)A.ng << (L - loge)),
-                       (size_t)8 * A.ng * f64_row_words(L, loge), stream, A);
+    hipLaunchKernelGGL(mid_fn(false, mode, L), grid, dim3((unsigned)A.ng << (L - loge)),
+                       (size_t)8 * A.ng * f64_row_words(L), stream, A);
 }
 
 void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
@@ -539,11 +534,10 @@ void f64_set_lds_attributes() {
             set((const void *)split_fn<2>(a));
             set((const void *)split_fn<3>(a));
         }
-        for (int m = 0; m < 4; ++m)
-            for (int e = 3; e <= 4; ++e) {
-                for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, e, l));
-                for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, e, l));
-            }
+        for (int m = 0; m < 4; ++m) {
+            for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, l));
+            for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, l));
+        }
         (void)hipGetLastError();
     });
 }

@@ -35,14 +35,11 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64q_col_fwd(F64Args
     }
 }
 
-// 8 residues a thread (n = 22: 25.6 us, 16 26.1; 2^13 of them, 1024 threads, gain nothing: 57.7, 56.9)
-constexpr int f64q_row_loge(int logg) { return logg <= 12 ? 3 : 4; }
-
 // 5 2^a workgroups, one row each.
 template <int LOGG, int MODE>
-__global__ void __launch_bounds__(1 << (LOGG - f64q_row_loge(LOGG))) k64q_row(F64Args A) {
+__global__ void __launch_bounds__(1 << (LOGG - f64_row_loge(LOGG))) k64q_row(F64Args A) {
     extern __shared__ double lds64[];
-    constexpr int LOGE = f64q_row_loge(LOGG);
+    constexpr int LOGE = f64_row_loge(LOGG);
     const F64QCrtP c = (F64QCrtP)A.crt;
     const uint32_t k = blockIdx.x >> A.a, row = blockIdx.x & ((1u << A.a) - 1u);
     const size_t at = ((size_t)k << A.tn) + ((size_t)row << LOGG);
@@ -214,7 +211,7 @@ void f64q_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream) {
 
 void f64q_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream) {
     const int L = A.tn - S.a;
-    hipLaunchKernelGGL(qrow_fn(mode, L), dim3(F64Q_PRIMES << S.a), dim3(1u << (L - f64q_row_loge(L))), (size_t)8 * f64_row_words(L, f64q_row_loge(L)), stream, A);
+    hipLaunchKernelGGL(qrow_fn(mode, L), dim3(F64Q_PRIMES << S.a), dim3(1u << (L - f64_row_loge(L))), (size_t)8 * f64_row_words(L), stream, A);
 }
 
 void f64q_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream) {
