@@ -3,13 +3,14 @@
 
 One JSON line on stdout (progress on stderr):
   * value      : ns per squaring of one candidate at n = 22 (N = 4,194,304 digits), b seeded in
-                 [1e7, 3.5e7] (prime set NTT3 31-bit), residue resident in HBM, W warm-up then K timed
-                 squarings (one step = one squaring = column pass, row pass, column pass, CRT + carry),
-                 timed with HIP events on the engine's stream;
-  * roofline   : the dominant kernel's algorithmic bytes (one read + one write of the rns x N uint32
-                 residues, 8 rns N bytes per launch) over its average launch duration, against 8 TB/s;
+                 [1e7, 3.5e7], residue resident in HBM, W warm-up then K timed
+                 squarings (one step = one squaring = column pass, row pass, column pass with CRT + carry;
+                 exact integers modulo 45-bit primes in float64), timed with HIP events on the
+                 engine's stream;
+  * roofline   : the dominant kernel's algorithmic bytes (one read + one write of the residues)
+                 over its average launch duration, against 8 TB/s;
   * passes     : every pass's algorithmic HBM rate (and the whole squaring's) against 8 TB/s;
-  * valu       : the same kernel's butterfly rate and estimated VALU-slot use (integer-bound path);
+  * valu       : the same kernel's butterfly rate and estimated VALU-slot use;
   * job_n22    : the n = 22 job end to end (config.job_n22): 100,000 PRP squarings with Gerbicz-Li
                  updates every 2000, engine set-up and read-out included, host clock; RES64 against
                  the reference's value at 100,000;
@@ -48,7 +49,8 @@ from genefer22_amd import workloads as W  # noqa: E402
 METRIC = "ns per squaring at n=22; candidates/hour at n=15 batched vs plain, bit-exact"
 HBM_PEAK_GBS = 8000.0
 # VALU issue peak: 256 CUs x 4 SIMDs x 16 lanes at 2.4 GHz, one wave-instruction per CU per clock
-# (integer multiplies, min and add3 issue at this rate on gfx950; 32-bit adds somewhat faster).
+# (integer multiplies, min and add3 and float64 fma, add, multiply and rndne issue at this rate on
+# gfx950; 32-bit adds somewhat faster).
 VALU_PEAK_LANE_INSTR = 256 * 64 * 2.4e9
 
 # Per-launch counters of the dominant kernel for plans profiled with rocprofv3 on MI355X: HBM bytes
@@ -65,6 +67,13 @@ MEASURED = {
 }
 MEASURED[("row", 7, 5, 1, 42)] = {"kernel": "gfe::ks_row_sq<gfe::ModS, 5, 14>", "fetch_mib": 96.8, "write_mib": 32.0,
                                   "valu_instr_per_butterfly": 11.92, "profile": "profiles/n22_limb_fused_kernels.md"}
+# the double-precision transform, by (limbs of 2^l digits, column levels)
+MEASURED[("f64", "row", 2, 8)] = {"kernel": "gfe::k64q_row<12, 0>", "fetch_mib": 62.0, "write_mib": 40.0,
+                                  "traffic": int((62.0 + 40.0) * 2**20), "valu_instr_per_butterfly": 11.41,
+                                  "profile": "profiles/n22_f64_kernels.md"}
+MEASURED[("f64", "col_inv_norm", 2, 8)] = {"kernel": "gfe::k64q_col_inv<8>", "fetch_mib": 40.5, "write_mib": 18.0,
+                                           "traffic": int((40.5 + 18.0) * 2**20), "valu_instr_per_butterfly": 23.62,
+                                           "profile": "profiles/n22_f64_kernels.md"}
 
 
 def measured(kernel: str, plan) -> dict:
@@ -114,7 +123,7 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
     rns = 3 if "NTT3" in plan else 2
     N = 1 << n
     # the double-precision limb transform (what an engine squares with unless a plan is fixed)
-    f64 = re.search(r"in doubles \(.* (\d) 49-bit primes, cols 2\^(\d+)", plan)
+    f64 = re.search(r"in doubles \(limbs of (two|four) digits, (\d) \d\d-bit primes, cols 2\^(\d+)", plan)
     # the transform: rns primes x N residues, or for the two-digit-limb transform 4 primes x N/2 limbs
     tn, tp = (n - 1, 4) if limb else (n, rns)
     words = tp << tn
@@ -122,7 +131,8 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
     ng = t.get_plan()[2]
     if f64:  # as the fused limb plan, residues of 8 bytes, ranges of 16 limbs
         names = ["col_fwd", "row", "col_inv_norm", "norm"]
-        tn, tp = n - 1, int(f64.group(1))
+        log_digits = 1 if f64.group(1) == "two" else 2
+        tn, tp = n - log_digits, int(f64.group(2))
         words, slots = tp << tn, N // 2
         alg = {0: 4 * N + 8 * words + slots, 1: 16 * words, 2: 8 * words + 4 * N + slots, 3: 0}
     elif limb and fused:  # digits (+ range carries) in, residues out | row | residues in, digits + carries out
@@ -143,15 +153,20 @@ def bench_n22(G, steps: int, warmup: int, plan_arg: str | None, tune: bool):
                           "GBps": round(sq_bytes / (ms / steps * 1e-3) / 1e9, 1),
                           "frac": round(sq_bytes / (ms / steps * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)}
     # butterflies of the dominant pass (row: (n - a) levels fwd + inv, N/2 per level per prime)
-    a = int(f64.group(2)) if f64 else t.get_plan()[0]
+    a = int(f64.group(3)) if f64 else t.get_plan()[0]
     row_levels = tn - a - (2 if f64 else 0)  # the double-precision rows stop two levels early
     levels = {0: a, 1: 2 * row_levels, 2: a}.get(dom, 0)
     bfly = tp * levels * ((1 << tn) // 2)
     bfly_rate = bfly / (km[dom] * 1e-3) if levels else 0.0
-    meas = MEASURED.get(("f64", names[dom], a), {}) if f64 else measured(names[dom], t.get_plan())
+    meas = MEASURED.get(("f64", names[dom], log_digits, a), {}) if f64 else measured(names[dom], t.get_plan())
     ipb = meas.get("valu_instr_per_butterfly")
+    if f64:
+        workload = f"2^{tn} limbs of {f64.group(1)} digits, {tp} primes, exact in float64"
+    else:
+        workload = "2^21 limbs of two digits, four 31-bit primes" if limb else "NTT3, 31-bit primes"
     res = {
-        "b": b, "plan": plan, "plan_tuple": list(t.get_plan()), "limb": limb, "ms_per_step": ms / steps, "ns_per_squaring": ms / steps * 1e6,
+        "b": b, "workload": workload, "dtype": "f64" if f64 else "u32", "plan": plan, "plan_tuple": list(t.get_plan()),
+        "ms_per_step": ms / steps, "ns_per_squaring": ms / steps * 1e6,
         "kernel_us": {names[i]: round(km[i] * 1e3, 2) for i in range(4)},
         "passes": passes,
         "roofline": {
@@ -529,11 +544,10 @@ def main():
         "higher_is_better": False,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "u32",
+        "dtype": res["dtype"],
         "data": "synthetic (seeded b; residue 2^k mod b^N+1 from set(1) and a fixed dup pattern)",
         "config": {
-            "workload": "one candidate b^(2^22)+1, N=4194304, b seeded in [1e7,3.5e7] ("
-                        + ("2^21 limbs of two digits, four 31-bit primes" if res["limb"] else "NTT3, 31-bit primes") + ")",
+            "workload": "one candidate b^(2^22)+1, N=4194304, b seeded in [1e7,3.5e7] (" + res["workload"] + ")",
             "n": 22, "b": res["b"], "plan": res["plan"], "plan_tuple": res["plan_tuple"], "kernel_us": res["kernel_us"],
             "job_n22": job, "batched_n15": batched, "serving": serving, "serving_light": serving_light, "parity": parity,
             "small_configs": small,

@@ -3,13 +3,14 @@
 // Replaces the reference's engines<RNS, is32> / transformGPUs<RNS, is32> (src/transformGPU.h:
 // 210-1195) and create_ocl (src/transform_ocl.cpp:20-52).  Device state of one engine:
 //   regs  : num_regs x N int32 digits (register 0 = r0), balanced, |d| <= b/2 + 4
-//   ws    : rns x N uint32 residues (transform-domain work space of one squaring)
-//   zp    : rns x N uint32 residues (multiplicand, transform domain)
-//   carry : N / 8 int64: workgroup carries of the normalisation, or segment carries of the fused
-//           inverse column pass
-//   tw    : rns x N uint32 twiddles (Montgomery form)
-// One squaring = k_col_fwd, k_row, k_col_inv, k_norm, k_carry_wg on the engine's stream, or with
-// a fused plan k_col_fwd_all, k_row, k_col_inv_norm, k_fold.
+//   ws    : 12 N bytes of residues (transform-domain work space of one squaring)
+//   zp    : 12 N bytes of residues (multiplicand, transform domain)
+//   carry : N bytes: range carries, workgroup carries of the normalisation, or segment carries of the
+//           fused inverse column pass
+//   tw64, twq : twiddles of the double-precision transform, limbs of two or four digits
+//   tw    : rns x N uint32 twiddles (Montgomery form) of the integer passes
+// One squaring is the double-precision transform's passes (gfe_f64.hip, gfe_f64q.hip); with a plan set
+// k_col_fwd, k_row, k_col_inv, k_norm, k_carry_wg, or fused k_col_fwd_all, k_row, k_col_inv_norm, k_fold.
 
 #include "gfe_engine.h"
 #include "gfe_limb.h"
@@ -411,10 +412,11 @@ static size_t work_bytes(size_t N) { return 4 * (size_t)F64_PRIMES * N; }
 
 // Device bytes of an engine: registers, work space and multiplicand, the twiddles of rns primes, the
 // carry buffer (N bytes), with limb_tables the limb transform's twiddles (4 x N/2 words), and the
-// double-precision transform's (3 x N/8 doubles).
+// double-precision transform's (3 x N/8 doubles, and 5 x N/16 where limbs of four digits may be used:
+// a rebase keeps both).
 size_t engine_bytes(int rns, size_t N, uint32_t num_regs, bool limb_tables) {
     return (size_t)num_regs * N * 4 + 2 * work_bytes(N) + (size_t)rns * N * 4 + N + (limb_tables ? 8 * N : 0) +
-           (size_t)F64_PRIMES * N;  // four-digit limbs: less
+           (size_t)F64_PRIMES * N + (N >> F64Q_MIN_N ? 5 * N / 2 : 0);
 }
 
 // An engine's first plan: the limb transform where it is exact (with the inverse column pass and

@@ -1,9 +1,8 @@
 // gfe_f64.hip -- kernels and host constants of the double-precision limb transform (gfe_f64.h).
 //
 // One squaring is three launches: forward column pass (digits -> residues of every prime), row pass
-// (forward, square, inverse), inverse column pass with the CRT and the carry; or, up to 2^12
-// limbs, two: the whole transform of each prime, then the CRT
-// and the carry.
+// (forward, square, inverse), inverse column pass with the CRT and the carry; or, up to 2^12 limbs,
+// two: the whole transform of each prime, then the CRT and the carry.
 #include "gfe_f64_host.h"
 
 #include <cstring>

@@ -175,14 +175,15 @@ void make_f64q_crt(uint32_t n, uint32_t b, F64QCrt *out) {
     c.qb = 0.25 * c.binv;
 }
 
-// Passes at one n, us (forward, rows, inverse; limbs of two digits in the same order after the bar):
-//   n = 19   4.6  6.8  6.3 | 4.2  7.9  5.5 (the sum is the same: limbs of two digits)
-//   n = 20   6.2 10.9  6.5, the primes side by side (7.7 10.9 11.0 one after the other); 2^7-point
-//            columns 7.3 9.3 11.1 | 8.4 13.5 9.0
-//   n = 21  10.0 14.7 11.8, side by side (11.4 14.7 13.6); 2^6-point columns 9.6 22.1 10.7 | 11.7 19.0 13.4
-//   n = 22  17.5 25.6 24.3, 2^8-point columns one prime after the other (23.1 25.6 24.3 with a workgroup per
-//            prime forward); 2^7-point columns, side by side 16.3 33.8 22.1 | 17.7 36.1 23.2
-//   n = 23  35.4 56.8 48.3 | 36 74 47
+// Passes of one squaring, us (forward, rows, inverse; after the bar limbs of two digits on the same machine):
+//   n = 19   4.6  6.8  6.3 | 4.6  7.6  4.6 (equal sums: limbs of two digits stay)
+//   n = 20   6.2 11.0  6.8, the primes side by side (7.7 11.0 11.0 one after the other); 2^7-point
+//            columns 7.3 9.3 11.1 | 6.9 11.9 7.0
+//   n = 21  10.1 15.5 12.5, side by side (inverse 13.6 one after the other); 2^6-point columns 9.6 22.1
+//            10.7 | 11.5 18.0 13.0
+//   n = 22  17.8 27.1 26.4, 2^8-point columns one prime after the other (forward with a workgroup per
+//            prime 23.1); 2^7-point columns side by side 16.3 33.8 22.1 | 17.8 38.8 23.4
+//   n = 23  34.8 57.3 49.6 | 31.0 79.7 40.4
 F64Shape f64q_shape(uint32_t n) {
     F64Shape S;
     S.quad = 1;
