@@ -179,20 +179,21 @@ __global__ void __launch_bounds__(16 << (LOGG - F64_COL_E)) k64_col_inv(F64Args 
     else f64_inv_body<3, LOGG>(A, J, dup, lds64);
 }
 
-// One candidate's inverse column pass with its primes side by side: K groups of 16 2^(LOGG - LOGE) threads,
-// one prime each, then all threads over the limbs.  C / 16 workgroups.
+// The inverse column pass with a candidate's primes side by side: K groups of 16 2^(LOGG - LOGE) threads,
+// one prime each, then all threads over the limbs.  C / 16 workgroups a slot; a slot of two primes ends
+// the third group before any barrier.
 template <int K, int LOGG>
-__global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_split(F64Args A) {
-    extern __shared__ double lds64[];
+__device__ __forceinline__ void f64_inv_split_body(const F64Args &A, const F64Job &J, int dup, double *lds) {
     constexpr int LOGE = F64_COL_E, E = 1 << LOGE;
     constexpr uint32_t T = 16u << (LOGG - LOGE), LIMBS = 16u << LOGG;
-    const F64CrtP c = (F64CrtP)A.crt;
+    const F64CrtP c = J.c;
     const uint32_t M = 1u << A.tn, C = M >> LOGG;
     const int k = __builtin_amdgcn_readfirstlane(threadIdx.x / T);
+    if (k >= K) return;
     const uint32_t t = threadIdx.x % T;
-    const unsigned blk = xcd_block(blockIdx.x, C / 16);
-    double x[E], *L = lds64 + k * LIMBS;
-    f64_col_load<LOGE, LOGG>(x, A.ws + (size_t)k * M, C, blk, t);
+    const unsigned blk = f64_block(A, J.w, C / 16);
+    double x[E], *L = lds + k * LIMBS;
+    f64_col_load<LOGE, LOGG>(x, A.ws + J.slot * A.ws_stride + (size_t)k * M, C, blk, t);
     f64_col_inv<F64Wide, LOGE, LOGG>(F64Mod{c->p[k], c->pinv[k]}, x, A.tw + (size_t)k * A.tws, t, L);
 #pragma unroll
     for (int rr = 0; rr < E; ++rr) L[((t >> 4) + ((uint32_t)rr << (LOGG - LOGE))) * 16 + (t & 15u)] = x[rr];
@@ -203,8 +204,25 @@ __global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_sp
         if (i >= LIMBS) break;  // whole waves
         double r[K];
 #pragma unroll
-        for (int m = 0; m < K; ++m) r[m] = lds64[m * LIMBS + i];
-        f64_norm_limb<K>(c, r, A.dup, (i >> 4) * C + blk * 16 + (i & 15u), M, A.regs, A.slots);
+        for (int m = 0; m < K; ++m) r[m] = lds[m * LIMBS + i];
+        f64_norm_limb<K>(c, r, dup, (i >> 4) * C + blk * 16 + (i & 15u), M, A.regs + J.slot * A.reg_stride,
+                         A.slots + J.slot * A.slot_stride);
+    }
+}
+
+// K: one candidate's primes (0.15 us a launch less than by the slot), or 0.
+template <int K, int LOGG>
+__global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_split(F64Args A) {
+    extern __shared__ double lds64[];
+    if constexpr (K != 0) {
+        const F64Job J{0, blockIdx.x, (F64CrtP)A.crt, K, true};
+        f64_inv_split_body<K, LOGG>(A, J, A.dup, lds64);
+    } else {
+        const F64Job J = f64_job(A, (1u << A.tn) >> (LOGG + 4));
+        if (!J.run) return;
+        const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
+        if (J.K == 2) f64_inv_split_body<2, LOGG>(A, J, dup, lds64);
+        else f64_inv_split_body<3, LOGG>(A, J, dup, lds64);
     }
 }
 
@@ -391,7 +409,7 @@ int f64q_build_twiddles(uint32_t n, double *tw, hipStream_t stream) {
 // With three passes, up to 2^19 limbs each is bound by latency: a wave issues one instruction in four
 // clocks, and with 16 residues a thread the row pass of 2^14 limbs was 5.2 us in a few waves.  So the
 // shapes that win there have many workgroups and short threads (8 residues per thread in the rows, and
-// `few`: the primes side by side in the inverse column pass; 2^14 limbs 14.7 -> 11.0, 2^16 16.5 ->
+// the primes side by side in the column passes, f64_few; 2^14 limbs 14.7 -> 11.0, 2^16 16.5 ->
 // 12.9, 2^17 19.1 -> 16.4, 2^18 23.4 -> 21.1, 2^19 36.3 -> 34.0) and short columns (2^14 limbs: 11.4
 // with 2^5-point columns, 11.9 with 2^6; 2^16: 13.0 and 13.6; 2^17 16.7 and 15.9).  From 2^20 limbs
 // the passes are bound by memory and fp64 issue and longer columns pay, the digits then being read
@@ -403,8 +421,6 @@ F64Shape f64_shape(uint32_t n) {
     const int tn = (int)n - 1;
     S.whole = tn <= F64_WHOLE_MAX;
     S.a = tn <= 16 ? 5 : tn <= 18 ? 6 : tn == 19 ? 7 : 8;
-    S.split = tn <= 19;
-    S.few = tn <= 19;
     return S;
 }
 
@@ -431,10 +447,11 @@ static F64Fn inv_fn(int a) {
     else return a == LOGG ? k64_col_inv<LOGG> : inv_fn<LOGG + 1>(a);
 }
 template <int K, int LOGG = F64_COL_MIN>
-static F64Fn split_fn(int a) {
+static F64Fn split_k(int a) {
     if constexpr (LOGG > F64_SPLIT_MAX) return nullptr;
-    else return a == LOGG ? k64_col_inv_split<K, LOGG> : split_fn<K, LOGG + 1>(a);
+    else return a == LOGG ? k64_col_inv_split<K, LOGG> : split_k<K, LOGG + 1>(a);
 }
+static F64Fn split_fn(int K, int a) { return K == 2 ? split_k<2>(a) : K == 3 ? split_k<3>(a) : split_k<0>(a); }
 template <int MODE, int LOGG = F64_ROW_MIN>
 static F64Fn row_fn(int logg) {
     if constexpr (LOGG > F64_ROW_MAX) return nullptr;
@@ -461,6 +478,14 @@ static F64Fn mid_fn(bool whole, int mode, int logg) {
 // would use 3 of the 8 XCDs: 118 and 63.
 static bool f64_pin(uint32_t slots) { return slots >= 7 && 7 * ((slots + 7) / 8) <= slots; }
 
+// Whether the column passes run the primes side by side: where one after the other they would be less than
+// a wave of 8 limbs a thread on every SIMD.  The forward pass then takes one prime per workgroup (else all
+// from one read of the digits), the inverse one a prime per group of threads.  us per round, one after the
+// other and side by side: 16 slots of n = 14 14.6 and 11.8, 16 of n = 15 17.7 and 15.6, 3 of n = 18 32.6 and
+// 29.1, 2 of n = 20 (2^20 limbs) 41.7 and 40.5; past it 64 of n = 15 34.3 and 36.3, 7 of n = 18 37.8 and
+// 39.0, 24 of n = 18 87.7 and 93.7, 512 of n = 15 205 and 218, 8 of n = 20 120 and 128.
+static bool f64_few(const F64Args &A) { return ((uint64_t)A.nslots << A.tn) <= (1u << 19); }
+
 // Workgroups of a launch of `per` a slot (f64_job).
 static dim3 f64_grid(F64Args &A, uint32_t per) {
     A.pin = !A.K && f64_pin(A.nslots);
@@ -470,8 +495,9 @@ static dim3 f64_grid(F64Args &A, uint32_t per) {
 void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream) {
     if (S.quad) return f64q_launch_fwd(A, S, stream);
     const unsigned nb = 1u << (A.tn - S.a - 4), T = 16u << (S.a - F64_COL_E);
-    const dim3 grid = f64_grid(A, S.split ? 3 * nb : nb);
-    hipLaunchKernelGGL(fwd_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A, S.split);
+    const int split = f64_few(A);
+    const dim3 grid = f64_grid(A, split ? 3 * nb : nb);
+    hipLaunchKernelGGL(fwd_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A, split);
 }
 
 void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) {
@@ -504,11 +530,12 @@ void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
         return;
     }
     const unsigned T = 16u << (S.a - F64_COL_E), nb = 1u << (A.tn - S.a - 4);
-    if (A.K && S.few) {
-        hipLaunchKernelGGL(A.K == 2 ? split_fn<2>(S.a) : split_fn<3>(S.a), dim3(nb), dim3(A.K * T), (size_t)A.K * 128 << S.a, stream, A);
+    const dim3 grid = f64_grid(A, nb);
+    if (f64_few(A)) {
+        const unsigned K = A.K ? A.K : 3;
+        hipLaunchKernelGGL(split_fn(A.K, S.a), grid, dim3(K * T), (size_t)K * 128 << S.a, stream, A);
         return;
     }
-    const dim3 grid = f64_grid(A, nb);
     hipLaunchKernelGGL(inv_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A);
 }
 
@@ -530,8 +557,7 @@ void f64_set_lds_attributes() {
         }
         f64q_set_lds_attributes();
         for (int a = F64_COL_MIN; a <= F64_SPLIT_MAX; ++a) {
-            set((const void *)split_fn<2>(a));
-            set((const void *)split_fn<3>(a));
+            for (int k : {0, 2, 3}) set((const void *)split_fn(k, a));
         }
         for (int m = 0; m < 4; ++m) {
             for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, l));

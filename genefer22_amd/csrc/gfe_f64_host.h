@@ -12,12 +12,10 @@
 namespace gfe {
 
 // Shape of the passes at one n.  whole: a prime's transform in one workgroup and the normalisation
-// after it; else three passes over 2^a rows of 2^(n-1-a) limbs, the forward column pass with one prime
-// per workgroup (split) instead of all.  few: one candidate's work is too little for the chip, so its
-// inverse column pass runs its primes side by side.  quad: limbs of four digits (gfe_f64q.h), three passes over
-// 2^(n-2) of them.
+// after it; else three passes over 2^a rows of 2^(n-1-a) limbs, or with quad of 2^(n-2-a) limbs of four
+// digits (gfe_f64q.h).
 struct F64Shape {
-    int whole = 0, a = 0, split = 0, few = 0, quad = 0;
+    int whole = 0, a = 0, quad = 0;
 };
 
 // Primes the transform needs for (b, n): 2 or 3, or 0 where it is not exact (or out of range).

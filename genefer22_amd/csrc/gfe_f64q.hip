@@ -188,7 +188,6 @@ F64Shape f64q_shape(uint32_t n) {
     F64Shape S;
     S.quad = 1;
     S.a = n >= 22 ? F64Q_COL_MAX : n == 21 ? 7 : 6;
-    S.split = S.few = S.a <= F64Q_SPLIT_MAX;
     return S;
 }
 
@@ -207,7 +206,8 @@ static F64QFn qrow_fn(int mode, int logg) {
 
 void f64q_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream) {
     const unsigned nb = 1u << (A.tn - S.a - 4);
-    hipLaunchKernelGGL(qfwd_fn(S.a), dim3(S.split ? F64Q_PRIMES * nb : nb), dim3(16u << (S.a - F64_COL_E)), (size_t)128 << S.a, stream, A, S.split);
+    const int split = S.a <= F64Q_SPLIT_MAX;  // the primes side by side
+    hipLaunchKernelGGL(qfwd_fn(S.a), dim3(split ? F64Q_PRIMES * nb : nb), dim3(16u << (S.a - F64_COL_E)), (size_t)128 << S.a, stream, A, split);
 }
 
 void f64q_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream) {
@@ -218,7 +218,7 @@ void f64q_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t 
 void f64q_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream) {
     const unsigned nb = 1u << (A.tn - S.a - 4);
     const size_t lds = (size_t)128 << S.a;
-    if (S.few) hipLaunchKernelGGL(qsplit_fn(S.a), dim3(nb), dim3(F64Q_PRIMES * f64q_split_threads(S.a)), F64Q_PRIMES * lds, stream, A);
+    if (S.a <= F64Q_SPLIT_MAX) hipLaunchKernelGGL(qsplit_fn(S.a), dim3(nb), dim3(F64Q_PRIMES * f64q_split_threads(S.a)), F64Q_PRIMES * lds, stream, A);
     else hipLaunchKernelGGL((k64q_col_inv<F64Q_COL_MAX>), dim3(nb), dim3(16u << (S.a - F64_COL_E)), (F64Geo<F64Q_COL_MAX, F64_COL_E>::NCH * lds), stream, A);
 }
 
