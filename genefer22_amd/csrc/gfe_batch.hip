@@ -902,9 +902,7 @@ void Batch::square(const uint8_t *active, const uint8_t *dup, const uint8_t *mul
     if (mode64()) {
         F64Args A = args64(active, dup, mulf);
         A.absorb = 1;
-        if (!shape.whole) f64_launch_fwd(A, shape, stream);
-        f64_launch_mid(A, shape, has_mul ? F64_EITHER : F64_SQUARE, stream);
-        f64_launch_inv(A, shape, stream);
+        f64_launch_square(A, shape, has_mul ? F64_EITHER : F64_SQUARE, stream);
         return;
     }
     BArgs A = args(active, dup);

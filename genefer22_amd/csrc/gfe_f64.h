@@ -292,10 +292,22 @@ __device__ __forceinline__ void f64_quad_mul(const F64Mod &md, double &a0, doubl
     a0 = c0; a1 = c1; a2 = c2; a3 = c3;
 }
 
-// load(x, base, YL): the first chunk's elements base + rr 2^YL, at most 0.52 p.  `data` / `zp` at the
+// The store of a row's result to `data`.
+template <int E>
+struct F64Store {
+    double *data;
+    template <class YL>
+    __device__ __forceinline__ void operator()(const double (&x)[E], uint32_t base, YL) const {
+#pragma unroll
+        for (int rr = 0; rr < E; ++rr) data[base + ((uint32_t)rr << YL::value)] = x[rr];
+    }
+};
+
+// load(x, base, YL): the first chunk's elements base + rr 2^YL, at most 0.52 p; store(x, base, YL): the same
+// elements of the result (F64_FWD writes `data`).  `data` / `zp` at the
 // row's first residue, `row` its index among the 2^a rows, L its LDS words.
-template <class SZ, int LOGG, int LOGE, int MODE, class LD>
-__device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, double *__restrict__ data,
+template <class SZ, int LOGG, int LOGE, int MODE, class LD, class ST>
+__device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, const ST &store, double *__restrict__ data,
                                              const double *__restrict__ zp, const double *__restrict__ tw, int a,
                                              uint32_t row, uint32_t s, double *L, bool mul) {
     using GM = F64Geo<LOGG, LOGE>;
@@ -388,8 +400,7 @@ __device__ __forceinline__ void f64_row_pass(const F64Mod &md, const LD &load, d
             }
             f64_inv_chunk<SZ, LOGE, NE, ci == LAST, true>(md, x, w);
             if constexpr (ci == 0) {
-#pragma unroll
-                for (int rr = 0; rr < E; ++rr) data[base + (rr << YL)] = x[rr];
+                store(x, base, std::integral_constant<int, YL>{});
             } else {
                 double *p = L + base + (base >> LOGE);
 #pragma unroll

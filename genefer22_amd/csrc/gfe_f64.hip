@@ -93,7 +93,7 @@ __global__ void __launch_bounds__(f64_row_threads(LOGG)) k64_row(F64Args A) {
 #pragma unroll
         for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = md.red(x[rr]);
     };
-    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
+    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, F64Store<1 << LOGE>{data}, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, s,
                                             lds64 + q * f64_row_words(LOGG),
                                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
@@ -129,7 +129,7 @@ __device__ __forceinline__ void f64_whole_body(const F64Args &A, const F64Job &J
 #pragma unroll
         for (int rr = 0; rr < E; ++rr) x[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
     };
-    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
+    f64_row_pass<F64Wide, LOGG, LOGE, MODE>(md, load, F64Store<E>{A.ws + at}, A.ws + at, A.zp + at, A.tw + (size_t)k * A.tws, 0, 0, s, lds,
                                             MODE == F64_EITHER && A.mulf && A.mulf[J.slot]);
 }
 
@@ -150,6 +150,68 @@ __global__ void __launch_bounds__(512) k64_whole_mixed(F64Args A) {
     if (!J.run || (int)J.w >= J.K) return;
     if (J.c->n == 13) f64_whole_body<12, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
     else if (threadIdx.x < 256) f64_whole_body<11, MODE>(A, J, (int)J.w, threadIdx.x, lds64);
+}
+
+// A slot's whole squaring in one workgroup: the primes one after the other, each thread keeping its limbs'
+// residues, then the CRT and the carry (the digits and range carries are read by every thread before the
+// first exchange's barrier, so before any is written).
+template <int K, int LOGG>
+__device__ __forceinline__ void f64_all_body(const F64Args &A, const F64Job &J, double *lds) {
+    constexpr int LOGE = f64_row_loge(LOGG), E = 1 << LOGE, YL = LOGG - LOGE;
+    const F64CrtP c = J.c;
+    const uint32_t s = threadIdx.x;
+    const double bd = c->bd;
+    const bool reduce = c->big != 0;
+    int32_t *regs = A.regs + J.slot * A.reg_stride;
+    int4 *slots = A.slots + J.slot * A.slot_stride;
+    int2 d[E];
+#pragma unroll
+    for (int rr = 0; rr < E; ++rr) d[rr] = reinterpret_cast<const int2 *>(regs)[s + ((uint32_t)rr << YL)];
+    if ((s & 15u) < 2) {  // as f64_load_digits
+        const uint32_t q = s & 1u;
+        int2 e[E];
+#pragma unroll
+        for (int rr = 0; rr < E; ++rr) e[rr] = reinterpret_cast<const int2 *>(slots + ((s + ((uint32_t)rr << YL)) >> 4))[q];
+#pragma unroll
+        for (int rr = 0; rr < E; ++rr) {
+            d[rr].x += e[rr].x;
+            d[rr].y += q == 0 ? e[rr].y : 0;
+        }
+    }
+    double x[K][E];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const F64Mod md{c->p[k], c->pinv[k]};
+        const auto load = [&](double (&y)[E], uint32_t, auto) {
+#pragma unroll
+            for (int rr = 0; rr < E; ++rr) y[rr] = f64_limb(md, d[rr].x, d[rr].y, bd, reduce);
+        };
+        const auto store = [&](const double (&y)[E], uint32_t, auto) {
+#pragma unroll
+            for (int rr = 0; rr < E; ++rr) x[k][rr] = y[rr];
+        };
+        if (k) __syncthreads();  // the last prime's reads of lds
+        f64_row_pass<F64Wide, LOGG, LOGE, F64_SQUARE>(md, load, store, nullptr, nullptr, A.tw + (size_t)k * A.tws, 0, 0, s,
+                                                      lds, false);
+    }
+    const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
+#pragma unroll
+    for (int rr = 0; rr < E; ++rr) {
+        double r[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) r[k] = x[k][rr];
+        f64_norm_limb<K>(c, r, dup, s + ((uint32_t)rr << YL), 1u << LOGG, regs, slots);
+    }
+}
+
+// One workgroup a slot.
+template <int LOGG>
+__global__ void __launch_bounds__(1 << (LOGG - f64_row_loge(LOGG))) k64_all(F64Args A) {
+    extern __shared__ double lds64[];
+    const F64Job J = f64_job(A, 1);
+    if (!J.run) return;
+    if (J.K == 2) f64_all_body<2, LOGG>(A, J, lds64);
+    else f64_all_body<3, LOGG>(A, J, lds64);
 }
 
 template <int K, int LOGG>
@@ -462,6 +524,7 @@ static F64Fn whole_fn(int logg) {
     if constexpr (LOGG > F64_WHOLE_MAX) return nullptr;
     else return logg == LOGG ? k64_whole<LOGG, MODE> : whole_fn<MODE, LOGG + 1>(logg);
 }
+static F64Fn all_fn(int logg) { return logg == 11 ? k64_all<11> : k64_all<12>; }
 static F64Fn mid_fn(bool whole, int mode, int logg) {
     switch (mode) {
         case F64_SQUARE: return whole ? whole_fn<F64_SQUARE>(logg) : row_fn<F64_SQUARE>(logg);
@@ -539,6 +602,24 @@ void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
     hipLaunchKernelGGL(inv_fn(S.a), grid, dim3(T), (size_t)128 << S.a, stream, A);
 }
 
+// Whether a round of one-workgroup slots (n = 12, 13) runs each slot's three primes and CRT in one workgroup
+// (k64_all): one launch, no residues to memory, but a CU's time for one slot or two or .. for
+// all: where the last layer of 256 slots is nearly full.  us per round, k64_whole with k64_norm and k64_all:
+// n = 12 128 slots 11.8 and 13.5, 200 15.1 and 13.9, 256 16.4 and 14.3, 301 19.0 and 20.2, 512 26.9 and
+// 21.7, 1024 46.1 and 38.6; n = 13 128 slots 18.5 and 20.6, 256 27.5 and 22.2, 301 32.7 and 40.1, 512 46.8 and 41.3.
+static bool f64_all(uint32_t slots) { return 8 * slots >= 7 * 256 * ((slots + 255) / 256); }
+
+void f64_launch_square(F64Args A, const F64Shape &S, int mode, hipStream_t stream) {
+    if (S.whole && !A.mixed && mode == F64_SQUARE && f64_all(A.nslots)) {
+        const dim3 grid = f64_grid(A, 1);
+        hipLaunchKernelGGL(all_fn(A.tn), grid, dim3(1u << (A.tn - f64_row_loge(A.tn))), (size_t)8 * f64_row_words(A.tn), stream, A);
+        return;
+    }
+    if (!S.whole) f64_launch_fwd(A, S, stream);
+    f64_launch_mid(A, S, mode, stream);
+    f64_launch_inv(A, S, stream);
+}
+
 void f64_launch_flush(const F64Args &A, hipStream_t stream) {
     const dim3 grid(((1u << (A.tn - 4)) + 255) / 256, A.nslots);
     hipLaunchKernelGGL(k64_flush, grid, dim3(256), 0, stream, A);
@@ -559,6 +640,7 @@ void f64_set_lds_attributes() {
         for (int a = F64_COL_MIN; a <= F64_SPLIT_MAX; ++a) {
             for (int k : {0, 2, 3}) set((const void *)split_fn(k, a));
         }
+        for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)all_fn(l));
         for (int m = 0; m < 4; ++m) {
             for (int l = F64_ROW_MIN; l <= F64_ROW_MAX; ++l) set((const void *)mid_fn(false, m, l));
             for (int l = F64_WHOLE_MIN; l <= F64_WHOLE_MAX; ++l) set((const void *)mid_fn(true, m, l));

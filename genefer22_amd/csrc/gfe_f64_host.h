@@ -64,6 +64,9 @@ struct F64Args {
 void f64_launch_fwd(F64Args A, const F64Shape &S, hipStream_t stream);           // three passes only
 void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream); // row, or whole
 void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream);
+// A batch's round, mode F64_SQUARE or F64_EITHER: the three in turn of register 0 with its range carries
+// (A.absorb), or one launch for all.
+void f64_launch_square(F64Args A, const F64Shape &S, int mode, hipStream_t stream);
 // Adds the pending range carries of register 0 and balances it.
 void f64_launch_flush(const F64Args &A, hipStream_t stream);
 void f64_set_lds_attributes();

@@ -49,7 +49,7 @@ __global__ void __launch_bounds__(1 << (LOGG - f64_row_loge(LOGG))) k64q_row(F64
 #pragma unroll
         for (int rr = 0; rr < 1 << LOGE; ++rr) x[rr] = data[base + ((uint32_t)rr << decltype(yl)::value)];
     };
-    f64_row_pass<F64Slim, LOGG, LOGE, MODE>(md, load, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, threadIdx.x, lds64, false);
+    f64_row_pass<F64Slim, LOGG, LOGE, MODE>(md, load, F64Store<1 << LOGE>{data}, data, A.zp + at, A.tw + (size_t)k * A.tws, A.a, row, threadIdx.x, lds64, false);
 }
 
 // C / 16 workgroups.

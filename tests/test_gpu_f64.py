@@ -109,12 +109,12 @@ def run_batch(gfe, n, bases, iters, integer=False, graphs=True, mixed=False):
     return sorted((r["tag"], r["res64"], r["old64"], r["hash64"]) for r in got)
 
 
-@pytest.mark.parametrize("n,count", [(12, 9), (12, 8), (13, 15), (14, 3), (14, 64), (14, 65), (15, 7), (17, 8), (18, 5),
-                                     (19, 2), (20, 1)])
+@pytest.mark.parametrize("n,count", [(12, 9), (12, 8), (12, 223), (12, 224), (13, 15), (13, 225), (14, 3), (14, 64), (14, 65),
+                                     (15, 7), (17, 8), (18, 5), (19, 2), (20, 1)])
 def test_batches_equal_the_integer_passes(gfe, n, count):
     """Slots spread over the XCDs or pinned to one each, two and three primes side by side, the primes one
-    after the other in the column passes (past 2^19 limbs) and side by side, slots that
-    end rounds before others, graphs and single launches."""
+    after the other in the column passes (past 2^19 limbs) and side by side, a slot's squaring in one
+    workgroup (from 224 slots) or one a prime, slots that end rounds before others, graphs and single launches."""
     e = largest_two_prime_base(n)
     bases = [(1026, 1999999898, e & ~1, (e & ~1) + 2, 146950, 20204692)[i % 6] + 2 * (i // 6) for i in range(count)]
     want = run_batch(gfe, n, bases, 70, integer=True)
