@@ -216,11 +216,11 @@ def base_pieces(x, b, count):
 
 
 def qpieces(x, b, n, dup, rng):
-    """f64q_crt_pieces on raw residues of any representative up to 18 p; every sum has to be exact."""
+    """f64q_crt_pieces on raw residues of any representative up to 64 p (8 p into the last chunk of three levels); every sum has to be exact."""
     v = []
     for k, p in enumerate(Q):
         pinv, s = 1.0 / p, pow(pow(2, n - 4, p), -1, p)
-        raw = float((x // (2 if dup else 1)) * pow(s, -1, p) % p + p * rng.randrange(-18, 18))
+        raw = float((x // (2 if dup else 1)) * pow(s, -1, p) % p + p * rng.randrange(-64, 64))
         t = mul(raw, bal(s * (2 if dup else 1), p), p, pinv)
         for j in range(k):
             t = mul(t - v[j], bal(pow(Q[j], -1, p), p), p, pinv)
