@@ -112,7 +112,7 @@ int gfe_time_squarings(gfe_engine *e, uint32_t count, uint64_t dup_bits, double 
 int gfe_tune(gfe_engine *e, uint32_t reps);
 
 /* An engine squares, and forms multiplicands, in a double-precision limb transform (exact: integer
- * residues of 49-bit primes in doubles) wherever that is exact for its (b, n), which leaves out only
+ * residues of 49- or 45-bit primes in doubles) wherever that is exact for its (b, n), which leaves out only
  * bases below 2,300 at n >= 21.  The plan below shapes the integer passes: they run where it is not,
  * and from gfe_set_plan on (gfe_tune keeps whichever is faster, gfe_rebase goes back to the default).
  *
