@@ -240,8 +240,10 @@ __global__ void __launch_bounds__(256) kb_set(BArgs A) {
     if (i < N) A.regs[s * A.reg_stride + A.dst_reg * N + i] = (i == 0) ? A.value : 0;
 }
 
-// A slot taken by a candidate: its constants, and r0 = r1 = 1.  They come as arguments of the one launch:
-// four uploads and two kb_set launches over every slot's workgroups took 30-37 us a candidate.
+// A slot taken by a candidate: its constants, r0 = r1 = 1, and no pending carries (the last candidate's
+// would be added to r0: timed rounds leave some in a slot that only waits for its read-back).  The
+// constants come as arguments of the one launch: four uploads and two kb_set launches over every
+// slot's workgroups took 30-37 us a candidate.
 struct SlotInit {
     SlotInfo si;
     CrtConst c;
@@ -249,14 +251,15 @@ struct SlotInit {
     SlotInfo *slots;
     CrtConst *crt;
     F64Crt *crt64;
-    int4 *r0, *r1;
-    uint32_t n4;
+    int4 *r0, *r1, *carry;
+    uint32_t n4, c4;  // c4 <= n4: carries of the batch's largest n
     int s;
 };
 __global__ void __launch_bounds__(256) kb_take_slot(SlotInit A) {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= A.n4) return;
     A.r0[i] = A.r1[i] = make_int4(i == 0, 0, 0, 0);
+    if (i < A.c4) A.carry[i] = make_int4(0, 0, 0, 0);
     if (i == 0) {
         A.slots[A.s] = A.si;
         A.crt[A.s] = A.c;
@@ -1105,6 +1108,8 @@ int Batch::submit(uint32_t b, uint64_t iters, uint64_t tag, int32_t *slot_out, u
     A.slots = slots_dev; A.crt = crt; A.crt64 = crt64; A.s = s;
     A.r0 = reinterpret_cast<int4 *>(reg(s, 0)); A.r1 = reinterpret_cast<int4 *>(reg(s, 1));
     A.n4 = (uint32_t)(slot_N(s) / 4);
+    A.carry = reinterpret_cast<int4 *>(carry) + (size_t)s * (NA / 16);
+    A.c4 = (uint32_t)(NA / 16);
     zl = std::max(zl, (uint32_t)s + 1);
     hipLaunchKernelGGL(kb_take_slot, dim3((A.n4 + 255) / 256), dim3(256), 0, stream, A);
     if (slot_out) *slot_out = s;
