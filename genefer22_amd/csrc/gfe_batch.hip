@@ -413,10 +413,12 @@ struct Batch {
     // 512 slots, measured on MI355X: 0.367 ms per round either way; n = 20, one slot: 52.9 us against
     // 54.8 us with the carry kernel).
     bool carries_pending = false;
-    // The double-precision limb transform: selected until gfe_batch_set_plan (n <= F64_ALL_BASES_N), and
-    // in use while a power run holds a multiplicand in it.  Its range carries stay pending from round
-    // to round in every shape.  carry64: the form `carry` holds.
+    // The double-precision limb transform: selected until gfe_batch_set_plan, or by the tuner
+    // (n <= F64_ALL_BASES_N), but a power run ends in the transform that holds its multiplicand
+    // (mode64).  Its range carries stay pending from round to round in every shape.  carry64: the form
+    // `carry` holds.  timed64: what the tuner times, 0 or 1, whatever is under way (no products then).
     bool f64 = false, carry64 = false;
+    int timed64 = -1;
     F64Shape shape;
     double *tw64 = nullptr;
     F64Crt *crt64 = nullptr;
@@ -731,14 +733,14 @@ F64Args Batch::args64(const uint8_t *active, const uint8_t *dup, const uint8_t *
     return A;
 }
 
-// Whether squarings and products run in doubles: selected, or a power run's multiplicand is in them.
+// Whether squarings and products run in doubles: as the multiplicands of the power runs under way (which
+// are all in one transform, since a multiplicand made beside them goes into theirs), else as selected.
 bool Batch::mode64() const {
-    if (f64) return true;
-    for (uint32_t s = 0; s < cap; ++s)
-        if (slots[s].busy && slots[s].zp64 && !slots[s].q.empty() && slots[s].q.front().kind == IT_RUN &&
-            slots[s].q.front().run == RUN_POW)
-            return true;
-    return false;
+    if (timed64 >= 0) return timed64 != 0;
+    for (uint32_t s = 0; depth > 0 && s < cap; ++s)  // powers are a proof's
+        if (slots[s].busy && !slots[s].q.empty() && slots[s].q.front().kind == IT_RUN && slots[s].q.front().run == RUN_POW)
+            return slots[s].zp64;
+    return f64;
 }
 
 // `carry` in the form of the transform about to run: pending carries of the other are applied first.
@@ -1640,8 +1642,7 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
     if (hipMalloc(&save, (size_t)B.cap * row) != hipSuccess) return set_error(GFE_ENOMEM, "tune save");
     (void)hipMemcpy2DAsync(save, row, B.regs, pitch, row, B.cap, hipMemcpyDeviceToDevice, B.stream);
     const gfe::Plan orig = B.plan;
-    const bool f64_was = B.f64;
-    B.f64 = false;
+    B.timed64 = 0;
     gfe::Plan best = orig;
     double best_ms = 1e30;
     const bool graphs = B.use_graphs;
@@ -1694,10 +1695,10 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
     B.use_graphs = graphs;
     B.drop_graphs();
     (void)B.zero_carries();
-    if (f64_was) {  // the double-precision transform against the chosen plan, as blocks run
+    if (B.n <= gfe::F64_ALL_BASES_N) {  // the double-precision transform against the chosen plan, as blocks run
         double t[2] = {1e30, 1e30};
         for (int pass = 0; pass < 4; ++pass) {
-            B.f64 = (pass & 1) != 0;
+            B.timed64 = pass & 1;
             double ms = 0;
             if (gfe_batch_time_rounds(b, 64, &ms) != GFE_OK || gfe_batch_time_rounds(b, 128, &ms) != GFE_OK) continue;
             t[pass & 1] = std::min(t[pass & 1], ms);
@@ -1705,8 +1706,8 @@ int gfe_batch_tune(gfe_batch *b, uint32_t reps) {
         B.f64 = t[1] < t[0];
         B.drop_graphs();
         (void)B.zero_carries();
-        B.carry64 = B.f64;
     }
+    B.timed64 = -1;
     (void)hipMemcpy2DAsync(B.regs, pitch, save, row, row, B.cap, hipMemcpyDeviceToDevice, B.stream);
     (void)hipStreamSynchronize(B.stream);
     (void)hipFree(save);

@@ -77,8 +77,9 @@ size_t gfe_batch_proof_slot_bytes(uint32_t n, uint32_t depth);
 int gfe_batch_tune(gfe_batch *bt, uint32_t reps);
 int gfe_batch_info(const gfe_batch *bt, char *buf, size_t len);
 /* The batch's pass plan, as gfe_get_plan / gfe_set_plan of gfe.h: up to n = 20 a batch squares in the
- * double-precision limb transform until gfe_batch_set_plan selects the integer passes (power runs
- * under way then end in the transform that holds their multiplicand). */
+ * double-precision limb transform until gfe_batch_set_plan selects the integer passes, and again once
+ * gfe_batch_tune finds it to be faster (power runs under way end in the transform that holds their
+ * multiplicand, and the batch with them). */
 int gfe_batch_get_plan(const gfe_batch *bt, int32_t plan[6]);
 int gfe_batch_set_plan(gfe_batch *bt, const int32_t plan[6]);
 
