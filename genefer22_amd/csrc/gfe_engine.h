@@ -115,8 +115,8 @@ struct Engine {
     std::vector<hipEvent_t> events;
     bool dev_ok = false;
     // The carries of the last normalisation are not yet in register 0: the next squaring's column
-    // forward pass adds them on the way in (plans with compile-time passes); every other use of the
-    // registers runs the carry kernel first (flush_carry).
+    // forward pass adds them on the way in (plans with compile-time passes); other readers of register 0
+    // take it from where `flushed` leaves it or run the carry kernel first (flush_carry).
     bool carry_pending = false;
     // what the pending carries are: 0 k_norm's workgroup carries, 1 k_norm_limb's boundary pairs,
     // 2 the range slots of ks_col_inv_norm_limb (ranges of 2^pend_rlog limbs), 3 those of the
@@ -124,6 +124,14 @@ struct Engine {
     int pend_kind = 0, pend_rlog = 0;
     bool defer_carry() const { return plan.spec && !plan.pipe && (!plan.fused || plan.limb) && !plan.fuse_sq; }
     void flush_carry();
+    // Where register 0 stands with the pending carries added, for a reader: the double-precision
+    // transform's go with it to `dst` (another register, or null: the work space) in one launch and stay
+    // pending, others into the register first.  ws0: the work space holds it so, until the next pass
+    // writes there or register 0 changes.
+    bool ws0 = false;
+    const int32_t *flushed(int32_t *dst);
+    // Register 0 is overwritten whole: its pending carries are gone with it.
+    void drop_carry() { carry_pending = ws0 = false; }
 
     ~Engine();
     int init(uint32_t b, uint32_t n, uint32_t num_regs, int device);

@@ -88,13 +88,14 @@ __global__ void __launch_bounds__(256) k_fold(FoldArgs A) {
 }
 
 struct MulScalarArgs {
+    const int32_t *src;
     int32_t *dst;
     int64_t *carry;
     uint32_t b;
     int32_t a;
 };
 
-__global__ void __launch_bounds__(256) k_mulscalar(MulScalarArgs A) { mulscalar_body(A.dst, A.carry, A.b, A.a, blockIdx.x); }
+__global__ void __launch_bounds__(256) k_mulscalar(MulScalarArgs A) { mulscalar_body(A.src, A.dst, A.carry, A.b, A.a, blockIdx.x); }
 
 // Register copy, 16 bytes per thread (the reference's copy kernel, ocl/kernel.cl:2501-2506).
 __global__ void __launch_bounds__(256) k_copy(int4 *__restrict__ dst, const int4 *__restrict__ src, size_t n4) {
@@ -1046,8 +1047,21 @@ void Engine::launch_norm(int dup) {
 
 void Engine::flush_carry() {
     if (!carry_pending) return;
-    carry_pending = false;
+    drop_carry();
     launch_carry();
+}
+
+const int32_t *Engine::flushed(int32_t *dst) {
+    if (!carry_pending || pend_kind != 3) {
+        flush_carry();
+        return regs;
+    }
+    int32_t *const w = reinterpret_cast<int32_t *>(ws);
+    if (ws0) return w;
+    ws0 = dst == nullptr;
+    if (ws0) dst = w;
+    f64_launch_flush_to(f64_args(0), shape, b, dst, stream);
+    return dst;
 }
 
 void Engine::launch_carry() {
@@ -1141,11 +1155,12 @@ F64Args Engine::f64_args(int dup) const {
 // Register `src` through the passes up to the row pass of `mode`, into `out` (ws or zp); from register 0
 // its range carries are added on the way in, and the caller overwrites the register.
 void Engine::f64_run(uint32_t src, uint32_t *out, int mode) {
-    if (carry_pending && (src != 0 || pend_kind != 3)) flush_carry();
+    if (carry_pending && src == 0 && pend_kind != 3) flush_carry();
     F64Args A = f64_args(0);
     A.src_reg = src;
     A.ws = reinterpret_cast<double *>(out);
-    A.absorb = carry_pending;
+    A.absorb = carry_pending && src == 0;
+    if (out == ws) ws0 = false;
     if (!shape.whole) f64_launch_fwd(A, shape, stream);
     f64_launch_mid(A, shape, mode, stream);
 }
@@ -1186,7 +1201,7 @@ void Engine::mul() {
 }
 
 void Engine::init_multiplicand(uint32_t src) {
-    flush_carry();  // register 0 is read but not rewritten
+    if (!f64 || src == 0) flush_carry();  // register 0 is read but not rewritten
     zp_f64 = f64;
     if (f64) {
         f64_run(src, zp, F64_FWD);
@@ -1197,8 +1212,9 @@ void Engine::init_multiplicand(uint32_t src) {
 }
 
 void Engine::mul_scalar(int32_t a) {
-    flush_carry();
     MulScalarArgs A;
+    A.src = flushed(nullptr);
+    drop_carry();
     A.dst = regs; A.carry = carry; A.b = b; A.a = a;
     const unsigned nwg = (unsigned)(N / (8 * 256));
     hipLaunchKernelGGL(k_mulscalar, dim3(nwg, 1, 1), dim3(256), 0, stream, A);
@@ -1208,13 +1224,17 @@ void Engine::mul_scalar(int32_t a) {
 void Engine::copy(uint32_t dst, uint32_t src) {
     const size_t n4 = N / 4;
     const int T = 256;
+    int32_t *to = regs + (size_t)dst * N;
+    const int32_t *from = src == 0 ? flushed(to) : regs + (size_t)src * N;
+    if (dst == 0) drop_carry();
+    if (from == to) return;  // flushed there
     hipLaunchKernelGGL(k_copy, dim3((unsigned)((n4 + T - 1) / T), 1, 1), dim3(T), 0, stream,
-                       reinterpret_cast<int4 *>(regs + (size_t)dst * N), reinterpret_cast<const int4 *>(regs + (size_t)src * N),
-                       n4);
+                       reinterpret_cast<int4 *>(to), reinterpret_cast<const int4 *>(from), n4);
 }
 
 void Engine::set(uint32_t a) {
     const int T = 256;
+    drop_carry();
     hipLaunchKernelGGL(k_set, dim3((unsigned)((N + T - 1) / T), 1, 1), dim3(T), 0, stream, regs, N, (int32_t)a);
 }
 
@@ -1279,7 +1299,6 @@ int gfe_destroy(gfe_engine *e) {
 int gfe_set(gfe_engine *e, uint32_t a) {
     GFE_GUARD(e);
     if ((uint64_t)a > (uint64_t)(e->eng.b / 2) + 4) return set_error(GFE_EINVAL, "set: a exceeds b/2 + 4");
-    e->eng.flush_carry();
     e->eng.set(a);
     return e->eng.check("set");
 }
@@ -1317,7 +1336,6 @@ int gfe_mul(gfe_engine *e) {
 
 int gfe_copy(gfe_engine *e, uint32_t dst, uint32_t src) {
     GFE_GUARD(e);
-    e->eng.flush_carry();
     Engine &g = e->eng;
     if (dst >= g.num_regs || src >= g.num_regs) return set_error(GFE_EINVAL, "register index out of range");
     if (dst == src) return GFE_OK;
@@ -1327,11 +1345,11 @@ int gfe_copy(gfe_engine *e, uint32_t dst, uint32_t src) {
 
 int gfe_get_digits(gfe_engine *e, uint32_t reg, int32_t *out) {
     GFE_GUARD(e);
-    e->eng.flush_carry();
     Engine &g = e->eng;
     if (!out) return set_error(GFE_EINVAL, "null output");
     if (reg >= g.num_regs) return set_error(GFE_EINVAL, "register index out of range");
-    if (hipMemcpyAsync(out, g.regs + (size_t)reg * g.N, g.N * 4, hipMemcpyDeviceToHost, g.stream) != hipSuccess)
+    const int32_t *from = reg == 0 ? g.flushed(nullptr) : g.regs + (size_t)reg * g.N;
+    if (hipMemcpyAsync(out, from, g.N * 4, hipMemcpyDeviceToHost, g.stream) != hipSuccess)
         return set_error(GFE_EHIP, "read");
     if (hipStreamSynchronize(g.stream) != hipSuccess) return set_error(GFE_EHIP, "read sync");
     return GFE_OK;
@@ -1339,7 +1357,6 @@ int gfe_get_digits(gfe_engine *e, uint32_t reg, int32_t *out) {
 
 int gfe_set_digits(gfe_engine *e, uint32_t reg, const int32_t *in) {
     GFE_GUARD(e);
-    e->eng.flush_carry();
     Engine &g = e->eng;
     if (!in) return set_error(GFE_EINVAL, "null input");
     if (reg >= g.num_regs) return set_error(GFE_EINVAL, "register index out of range");
@@ -1348,6 +1365,7 @@ int gfe_set_digits(gfe_engine *e, uint32_t reg, const int32_t *in) {
     const int64_t bound = (int64_t)(g.b / 2) + 4;
     for (size_t i = 0; i < g.N; ++i)
         if ((int64_t)in[i] > bound || (int64_t)in[i] < -bound) return set_error(GFE_EINVAL, "digit out of balanced range");
+    if (reg == 0) g.drop_carry();
     if (hipMemcpyAsync(g.regs + (size_t)reg * g.N, in, g.N * 4, hipMemcpyHostToDevice, g.stream) != hipSuccess)
         return set_error(GFE_EHIP, "write");
     if (hipStreamSynchronize(g.stream) != hipSuccess) return set_error(GFE_EHIP, "write sync");
@@ -1426,7 +1444,6 @@ static void balance_digits(int32_t *d, size_t N, uint32_t b) {
 // balanced here, as the engine keeps them.
 int gfe_load(gfe_engine *e, uint32_t num_regs, const void *buf, size_t size) {
     GFE_GUARD(e);
-    e->eng.flush_carry();
     Engine &g = e->eng;
     if (num_regs == 0) num_regs = g.num_regs;
     if (num_regs > g.num_regs) return set_error(GFE_EINVAL, "num_regs");
@@ -1456,6 +1473,7 @@ int gfe_load(gfe_engine *e, uint32_t num_regs, const void *buf, size_t size) {
         }
         balance_digits(dr, g.N, g.b);
     }
+    g.drop_carry();
     if (hipMemcpyAsync(g.regs, d.data(), d.size() * 4, hipMemcpyHostToDevice, g.stream) != hipSuccess)
         return set_error(GFE_EHIP, "load");
     if (hipStreamSynchronize(g.stream) != hipSuccess) return set_error(GFE_EHIP, "load sync");
@@ -1479,7 +1497,7 @@ int gfe_info(const gfe_engine *e, char *buf, size_t len) {
 
 int gfe_sync(gfe_engine *e) {
     GFE_GUARD(e);
-    e->eng.flush_carry();
+    (void)e->eng.flushed(nullptr);
     if (hipStreamSynchronize(e->eng.stream) != hipSuccess) return set_error(GFE_EHIP, "sync");
     return e->eng.check("sync");
 }

@@ -697,13 +697,19 @@ __device__ __forceinline__ void f64_norm_store(F64CrtP c, const double (&x)[K][1
     }
 }
 
-// Digits of range w (32 digits from 32 w) with their range carry, balanced; the carry out stays in
-// slots[w].w (which no pass reads) for f64_carry_body, which adds it to the range above once every
-// range is done; the range carry is cleared.
-__device__ __forceinline__ void f64_flush_body(int32_t *dst, int4 *slots, uint32_t b, uint32_t w) {
+// Digits of range w (32 digits from 32 w of src) with their range carry, balanced, to the same place of
+// dst (STORE); returns the carry out.  All are loaded before the first is stored: in turn (src may be
+// dst) each load waited for memory by itself: a squaring and a copy out 14.3 us at n = 14, not 13.1, 81.2
+// at n = 22, not 79.8.
+template <bool STORE = true>
+__device__ __forceinline__ int32_t f64_flush_range(const int32_t *src, int32_t *dst, const int4 *slots, uint32_t b, uint32_t w) {
     const double bd = (double)b, binv = 1.0 / bd, qb = 0.25 * binv;
     const int4 v = slots[w];
-    int4 *p = reinterpret_cast<int4 *>(dst + (size_t)w * 32);
+    const int4 *p = reinterpret_cast<const int4 *>(src + (size_t)w * 32);
+    int4 *o = reinterpret_cast<int4 *>(dst + (size_t)w * 32);
+    int4 in[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) in[i] = p[i];
     double c = 0.0;
     auto digit = [&](int32_t d, int32_t e) -> int32_t {
         const double D = (double)d + (double)e + c;
@@ -712,14 +718,20 @@ __device__ __forceinline__ void f64_flush_body(int32_t *dst, int4 *slots, uint32
     };
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        int4 x = p[i];
+        int4 x = in[i];
         x.x = digit(x.x, i == 0 ? v.x : 0);
         x.y = digit(x.y, i == 0 ? v.y : 0);
         x.z = digit(x.z, i == 0 ? v.z : 0);
         x.w = digit(x.w, 0);
-        p[i] = x;
+        if constexpr (STORE) o[i] = x;
     }
-    slots[w] = make_int4(0, 0, 0, (int32_t)c);
+    return (int32_t)c;
+}
+
+// In place: the carry out stays in slots[w].w (which no pass reads) for f64_carry_body, which adds it to
+// the range above once every range is done; the range carry is cleared.
+__device__ __forceinline__ void f64_flush_body(int32_t *dst, int4 *slots, uint32_t b, uint32_t w) {
+    slots[w] = make_int4(0, 0, 0, f64_flush_range(dst, dst, slots, b, w));
 }
 
 // A carry c into balanced digits p[0..N-1], N digits of a range.
@@ -733,6 +745,24 @@ __device__ __forceinline__ void f64_carry_digits(int32_t *p, int32_t c, uint32_t
         p[i] = d - c * (int32_t)b;
     }
     if (c) p[N - 1] += c;
+}
+
+// Register 0 with its pending range carries, balanced, to dst, in one launch; the register and its carries
+// stay as they are.  F64_FLUSH_R ranges of N digits a workgroup, range(std::bool_constant<STORE>, w) one of
+// them; a wave of its own works out the carry out of the range below again.
+constexpr uint32_t F64_FLUSH_R = 64;
+template <int N, class R>
+__device__ __forceinline__ void f64_flush_to_body(const R &range, int32_t *dst, uint32_t nrange, uint32_t b) {
+    __shared__ int32_t cs[F64_FLUSH_R + 1];
+    const uint32_t t = threadIdx.x, w0 = blockIdx.x * F64_FLUSH_R, w = w0 + t;
+    if (t < F64_FLUSH_R) {
+        cs[t + 1] = range(std::true_type{}, w);
+    } else if (t == F64_FLUSH_R) {
+        const int32_t c = range(std::false_type{}, w0 == 0 ? nrange - 1 : w0 - 1);
+        cs[0] = w0 == 0 ? -c : c;  // B^M = -1
+    }
+    __syncthreads();
+    if (t < F64_FLUSH_R) f64_carry_digits<N>(dst + (size_t)w * N, cs[t], b);
 }
 
 __device__ __forceinline__ void f64_carry_body(int32_t *dst, const int4 *slots, uint32_t nrange, uint32_t b, uint32_t w) {

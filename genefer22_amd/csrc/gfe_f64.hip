@@ -331,6 +331,17 @@ __global__ void __launch_bounds__(256) k64_carry(F64Args A) {
     f64_carry_body(A.regs + s * A.reg_stride, A.slots + s * A.slot_stride, (1u << c->n) / 32, c->b, w);
 }
 
+// One candidate's register 0 with its pending range carries, balanced, to dst: M / 16 / F64_FLUSH_R
+// workgroups.  Copies, scalar products, waits and read-outs take it so: flushing in place takes two launches
+// (a range's carry out may only be added once the range above it is done), which at n <= 16 was more
+// than the squaring had gained on the integer passes.  us a squaring and the operation, flushed in place,
+// here, and in integers, at n = 14: copy out 20.2, 13.1, 17.3; wait 28.0, 24.5, 26.9; scalar product 23.2,
+// 19.2, 20.4; the Gerbicz-Li update (a product and three copies) 55.8, 36.1, 48.4.
+__global__ void __launch_bounds__(2 * F64_FLUSH_R) k64_flush_to(F64Args A, uint32_t b, int32_t *dst) {
+    const auto range = [&](auto st, uint32_t w) { return f64_flush_range<decltype(st)::value>(A.regs, dst, A.slots, b, w); };
+    f64_flush_to_body<32>(range, dst, (1u << A.tn) / 16, b);
+}
+
 struct F64TwArgs {
     double *tw;
     uint32_t words;                       // per prime
@@ -624,6 +635,11 @@ void f64_launch_flush(const F64Args &A, hipStream_t stream) {
     const dim3 grid(((1u << (A.tn - 4)) + 255) / 256, A.nslots);
     hipLaunchKernelGGL(k64_flush, grid, dim3(256), 0, stream, A);
     hipLaunchKernelGGL(k64_carry, grid, dim3(256), 0, stream, A);
+}
+
+void f64_launch_flush_to(const F64Args &A, const F64Shape &S, uint32_t b, int32_t *dst, hipStream_t stream) {
+    if (S.quad) return f64q_launch_flush_to(A, b, dst, stream);
+    hipLaunchKernelGGL(k64_flush_to, dim3((1u << (A.tn - 4)) / F64_FLUSH_R), dim3(2 * F64_FLUSH_R), 0, stream, A, b, dst);
 }
 
 void f64_set_lds_attributes() {

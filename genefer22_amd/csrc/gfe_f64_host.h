@@ -69,12 +69,15 @@ void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream);
 void f64_launch_square(F64Args A, const F64Shape &S, int mode, hipStream_t stream);
 // Adds the pending range carries of register 0 and balances it.
 void f64_launch_flush(const F64Args &A, hipStream_t stream);
+// The same to dst (not register 0), which leaves the register and its carries; one candidate of base b.
+void f64_launch_flush_to(const F64Args &A, const F64Shape &S, uint32_t b, int32_t *dst, hipStream_t stream);
 void f64_set_lds_attributes();
 // The same for limbs of four digits (called by the above where S.quad).
 void f64q_launch_fwd(const F64Args &A, const F64Shape &S, hipStream_t stream);
 void f64q_launch_mid(const F64Args &A, const F64Shape &S, int mode, hipStream_t stream);
 void f64q_launch_inv(const F64Args &A, const F64Shape &S, hipStream_t stream);
 void f64q_launch_flush(const F64Args &A, uint32_t b, hipStream_t stream);
+void f64q_launch_flush_to(const F64Args &A, uint32_t b, int32_t *dst, hipStream_t stream);
 void f64q_set_lds_attributes();
 
 }  // namespace gfe

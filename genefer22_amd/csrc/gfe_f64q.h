@@ -144,11 +144,16 @@ __device__ __forceinline__ void f64q_norm_limb(F64QCrtP c, const double (&r)[5],
     }
 }
 
-// As f64_flush_body for range w of 64 digits; the carry out stays in slots[2 w + 1].w.
-__device__ __forceinline__ void f64q_flush_body(int32_t *dst, int4 *slots, uint32_t b, uint32_t w) {
+// As f64_flush_range for range w of 64 digits.
+template <bool STORE = true>
+__device__ __forceinline__ int32_t f64q_flush_range(const int32_t *src, int32_t *dst, const int4 *slots, uint32_t b, uint32_t w) {
     const double bd = (double)b, binv = 1.0 / bd, qb = 0.25 * binv;
     const int4 u = slots[2 * w], v = slots[2 * w + 1];
-    int4 *p = reinterpret_cast<int4 *>(dst + (size_t)w * 64);
+    const int4 *p = reinterpret_cast<const int4 *>(src + (size_t)w * 64);
+    int4 *o = reinterpret_cast<int4 *>(dst + (size_t)w * 64);
+    int4 in[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) in[i] = p[i];
     double c = 0.0;
     auto digit = [&](int32_t d, int32_t e) -> int32_t {
         const double D = (double)d + (double)e + c;
@@ -157,15 +162,21 @@ __device__ __forceinline__ void f64q_flush_body(int32_t *dst, int4 *slots, uint3
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        int4 x = p[i];
+        int4 x = in[i];
         x.x = digit(x.x, i == 0 ? u.x : i == 1 ? v.x : 0);
         x.y = digit(x.y, i == 0 ? u.y : 0);
         x.z = digit(x.z, i == 0 ? u.z : 0);
         x.w = digit(x.w, i == 0 ? u.w : 0);
-        p[i] = x;
+        if constexpr (STORE) o[i] = x;
     }
+    return (int32_t)c;
+}
+
+// As f64_flush_body; the carry out stays in slots[2 w + 1].w.
+__device__ __forceinline__ void f64q_flush_body(int32_t *dst, int4 *slots, uint32_t b, uint32_t w) {
+    const int32_t c = f64q_flush_range(dst, dst, slots, b, w);
     slots[2 * w] = make_int4(0, 0, 0, 0);
-    slots[2 * w + 1] = make_int4(0, 0, 0, (int32_t)c);
+    slots[2 * w + 1] = make_int4(0, 0, 0, c);
 }
 
 }  // namespace gfe

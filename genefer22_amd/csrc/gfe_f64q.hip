@@ -116,6 +116,12 @@ __global__ void __launch_bounds__(256) k64q_carry(F64Args A, uint32_t b) {
     if (w < nrange) f64_carry_digits<64>(A.regs + (size_t)w * 64, w == 0 ? -A.slots[2 * nrange - 1].w : A.slots[2 * w - 1].w, b);
 }
 
+// As k64_flush_to.
+__global__ void __launch_bounds__(2 * F64_FLUSH_R) k64q_flush_to(F64Args A, uint32_t b, int32_t *dst) {
+    const auto range = [&](auto st, uint32_t w) { return f64q_flush_range<decltype(st)::value>(A.regs, dst, A.slots, b, w); };
+    f64_flush_to_body<64>(range, dst, (1u << A.tn) / 16, b);
+}
+
 // ------------------------------------------------------------------------------------------------
 // Host
 
@@ -226,6 +232,10 @@ void f64q_launch_flush(const F64Args &A, uint32_t b, hipStream_t stream) {
     const dim3 grid(((1u << (A.tn - 4)) + 255) / 256);
     hipLaunchKernelGGL(k64q_flush, grid, dim3(256), 0, stream, A, b);
     hipLaunchKernelGGL(k64q_carry, grid, dim3(256), 0, stream, A, b);
+}
+
+void f64q_launch_flush_to(const F64Args &A, uint32_t b, int32_t *dst, hipStream_t stream) {
+    hipLaunchKernelGGL(k64q_flush_to, dim3((1u << (A.tn - 4)) / F64_FLUSH_R), dim3(2 * F64_FLUSH_R), 0, stream, A, b, dst);
 }
 
 void f64q_set_lds_attributes() {

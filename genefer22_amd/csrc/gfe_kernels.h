@@ -723,13 +723,14 @@ __device__ __forceinline__ void norm_loop(const CrtConst &c, const uint32_t *__r
 }
 
 // r = a r on the balanced digits (the reference's mulscalar, ocl/kernel.cl:2461-2492, run after
-// the normalisation as baseModMul does, src/transformGPU.h:828-837), 8 digits per thread.
-__device__ __forceinline__ void mulscalar_body(int32_t *dc, int64_t *wc, uint32_t b, int32_t a, unsigned blk) {
+// the normalisation as baseModMul does, src/transformGPU.h:828-837), 8 digits per thread, from src to dc
+// (which may be src).
+__device__ __forceinline__ void mulscalar_body(const int32_t *src, int32_t *dc, int64_t *wc, uint32_t b, int32_t a, unsigned blk) {
     constexpr int S = 8;
     const size_t i0 = ((size_t)blk * 256 + threadIdx.x) * S;
     const double binv = 1.0 / (double)b;
     int32_t d[S];
-    const int4 v0 = *reinterpret_cast<const int4 *>(dc + i0), v1 = *reinterpret_cast<const int4 *>(dc + i0 + 4);
+    const int4 v0 = *reinterpret_cast<const int4 *>(src + i0), v1 = *reinterpret_cast<const int4 *>(src + i0 + 4);
     d[0] = v0.x; d[1] = v0.y; d[2] = v0.z; d[3] = v0.w; d[4] = v1.x; d[5] = v1.y; d[6] = v1.z; d[7] = v1.w;
     int64_t c = 0;
 #pragma unroll
