@@ -373,6 +373,11 @@ static uint64_t pow64(uint64_t a, uint64_t e, uint64_t p) {
     return r;
 }
 uint64_t f64_inv_mod(uint64_t a, uint64_t p) { return pow64(a % p, p - 2, p); }
+uint64_t f64_inv_pow2(int k, uint64_t p) {
+    uint64_t s = 1;
+    while (k-- > 0) s = ((s & 1) ? s + p : s) / 2;
+    return s;
+}
 double f64_balanced(uint64_t a, uint64_t p) { return a > p / 2 ? -(double)(p - a) : (double)a; }
 
 // Largest doubled coefficient against the primes' product.  Limbs are at most L = (b/2 + 4)(b + 1),
@@ -414,13 +419,16 @@ F64Crt make_f64_crt(uint32_t n, uint32_t b, int K) {
         c.p[k] = (double)p;
         c.pinv[k] = 1.0 / (double)p;
         // n - 3 of the transform's n - 1 levels are run and undone: 2^(n-3) comes out of the inverse
-        const uint64_t s = f64_inv_mod((uint64_t)1 << (n - 3), p);
+        const uint64_t s = f64_inv_pow2((int)n - 3, p);
         c.s[0][k] = f64_balanced(s, p);
         c.s[1][k] = f64_balanced(mul64(s, 2, p), p);
     }
-    c.i12 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[1]), F64_P[1]);
-    c.i13 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[2]), F64_P[2]);
-    c.i23 = f64_balanced(f64_inv_mod(F64_P[1], F64_P[2]), F64_P[2]);
+    // the primes' inverses once: made with every base's constants they took 3 us, and 7 in make_f64q_crt, of a
+    // rebase or submission
+    static const double i12 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[1]), F64_P[1]);
+    static const double i13 = f64_balanced(f64_inv_mod(F64_P[0], F64_P[2]), F64_P[2]);
+    static const double i23 = f64_balanced(f64_inv_mod(F64_P[1], F64_P[2]), F64_P[2]);
+    c.i12 = i12; c.i13 = i13; c.i23 = i23;
     auto split = [&](__int128 x, int pieces, double *w, uint32_t *wl) {
         for (int i = 0; i < pieces; ++i) {
             __int128 r = x;

@@ -29,6 +29,7 @@ F64Crt make_f64_crt(uint32_t n, uint32_t b, int K);
 inline size_t f64_tw_words(uint32_t n) { return ((size_t)1 << n) / 8; }
 int f64_build_twiddles(uint32_t n, double *tw, hipStream_t stream);
 uint64_t f64_inv_mod(uint64_t a, uint64_t p);
+uint64_t f64_inv_pow2(int k, uint64_t p);     // 2^-k mod p
 double f64_balanced(uint64_t a, uint64_t p);  // in (-p/2, p/2]
 
 // Limbs of four digits, for one candidate: where they are exact and pay, constants and tables.

@@ -142,15 +142,23 @@ bool f64q_ok(uint32_t b, uint32_t n) {
 void make_f64q_crt(uint32_t n, uint32_t b, F64QCrt *out) {
     F64QCrt &c = *out;
     memset(&c, 0, sizeof(c));
+    struct Inverses {
+        double i[5][4];
+        Inverses() {
+            for (int k = 0; k < F64Q_PRIMES; ++k)
+                for (int j = 0; j < k; ++j) i[k][j] = f64_balanced(f64_inv_mod(F64Q_P[j], F64Q_P[k]), F64Q_P[k]);
+        }
+    };
+    static const Inverses inv;
     for (int k = 0; k < F64Q_PRIMES; ++k) {
         const uint64_t p = F64Q_P[k];
         c.p[k] = (double)p;
         c.pinv[k] = 1.0 / (double)p;
         // n - 4 of the transform's n - 2 levels are run and undone
-        const uint64_t s = f64_inv_mod((uint64_t)1 << (n - 4), p);
+        const uint64_t s = f64_inv_pow2((int)n - 4, p);
         c.s[0][k] = f64_balanced(s, p);
         c.s[1][k] = f64_balanced(2 * s % p, p);
-        for (int j = 0; j < k; ++j) c.inv[k][j] = f64_balanced(f64_inv_mod(F64Q_P[j], p), p);
+        for (int j = 0; j < k; ++j) c.inv[k][j] = inv.i[k][j];
         c.sq[k] = f64_balanced((uint64_t)b * b % p, p);
     }
     // base-b pieces of p1, p1 p2, .. and of 2^23 times each
