@@ -216,3 +216,38 @@ def test_four_digit_limbs_equal_the_integer_passes(gfe, n):
         assert np.array_equal(t.get_digits(), u.get_digits())
         t.close()
         u.close()
+
+
+def test_full_tests_in_a_batch_of_three_passes(gfe):
+    """Whole tests at n = 14, with the Gerbicz-Li products (forward passes into the multiplicand and
+    products of the active slots only) on slots of two and of three primes that reach them at
+    different rounds; the residues are the single engine's."""
+    n, e = 14, largest_two_prime_base(14)
+    bases = [1026, (e & ~1) + 2, 4098]
+    bt = gfe.Batch(n, len(bases))
+    for i, b in enumerate(bases):
+        assert bt.submit(b, 0, i) == i
+    got = {}
+    while len(got) < len(bases):
+        bt.step()
+        got.update((r["tag"], r) for r in bt.poll())
+    bt.close()
+    for i, b in enumerate(bases):
+        w = gfe.run_quick(b, n)
+        assert (got[i]["res64"], got[i]["old64"], got[i]["gl_ok"]) == (w["res64"], w["old64"], 1), b
+
+
+def test_proofs_in_a_batch_of_three_passes(gfe):
+    """The powers of a proof at n = 14: rows that square some slots and multiply others."""
+    n, depth, bases = 14, 2, [1026, 4098]
+    bt = gfe.Batch(n, len(bases), depth=depth)
+    for i, b in enumerate(bases):
+        assert bt.submit(b, 0, i) == i
+    got = {}
+    while len(got) < len(bases):
+        bt.step()
+        got.update((r["tag"], r) for r in bt.poll())
+    bt.close()
+    for i, b in enumerate(bases):
+        w = gfe.run_proof(b, n, depth)
+        assert (got[i]["res64"], got[i]["pkey"], got[i]["mu_hash64"], got[i]["gl_ok"]) == (w["res64"], w["pkey"], w["mu_hash64"], 1), b
