@@ -645,7 +645,7 @@ int Batch::init(uint32_t n_, uint32_t cap_, int device_, int depth_, bool mixed_
         hipMalloc(&slots_dev, (size_t)cap * sizeof(SlotInfo)) != hipSuccess ||
         hipMalloc(&act_dev, (size_t)64 * cap) != hipSuccess || hipMalloc(&dup_dev, (size_t)64 * cap) != hipSuccess ||
         hipMalloc(&mul_dev, (size_t)64 * cap) != hipSuccess ||
-        hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess ||
+        (n <= F64_ALL_BASES_N && hipMalloc(&tw64, F64_PRIMES * f64_tw_words(n) * 8) != hipSuccess) ||
         hipMalloc(&crt64, (size_t)cap * sizeof(F64Crt)) != hipSuccess)
         return set_error(GFE_ENOMEM, "device allocation failed");
     for (int i = 0; i < NSTAGE; ++i) {
@@ -1562,8 +1562,8 @@ int gfe_batch_backlog(gfe_batch *b) {
 size_t gfe_batch_device_bytes(uint32_t n, uint32_t capacity) { return gfe_batch_proof_device_bytes(n, capacity, 0); }
 
 size_t gfe_batch_proof_device_bytes(uint32_t n, uint32_t capacity, uint32_t depth) {
-    const size_t N = (size_t)1 << n;
-    return (size_t)capacity * (gfe_batch_proof_slot_bytes(n, depth) + 3 * 64) + 6 * N * 4 + gfe::F64_PRIMES * gfe::f64_tw_words(n) * 8;
+    const size_t tables = n <= gfe::F64_ALL_BASES_N ? gfe::F64_PRIMES * gfe::f64_tw_words(n) * 8 : (size_t)24 << n;
+    return (size_t)capacity * (gfe_batch_proof_slot_bytes(n, depth) + 3 * 64) + tables;
 }
 
 int gfe_batch_get_digits(gfe_batch *b, int32_t slot, uint32_t reg, int32_t *out) {

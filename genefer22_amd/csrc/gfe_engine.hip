@@ -411,13 +411,19 @@ bool limb_fused_ok(uint32_t b, uint32_t n, int ng) {
 // double-precision limb transform's 3 x N/2 of 8.
 static size_t work_bytes(size_t N) { return 4 * (size_t)F64_PRIMES * N; }
 
-// Device bytes of an engine: registers, work space and multiplicand, the twiddles of rns primes, the
-// carry buffer (N bytes), with limb_tables the limb transform's twiddles (4 x N/2 words), and the
-// double-precision transform's (3 x N/8 doubles, and 5 x N/16 where limbs of four digits may be used:
-// a rebase keeps both).
-size_t engine_bytes(int rns, size_t N, uint32_t num_regs, bool limb_tables) {
-    return (size_t)num_regs * N * 4 + 2 * work_bytes(N) + (size_t)rns * N * 4 + N + (limb_tables ? 8 * N : 0) +
-           (size_t)F64_PRIMES * N + (N >> F64Q_MIN_N ? 5 * N / 2 : 0);
+// Bytes of the twiddles: of the integer passes' rns primes, of the integer limb transform (4 x N/2 words),
+// of limbs of two digits in doubles (3 x N/8) and of four (5 x N/16).
+static size_t table_bytes(size_t N, int rns, bool integer, bool limb, bool two, bool four) {
+    return (integer ? (size_t)rns * N * 4 + (limb ? 8 * N : 0) : 0) + (two ? F64_PRIMES * N : 0) + (four ? F64Q_PRIMES * N / 2 : 0);
+}
+
+// Device bytes an engine needs for every base of its prime set (limb_tables: and for those of the limb
+// transform) with no plan set: registers, work space, multiplicand, carries, and the tables that a
+// rebase adds to and keeps.
+size_t engine_bytes(int rns, uint32_t n, uint32_t num_regs, bool limb_tables) {
+    const size_t N = (size_t)1 << n;
+    return (size_t)num_regs * N * 4 + 2 * work_bytes(N) + N +
+           table_bytes(N, rns, n > F64_ALL_BASES_N, limb_tables, true, n >= F64Q_MIN_N);
 }
 
 // An engine's first plan: the limb transform where it is exact (with the inverse column pass and
@@ -1375,7 +1381,8 @@ int gfe_set_digits(gfe_engine *e, uint32_t reg, const int32_t *in) {
 size_t gfe_mem_size(const gfe_engine *e) {
     if (!e) return 0;
     const Engine &g = e->eng;
-    return gfe::engine_bytes(g.rns, g.N, g.num_regs, g.limb_made);
+    return (size_t)g.num_regs * g.N * 4 + 2 * gfe::work_bytes(g.N) + g.N +
+           gfe::table_bytes(g.N, g.rns, g.tw, g.tw_limb, g.tw64, g.twq);
 }
 
 size_t gfe_cache_size(const gfe_engine *e) {

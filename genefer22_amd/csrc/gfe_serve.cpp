@@ -137,7 +137,7 @@ struct gfe_server {
         gfe::select_primes(b, n, &w.rns, &w.is32);
         w.is32 = gfe::transform_is32(w.rns, w.is32);
         w.limb = gfe::limb_ok(b, n) && gfe::default_limb_plan(n).limb;
-        w.bytes = gfe::engine_bytes(w.rns, size_t(1) << n, 3, w.limb);
+        w.bytes = gfe::engine_bytes(w.rns, n, 3, w.limb);
         return w;
     }
     // A warm engine that can take kind k: same n and prime set, and the limb transform's tables

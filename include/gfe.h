@@ -60,7 +60,9 @@ int gfe_copy(gfe_engine *e, uint32_t dst, uint32_t src);
  * and gint canonicalisation on the caller side); any register. */
 int gfe_get_digits(gfe_engine *e, uint32_t reg, int32_t *out);
 int gfe_set_digits(gfe_engine *e, uint32_t reg, const int32_t *in);
-/* transform::getMemSize / getCacheSize, src/transform.h:65-66. */
+/* transform::getMemSize / getCacheSize, src/transform.h:65-66.  The memory is what the engine holds; the
+ * first gfe_set_plan or gfe_tune adds the integer passes' twiddle tables, a gfe_rebase those its base needs
+ * (GFE_ENOMEM where they do not fit). */
 size_t gfe_mem_size(const gfe_engine *e);
 size_t gfe_cache_size(const gfe_engine *e);
 /* transform::saveContext / readContext, src/transform.h:68-69: the payload of the context file

@@ -100,7 +100,9 @@ int gfe_batch_poll(gfe_batch *bt, gfe_batch_result *out, uint32_t max, uint32_t 
 int gfe_batch_active(const gfe_batch *bt);
 /* Squaring blocks enqueued on the device and not finished yet (>= 0), or a negative error code. */
 int gfe_batch_backlog(gfe_batch *bt);
-/* Device bytes a batch of `capacity` slots allocates (slots, shared twiddles, flags). */
+/* Device bytes a batch of `capacity` slots allocates (slots, shared twiddles, flags).  Up to n = 20 the first
+ * gfe_batch_set_plan or gfe_batch_tune adds the integer passes' twiddles, 24 2^n bytes (GFE_ENOMEM where
+ * they do not fit). */
 size_t gfe_batch_device_bytes(uint32_t n, uint32_t capacity);
 size_t gfe_batch_proof_device_bytes(uint32_t n, uint32_t capacity, uint32_t depth);
 /* Canonical digits of register `reg` (< 3, or < 3 + 2^depth in a proof batch) of a busy slot (for

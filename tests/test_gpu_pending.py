@@ -98,3 +98,16 @@ def test_any_order_of_operations_equals_the_integer_passes(gfe, b, n, count):
         same(reg)
     t.close()
     u.close()
+
+
+@pytest.mark.parametrize("b,n,rns", [(1026, 12, 2), (50000000, 14, 3), (1999999998, 14, 3), (20204692, 20, 3)])
+def test_memory_is_what_the_engine_holds(gfe, b, n, rns):
+    """Registers, work space, multiplicand and carries, and the tables made so far: in doubles, limbs of
+    two digits or of four; the integer passes' with the first plan set."""
+    N = 1 << n
+    t = gfe.Transform(b, n)
+    held = 3 * 4 * N + 2 * 12 * N + N + (5 * N // 2 if "four digits" in t.info() else 3 * N)
+    assert t.mem_size() == held
+    t.set_plan(t.get_plan())
+    assert t.mem_size() == held + 4 * rns * N + (8 * N if t.get_plan()[5] & 32 else 0)
+    t.close()

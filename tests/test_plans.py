@@ -180,3 +180,14 @@ def test_limb_plans_need_the_compile_time_passes(G):
     assert G.plan_admissible(22, base[:5] + (42,))  # compile-time passes, inverse columns fused with the norm
     # the fused kernel runs the four primes' column groups in one workgroup: 4 T <= 1024 threads
     assert not G.plan_admissible(22, (7, 3, 32, 5, 1, 42)) and G.plan_admissible(22, (7, 3, 32, 5, 1, 40))
+
+
+@pytest.mark.parametrize("n", range(12, 24))
+def test_batch_footprint_counts_what_is_allocated(G, n):
+    """Up to n = 20 a batch holds the three primes' tables in doubles, 3 x 2^n / 8 entries, and no
+    integer table until a plan is set; above, the six integer tables: in no case more than on the
+    integer passes, so a budget that held a batch holds it still."""
+    L = G.lib()
+    for cap in (1, 5):
+        tables = L.gfe_batch_device_bytes(n, cap) - cap * (L.gfe_batch_slot_bytes(n) + 192)
+        assert tables == (3 << n if n <= 20 else 24 << n)
