@@ -356,9 +356,6 @@ struct Batch {
     uint8_t *stage[NSTAGE] = {};                      // each 3 x 64 x cap
     hipEvent_t stage_ev[NSTAGE] = {};
     int stage_i = 0;
-    // Pinned mirrors of the per-slot tables.  Entry s is written only by submit() into a free
-    // slot; the previous occupant's program ended with a read-back, whose completion the host
-    // waited for, so no upload of entry s is still pending then.
     int32_t *readback = nullptr;                      // pinned N int32 (synchronous reads)
     // Asynchronous result read-backs: pinned N-digit buffers, each with a completion event,
     // processed in stream order.
@@ -461,7 +458,7 @@ struct Batch {
     void launch_row(const BArgs &A, int mode);
     void launch_col_inv(const BArgs &A);
     void launch_norm_carry(const BArgs &A);
-    void square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf = nullptr, bool has_mul = true);
+    void square(const uint8_t *active, const uint8_t *dup, const uint8_t *mulf, bool has_mul);
     void op_copy(const uint8_t *active, uint32_t dst, uint32_t src);
     void op_set(const uint8_t *active, uint32_t dst, int32_t value);
     void op_initmul(const uint8_t *active, uint32_t src);
@@ -583,7 +580,7 @@ int Batch::run_block(int rounds, uint32_t nact, bool has_mul, uint32_t nbig) {
         return set_error(GFE_EHIP, "squaring block graph capture failed");
     }
     for (int r = 0; r < rounds; ++r)
-        square(act_dev + (size_t)r * cap, dup_dev + (size_t)r * cap, mul_dev + (size_t)r * cap);
+        square(act_dev + (size_t)r * cap, dup_dev + (size_t)r * cap, mul_dev + (size_t)r * cap, has_mul);
     return check("square block");
 }
 

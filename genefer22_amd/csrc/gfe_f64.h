@@ -28,8 +28,9 @@
 // any representatives of v1 and v2 and the centred one of v3 (|x| < 0.3 P puts it well inside).  With
 // p1 and p1 p2 split into base-b pieces on the host, x = g0 + g1 b + g2 b^2 + g3 b^3 + g4 b^4 follows
 // digit by digit: a sum S known as a double and mod 2^32, the quotient q = rint(S / b) within 0.75
-// of S / b, the piece S - q b exact in 32 bits.  Every piece but the last is at most 0.75 b in size,
-// the last at most N / 4 + 2.
+// of S / b, the piece S - q b exact in 32 bits.  Every piece but the last is at most 0.75 b in size, the
+// last at most a coefficient over b^4 (f64_bound's G, range carries included: 0.3 N for large bases, never
+// over b^2 or 1e8).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -45,11 +46,10 @@ constexpr int F64_PRIMES = 3;
 // p = k 2^24 + 1 below 2^49 with their least primitive roots
 constexpr uint64_t F64_P[F64_PRIMES] = {562949869535233ull, 562949517213697ull, 562949282332673ull};
 constexpr uint32_t F64_G[F64_PRIMES] = {5, 10, 3};
-constexpr int F64_NG = 16;       // columns per workgroup: one 16-lane DPP row of limbs
-constexpr int F64_ROW_MIN = 8, F64_ROW_MAX = 14, F64_COL_MIN = 5, F64_COL_MAX = 8,
-              F64_SPLIT_MAX = 7;
+constexpr int F64_ROW_MIN = 8, F64_ROW_BATCH = 12, F64_ROW_MAX = 14;  // the longest rows of a batch (n <= 20) and of all
+constexpr int F64_COL_MIN = 5, F64_COL_MAX = 8, F64_SPLIT_MAX = 7;
 constexpr int F64_WHOLE_MIN = 11, F64_WHOLE_MAX = 12;           // log2 limbs of a one-workgroup transform
-constexpr uint32_t F64_NORM_T = 64, F64_NORM_PER = 1, F64_NORM_RANGE = F64_NORM_T * F64_NORM_PER;  // its normalisation
+constexpr uint32_t F64_NORM_T = 64;  // limbs per workgroup of its normalisation
 constexpr int F64_COL_E = 3;     // log2 of the residues per thread in the column passes
 
 // Constants of one candidate, read with scalar loads.

@@ -290,25 +290,21 @@ __global__ void __launch_bounds__(3 * (16 << (LOGG - F64_COL_E))) k64_col_inv_sp
 
 template <int K>
 __device__ __forceinline__ void f64_norm_body(const F64Args &A, const F64Job &J, uint32_t M, int dup) {
-    const uint32_t i0 = J.w * F64_NORM_RANGE + threadIdx.x;
+    const uint32_t i = J.w * F64_NORM_T + threadIdx.x;
     const double *ws = A.ws + J.slot * A.ws_stride;
-    double r[F64_NORM_PER][K];
+    double r[K];
 #pragma unroll
-    for (int j = 0; j < F64_NORM_PER; ++j)
-#pragma unroll
-        for (int k = 0; k < K; ++k) r[j][k] = ws[(size_t)k * M + i0 + j * F64_NORM_T];
-#pragma unroll
-    for (int j = 0; j < F64_NORM_PER; ++j)
-        f64_norm_limb<K>(J.c, r[j], dup, i0 + j * F64_NORM_T, M, A.regs + J.slot * A.reg_stride, A.slots + J.slot * A.slot_stride);
+    for (int k = 0; k < K; ++k) r[k] = ws[(size_t)k * M + i];
+    f64_norm_limb<K>(J.c, r, dup, i, M, A.regs + J.slot * A.reg_stride, A.slots + J.slot * A.slot_stride);
 }
 
-// The normalisation after k64_whole: M / F64_NORM_RANGE workgroups a slot (a mixed batch's slots of the
+// The normalisation after k64_whole: M / F64_NORM_T workgroups a slot (a mixed batch's slots of the
 // smaller n leave the rest idle).
 __global__ void __launch_bounds__(F64_NORM_T) k64_norm(F64Args A) {
-    const F64Job J = f64_job(A, (1u << A.tn) / F64_NORM_RANGE);
+    const F64Job J = f64_job(A, (1u << A.tn) / F64_NORM_T);
     if (!J.run) return;
     const uint32_t M = A.K ? 1u << A.tn : 1u << (J.c->n - 1);
-    if (J.w * F64_NORM_RANGE >= M) return;
+    if (J.w * F64_NORM_T >= M) return;
     const int dup = A.dupf ? (A.dupf[J.slot] != 0) : A.dup;
     if (J.K == 2) f64_norm_body<2>(A, J, M, dup);
     else f64_norm_body<3>(A, J, M, dup);
@@ -535,7 +531,7 @@ static F64Fn split_k(int a) {
 static F64Fn split_fn(int K, int a) { return K == 2 ? split_k<2>(a) : K == 3 ? split_k<3>(a) : split_k<0>(a); }
 template <int MODE, int LOGG = F64_ROW_MIN>
 static F64Fn row_fn(int logg) {
-    if constexpr (LOGG > F64_ROW_MAX) return nullptr;
+    if constexpr (LOGG > (MODE == F64_EITHER ? F64_ROW_BATCH : F64_ROW_MAX)) return nullptr;
     else return logg == LOGG ? k64_row<LOGG, MODE> : row_fn<MODE, LOGG + 1>(logg);
 }
 template <int MODE, int LOGG = F64_WHOLE_MIN>
@@ -555,9 +551,10 @@ static F64Fn mid_fn(bool whole, int mode, int logg) {
 
 // Slots are pinned to XCDs (slot s on XCD s mod 8) where that leaves at most an eighth of the XCDs'
 // time idle: what one pass leaves in the XCD's L2 the next one finds there.  us per round of a
-// batch, pinned and not: 301 slots of n = 12 19.9 and 29.5, 32 slots 9.7 and 10.9, 7 slots of n = 18
-// 40.8 and 44.4, 512 of n = 15 (4 MiB of L2 hold 1 % of an XCD's share) 228 and 229; 3 slots of n = 20
-// would use 3 of the 8 XCDs: 118 and 63.
+// batch, pinned and not: 301 slots of n = 12 18.5 and 26.4, 32 slots 7.8 and 9.2, 64 of n = 13 11.6 and
+// 15.9, of n = 14 21.4 and 29.9, of n = 15 32.8 and 36.3, 7 of n = 18 37.1 and 40.3; equal where 4 MiB of L2
+// hold little of an XCD's share (512 of n = 15 204 and 206, 24 of n = 18 88); 3 slots of n = 20 would use
+// 3 of the 8 XCDs: 112 and 55.6.
 static bool f64_pin(uint32_t slots) { return slots >= 7 && 7 * ((slots + 7) / 8) <= slots; }
 
 // Whether the column passes run the primes side by side: where one after the other they would be less than
@@ -607,7 +604,7 @@ void f64_launch_mid(F64Args A, const F64Shape &S, int mode, hipStream_t stream) 
 void f64_launch_inv(F64Args A, const F64Shape &S, hipStream_t stream) {
     if (S.quad) return f64q_launch_inv(A, S, stream);
     if (S.whole) {
-        const dim3 grid = f64_grid(A, (1u << A.tn) / F64_NORM_RANGE);
+        const dim3 grid = f64_grid(A, (1u << A.tn) / F64_NORM_T);
         hipLaunchKernelGGL(k64_norm, grid, dim3(F64_NORM_T), 0, stream, A);
         return;
     }

@@ -7,9 +7,10 @@
 // elements.  Exact for b from 2^20 to about 2^25.8 at n = 22 (f64q_ok), and faster from n = 20 on; us a
 // squaring, limbs of two digits and of four on one machine: n = 20 33.9 and 30.6, 21 45.7 and 41.6,
 // 22 80.2 and 70.6 (76.9 and 65.5 on a cooler one), 23 152.5 and 139.0.
-// A pass takes the sum of its moves and its arithmetic, hardly overlapped: its workgroups are all
-// resident at once and load, compute and store together.  At n = 22: forward 9.6 of moves and 6 of
-// arithmetic, rows 12.6 and 18, inverse 8.5 and 13.
+// A pass takes about the sum of its moves and its arithmetic.  At n = 22: forward 9.6 of moves and 6 of
+// arithmetic, rows 12.6 and 18, inverse 8.5 and 13.  A column pass's 256 workgroups are all resident at
+// once, two waves a SIMD, and load, compute and store together; the row pass's 1280 of 8 waves are four
+// a CU and a quarter of a layer more.
 //
 // CRT: as in gfe_f64.h, mixed-radix digits v1..v5 of the coefficient (v5 the centred one) and the
 // base-b pieces of p1, p1 p2, .., here modulo b^9: nine pieces g0..g8 of at most 0.51 b, the last
