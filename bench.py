@@ -69,7 +69,7 @@ MEASURED[("row", 7, 5, 1, 42)] = {"kernel": "gfe::ks_row_sq<gfe::ModS, 5, 14>", 
                                   "valu_instr_per_butterfly": 11.92, "profile": "profiles/n22_limb_fused_kernels.md"}
 # the double-precision transform, by (limbs of 2^l digits, column levels)
 MEASURED[("f64", "row", 2, 8)] = {"kernel": "gfe::k64q_row<12, 0>", "fetch_mib": 62.0, "write_mib": 40.0,
-                                  "traffic": int((62.0 + 40.0) * 2**20), "valu_instr_per_butterfly": 11.41,
+                                  "traffic": int((62.0 + 40.0) * 2**20), "valu_instr_per_butterfly": 11.56,
                                   "profile": "profiles/n22_f64_kernels.md"}
 MEASURED[("f64", "col_inv_norm", 2, 8)] = {"kernel": "gfe::k64q_col_inv<8>", "fetch_mib": 40.5, "write_mib": 18.0,
                                            "traffic": int((40.5 + 18.0) * 2**20), "valu_instr_per_butterfly": 23.62,

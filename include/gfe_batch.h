@@ -56,12 +56,13 @@ int gfe_batch_create(uint32_t n, uint32_t capacity, int device, gfe_batch **out)
  * GFE_BATCH_MAX_DEPTH (0: a quick-test batch). */
 int gfe_batch_create_proof(uint32_t n, uint32_t capacity, uint32_t depth, int device, gfe_batch **out);
 /* A mixed batch: candidates of n = 12 and n = 13 in the same slots (submit with gfe_batch_submit_n;
- * gfe_batch_submit means n = 13).  Every squaring block is one launch of the single-workgroup
- * squaring in which each workgroup works at its slot's n; while fewer than 128 slots of n = 13 are
- * active (where the single-workgroup squaring at n = 13 is slower than the four-step passes, one
- * candidate: 166 ms against 76 ms for 4096 squarings on MI355X) that launch takes the slots of
- * n = 12 and the slots of n = 13 run the four-step passes after it.  Register operations run on the
- * four-step passes of each slot's n.  A candidate's residues are those of its own n's batch. */
+ * gfe_batch_submit means n = 13).  A squaring round takes the slots of both n in the same two launches, each
+ * workgroup at its slot's n.  On the integer passes (gfe_batch_set_plan) every block is one launch of
+ * the single-workgroup squaring; while fewer than 128 slots of n = 13 are active (where the
+ * single-workgroup squaring at n = 13 is slower than the four-step passes, one candidate: 166 ms
+ * against 76 ms for 4096 squarings on MI355X) that launch takes the slots of n = 12 and the slots of
+ * n = 13 run the four-step passes after it, as register operations do on each slot's n.  A candidate's
+ * residues are those of its own n's batch. */
 int gfe_batch_create_mixed(uint32_t capacity, int device, gfe_batch **out);
 int gfe_batch_destroy(gfe_batch *bt);
 /* Device bytes one slot holds (registers, work space, multiplicand, carries): the admission unit. */
